@@ -16,12 +16,13 @@ __global__ void __launch_bounds__(1024) k_tdma_seg(const double* __restrict__ A,
                                                    long long es, long long ls, int LPB, int P, int cyclic) {
     extern __shared__ unsigned char smem[];
     const int tid = threadIdx.x;
-    // consecutive lanes take consecutive lines, except for cyclic lines with
-    // contiguous rows (es = 1, IJI), where they take consecutive segments of
-    // one line (measured at 65536 x 192: 0.252 -> 0.183 ms; 0.203 -> 0.319 ms
-    // for non-cyclic lines, which keep the line-major order)
-    const bool rowc = es == 1 && cyclic;
-    const int ll = rowc ? tid / P : tid % LPB, seg = rowc ? tid % P : tid / LPB;
+    // consecutive lanes take consecutive lines, also where the rows are the
+    // contiguous ones (measured at 65536 x 192, es = 1, with consecutive
+    // segments of a line instead: 0.203 -> 0.319 ms)
+    int ll = tid % LPB, seg = tid / LPB;
+    // hides that ll and seg come from one division: with that known the loads'
+    // addresses are kept apart in registers (126 instead of 92 at MS = 8)
+    asm("" : "+v"(ll), "+v"(seg));
     const long long line = (long long)blockIdx.x * LPB + ll;
     const bool valid = line < nlines;
     double a[MS], b[MS], c[MS], d[MS];
@@ -72,7 +73,78 @@ __global__ void __launch_bounds__(1024) k_tdma_seg(const double* __restrict__ A,
     }
 }
 
-// Fallback for shapes the segmented kernel does not cover: one thread per
+// Cyclic lines of any length (k_tdma_seg's cyclic form needs n to be a whole
+// number of segments, since the wrap couples the last real row): the last
+// unknown is split off, the n-1 rows left are a non-cyclic line, padded with
+// identity rows like any other, with two right-hand sides held as one double2:
+// r, and minus the couplings to x_{n-1}, so that x_i = y_i + z_i x_{n-1} and
+// the line's last equation gives x_{n-1}.  The reduced systems go through the
+// parallel cyclic reduction of all segment threads.  At most 512 threads: the
+// double2 rows need more than the 128 registers of a 1024-thread block.
+// Bound by the latency of its load - eliminate - reduce chain on few lines,
+// by HBM on many (40 B a row).  Replaces one thread per line with a device
+// workspace (k_tdma_seq): 1500 lines of 135 rows,
+// rows contiguous, 230 -> 8.4 us.
+template <int MS>
+__global__ void __launch_bounds__(512) k_tdma_cyc(const double* __restrict__ A, const double* __restrict__ B,
+                                                  const double* __restrict__ Cc, double* __restrict__ Rr, int n,
+                                                  int nlines, long long es, long long ls, int LPB, int P) {
+    extern __shared__ unsigned char smem[];
+    const int tid = threadIdx.x, ni = n - 1;
+    // rows contiguous: consecutive lanes take consecutive segments of a line
+    const bool rowc = es == 1;
+    const int ll = rowc ? tid / P : tid % LPB, seg = rowc ? tid % P : tid / LPB;
+    const long long line = (long long)blockIdx.x * LPB + ll;
+    const bool valid = line < nlines;
+    const long long base = valid ? line * ls : 0;
+    double a[MS], b[MS], c[MS];
+    double2 d[MS];
+#pragma unroll
+    for (int l = 0; l < MS; ++l) {
+        const long long o = base + (long long)min(seg * MS + l, ni - 1) * es;
+        a[l] = A[o];
+        b[l] = B[o];
+        c[l] = Cc[o];
+        d[l].x = Rr[o];
+    }
+    const long long on = base + (long long)ni * es;   // the line's last row
+    const double an = A[on], bn = B[on], cn = Cc[on], rn = Rr[on];
+#pragma unroll
+    for (int l = 0; l < MS; ++l) {
+        const int j = seg * MS + l;
+        d[l].y = (j == 0 ? -a[l] : 0.0) + (j == ni - 1 ? -c[l] : 0.0);
+        if (j == 0) a[l] = 0.0;
+        if (j == ni - 1) c[l] = 0.0;
+        if (!(valid && j < ni)) {   // padding rows: identity, decoupled
+            a[l] = 0.0;
+            b[l] = 1.0;
+            c[l] = 0.0;
+            d[l] = make_double2(0.0, 0.0);
+        }
+    }
+    seg_solve<MS, double2>(a, b, c, d, LPB, P, ll, seg, valid, false, smem);
+    // the reduced systems are dead (seg_solve's last barrier): the line's end
+    // values (y_0, z_0), (y_{n-2}, z_{n-2}) take their place
+    double2* ends = reinterpret_cast<double2*>(smem);
+    if (seg == 0) ends[2 * ll] = d[0];
+    if ((ni - 1) / MS == seg) {
+#pragma unroll
+        for (int l = 0; l < MS; ++l)
+            if (l == (ni - 1) % MS) ends[2 * ll + 1] = d[l];
+    }
+    __syncthreads();
+    if (!valid) return;
+    const double2 e0 = ends[2 * ll], e1 = ends[2 * ll + 1];
+    const double xn = (rn - cn * e0.x - an * e1.x) / (bn + cn * e0.y + an * e1.y);
+#pragma unroll
+    for (int l = 0; l < MS; ++l) {
+        const int j = seg * MS + l;
+        if (j < ni) Rr[base + (long long)j * es] = d[l].x + d[l].y * xn;
+    }
+    if (seg == 0) Rr[on] = xn;
+}
+
+// Fallback for shapes the segmented kernels do not cover: one thread per
 // line, the reference recurrences, H/G in a device workspace.
 __global__ void k_tdma_seq(const double* __restrict__ A, const double* __restrict__ B,
                            const double* __restrict__ Cc, double* __restrict__ Rr, const double* __restrict__ bc,
@@ -165,35 +237,65 @@ bool tdma_seg_config(int n, bool cyclic, int* MS, int* P, int* LPB, int maxthr, 
     return false;
 }
 
+// Lines per block of lpb0 (a power of two), halved to at least lo while the
+// block of p threads per line has more than thr threads.
+static int lines_per_block(int p, int lpb0, int lo, int thr) {
+    int lpb = lpb0;
+    while (lpb > lo && p * lpb > thr) lpb /= 2;
+    return lpb;
+}
+
 // ws: the sequential fallback's workspace of 3 n nlines doubles, or nullptr to
 // take it from the stream-ordered pool for this launch
 int tdma_launch(const double* a, const double* b, const double* c, double* r, const double* bc, int n, int nlines,
                 long long es, long long ls, int cyclic, hipStream_t s, double* ws_given = nullptr) {
-    int MS = 0, P = 0, LPB = 0;
-    bool seg = tdma_seg_config(n, cyclic != 0, &MS, &P, &LPB, 1024, false);
-    // measured at 65536 lines x 192 rows: lines contiguous (ls = 1, the IJJ
-    // layout) fastest in 12-row segments, 32 lines per block (0.141 -> 0.116
-    // ms non-cyclic, 0.168 -> 0.126 ms cyclic); rows contiguous (IJI) in
-    // 8-row segments, 16 lines per block (0.229 -> 0.200 ms non-cyclic) or 8
-    // for cyclic lines
-    {
-        const int ms = ls == 1 ? 12 : 8, lpb = ls == 1 ? 32 : (cyclic ? 8 : 16);
-        const int p = (n + ms - 1) / ms;
-        if (seg && p * lpb <= 1024 && (!cyclic || (n % ms == 0 && p >= 2))) {
-            MS = ms;
-            P = p;
-            LPB = lpb;
+    // Rows per segment and lines per block, swept on an MI355X for both
+    // layouts (lines x rows: best of the sweep; before: one configuration per
+    // layout, 12 x 32 for lines contiguous, 8 x 16 for rows contiguous):
+    //   lines contiguous   500x192 7.7 (11.4) us, 4000x192 11.0 (12.9),
+    //     2000x504 16.7 (37.3), 20000x504 113 (150): 8-row segments, 16 lines
+    //     (a 128-byte access) or 8 where few lines leave CUs idle; only a whole
+    //     grid's lines (65536x192) keep 12 x 32: 113 against 129 us
+    //   rows contiguous    500x192 7.2 (12.9), 10000x360 52.8 (75.3),
+    //     20000x504 131 (214): blocks of about 128 threads, whose phases
+    //     overlap; 65536x192 182 (189)
+    //   cyclic             through the split-off unknown (k_tdma_cyc), whose
+    //     reduced systems have no serial sweep: 500x192 8.3 (15.2), 2000x504
+    //     20.0 (20.1), rows contiguous 500x192 6.9 (20.3), 20000x504 144 (287);
+    //     only a whole grid's contiguous lines of whole 12-row segments stay
+    //     with k_tdma_seg: 65536x192 120 against 148 us
+    const bool grid_lines = nlines >= 32768, lines_contig = ls == 1;
+    int MS = 8, LPB = 0;
+    const int p12 = (n + 11) / 12;   // 12 x 32: blocks whose waves fill a CU's 16 (one block of 9 would leave 7 idle)
+    if (lines_contig && grid_lines && ((p12 >= 4 && p12 <= 16) || (p12 >= 28 && p12 <= 32)) &&
+        (!cyclic || n % 12 == 0)) {
+        MS = 12;
+        LPB = 32;
+    } else if (cyclic) {
+        const int p = (n - 1 + MS - 1) / MS;
+        LPB = es == 1 ? lines_per_block(p, 64, 2, 64)
+                      : lines_per_block(p, p <= 4 ? 32 : nlines < 2048 ? 8 : 16, 2, 512);
+        if (p * LPB <= 512) {
+            const size_t sm = std::max(seg_smem_bytes<double2>(LPB, p), 2 * sizeof(double2) * (size_t)LPB);
+            CHS_LAUNCH(k_tdma_cyc<8>, dim3((nlines + LPB - 1) / LPB), dim3(LPB * p), sm, s, a, b, c, r, n, nlines, es,
+                       ls, LPB, p);
+            return CHS_OK;
         }
+        LPB = 0;
+    } else if (lines_contig) {
+        const int p = (n + MS - 1) / MS;
+        LPB = lines_per_block(p, p <= 4 ? 32 : nlines < 2048 ? 8 : 16, 4, 1024);
+    } else {
+        LPB = lines_per_block((n + MS - 1) / MS, 32, 4, 128);
     }
-    if (seg) {
+    const int P = (n + MS - 1) / MS;
+    if (LPB > 0 && P * LPB <= 1024) {
         const dim3 grid((nlines + LPB - 1) / LPB), block(LPB * P);
         const size_t sm = seg_smem_bytes<double>(LPB, P);
-        switch (MS) {
-            case 16: CHS_LAUNCH(k_tdma_seg<16>, grid, block, sm, s, a, b, c, r, bc, n, nlines, es, ls, LPB, P, cyclic); break;
-            case 12: CHS_LAUNCH(k_tdma_seg<12>, grid, block, sm, s, a, b, c, r, bc, n, nlines, es, ls, LPB, P, cyclic); break;
-            case 4: CHS_LAUNCH(k_tdma_seg<4>, grid, block, sm, s, a, b, c, r, bc, n, nlines, es, ls, LPB, P, cyclic); break;
-            default: CHS_LAUNCH(k_tdma_seg<8>, grid, block, sm, s, a, b, c, r, bc, n, nlines, es, ls, LPB, P, cyclic); break;
-        }
+        if (MS == 12)
+            CHS_LAUNCH(k_tdma_seg<12>, grid, block, sm, s, a, b, c, r, bc, n, nlines, es, ls, LPB, P, cyclic);
+        else
+            CHS_LAUNCH(k_tdma_seg<8>, grid, block, sm, s, a, b, c, r, bc, n, nlines, es, ls, LPB, P, cyclic);
         return CHS_OK;
     }
     const int bs = 256;
