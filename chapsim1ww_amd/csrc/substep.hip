@@ -941,12 +941,10 @@ __global__ void __launch_bounds__(64) k_y_window(Geo g, const TR* __restrict__ R
 
 // z, register form: one thread per (i, j) column and chunk of zkc rows of k
 // (cyclic), the window slides along k; weights are the same for every lane.
-// zkc is ZKC or a multiple of it (longer chunks refill the window less often)
-// and divides N; the host checks both.
+// N need not be a multiple of zkc: the last chunk is shorter.  Both are
+// multiples of WU (N of KR: substep_supported), so a chunk has whole steps.
 // u subtracts D = DPGRNS * xone on load (the mass-flux correction pushed
 // through the x solve).  Reads RHS, writes RHS2.
-constexpr int ZKC = 64;
-static_assert(ZKC % WU == 0, "k_z_window steps a chunk WU rows at a time: a partial step would run past the chunk");
 // T: storage and arithmetic type (float in the mixed form).
 template <int KW, class T = double>
 __global__ void __launch_bounds__(256) k_z_window(Geo g, const T* __restrict__ R, T* __restrict__ R2,
@@ -954,7 +952,7 @@ __global__ void __launch_bounds__(256) k_z_window(Geo g, const T* __restrict__ R
                                                   const double* __restrict__ wz, int zkc) {
     const int L = g.L, M = g.M, N = g.N;
     const int ntx = (L + 63) / 64;
-    const int nch = N / zkc;
+    const int nch = (N + zkc - 1) / zkc;
     int b = blockIdx.x;
     const int lane = threadIdx.x & 63, ch = threadIdx.x >> 6;     // blockDim = 64 * 4
     const int it = b % ntx; b /= ntx;
@@ -971,7 +969,7 @@ __global__ void __launch_bounds__(256) k_z_window(Geo g, const T* __restrict__ R
     T w[W];
 #pragma unroll
     for (int m = 0; m < W; ++m) w[m] = T(wz[m]);
-    const int k0 = chunk * zkc;
+    const int k0 = chunk * zkc, k1 = min(N, k0 + zkc);
     T win[W];
 #pragma unroll
     for (int m = 0; m < W; ++m) {
@@ -979,7 +977,7 @@ __global__ void __launch_bounds__(256) k_z_window(Geo g, const T* __restrict__ R
         kk = kk < 0 ? kk + N : (kk >= N ? kk - N : kk);
         win[m] = Rc[(size_t)kk * LM] - D;
     }
-    for (int kb = k0; kb < k0 + zkc; kb += WU) {
+    for (int kb = k0; kb < k1; kb += WU) {
         T rn[WU];
 #pragma unroll
         for (int u = 0; u < WU; ++u) {
@@ -1595,6 +1593,17 @@ bool substep_supported(const chs_handle* h) {
     return h->L % XMS == 0 && P >= 2 && XLPB * P <= 1024 && h->N % KR == 0;
 }
 
+// Whether the CN solves run as stencils: widths within KMAX (cn.ok), and y
+// and z lines longer than the usual window of 17 rows (shorter z lines would
+// take either path with the time step).  A time step with the stencils and
+// with the Thomas solves: 64x64x24 225 / 302 us, 256x192x24 497 / 701,
+// 160x96x120 773 / 1115, 256x192x200 3158 / 5035.
+constexpr int ZMIN = 20;
+static_assert(KRS % WU == 0, "k_z_window steps a chunk WU rows at a time: a partial step would run past the chunk");
+static bool stencil_path(const chs_handle* h, const CnStencils& cn) {
+    return cn.ok && h->rhs2 != nullptr && h->cn_mode != 1 && h->N >= ZMIN && (h->M + YJC - 1) / YJC <= 8 && h->M > 16;
+}
+
 // last substep's CN solve path: 1 = truncated-inverse stencils, 0 = segmented Thomas
 int cn_last_path(chs_handle* h, double facoe, int* kx, int* kz, int* ky) {
     std::lock_guard<std::mutex> lk(h->cn_mu);
@@ -1603,7 +1612,7 @@ int cn_last_path(chs_handle* h, double facoe, int* kx, int* kz, int* ky) {
     *kx = cn->Kx;
     *kz = cn->Kz;
     *ky = cn->Ky;
-    return cn->ok && h->cn_mode != 1 && h->N % ZKC == 0 && (h->M + YJC - 1) / YJC <= 8 && h->M > 16 ? 1 : 0;
+    return stencil_path(h, *cn) ? 1 : 0;
 }
 
 // measured at 64^3 / 128^3 / 256x192x256 (FP64 substep): 2048 waves
@@ -1630,12 +1639,14 @@ static int ywin_chunk(const chs_handle* h) {
 static int xm_chunk(const chs_handle* h, size_t smem, bool fill) {
     return march_chunk_rows(h->M, h->N / KRS, smem, h->lds_max, fill);
 }
-// zkc divides N and is a multiple of WU (N is a multiple of ZKC on this path)
+// chunks of about 128 rows (measured at 256x192x256: 64 -> 128 rows, 139 ->
+// 134 us), of equal length to a multiple of WU
 static int zwin_chunk(const chs_handle* h) {
     const long per = 3L * h->M * ((h->L + 63) / 64);
-    int zkc = h->N % (2 * ZKC) == 0 ? 2 * ZKC : ZKC;
-    while (zkc > 8 && per * (h->N / zkc) < WIN_WAVES) zkc /= 2;
-    return zkc;
+    auto rows = [&](int nch) { return ((h->N + nch - 1) / nch + WU - 1) / WU * WU; };
+    int nch = (h->N + 127) / 128;
+    while (rows(nch) > 8 && per * nch < WIN_WAVES) nch *= 2;
+    return std::max(8, rows(nch));
 }
 
 int rk3_substep(chs_handle* h, int ns, double dt) {
@@ -1654,10 +1665,10 @@ int rk3_substep(chs_handle* h, int ns, double dt) {
     std::unique_lock<std::mutex> lk(h->cn_mu);
     CnStencils* cn = nullptr;
     CHS_TRY(cn_stencils_locked(h, facoe, &cn));
-    // stencil path needs: N in whole z tiles, at most 4 y chunks of YJC rows
-    // (blocks of 64*chunks threads), and chunks longer than the window
-    const bool use_st = cn->ok && h->rhs2 != nullptr && h->cn_mode != 1 && h->N % ZKC == 0 &&
-                        (h->M + YJC - 1) / YJC <= 8 && h->M > 16;
+    const bool use_st = stencil_path(h, *cn);
+    // the mixed form's FP32 stencils run where NCL3 is a multiple of 64; its
+    // other grids keep the precision they have always had, FP64 stencils
+    const bool f32_ok = h->precision == CHS_MIXED && h->N % 64 == 0;
     bool f32 = false;
     // 1. RHS + x solve
     {
@@ -1678,12 +1689,12 @@ int rk3_substep(chs_handle* h, int ns, double dt) {
         const bool use_xm = use_st && (h->cn_mode == 0 || h->cn_mode == 3) && (KRS / XM_CPT) * h->L % 64 == 0 &&
                             (KRS / XM_CPT) * h->L <= (XM_CPT == 1 ? 1024 : 512) &&
                             rhs_xm_smem(h->L, cn->KWx) <= (size_t)h->lds_max &&
-                            (h->cn_mode == 3 || h->precision == CHS_MIXED ||
+                            (h->cn_mode == 3 || f32_ok ||
                              xm_chunk(h, rhs_xm_smem(h->L, cn->KWx), true) >= MARCH_MIN);
         // the mixed form's FP32 stencils: RHS, the x solve and the z solve in
         // FP32 (RHS and RHS2 stored as float in the first half of the FP64
         // buffers), CONVH0 kept in FP32 (h0f); the y elimination stays FP64
-        f32 = h->precision == CHS_MIXED && use_xm;
+        f32 = f32_ok && use_xm;
         CHS_TRY(convh0_store(h, f32));
         h->timer.begin("rhs_x", s, &ev);
         if (f32) {
@@ -1759,9 +1770,8 @@ int rk3_substep(chs_handle* h, int ns, double dt) {
         const double xone = 1.0 / (xa + xb + xc);
         const int usedpg0 = 1;
         if (use_st) {
-            // 128-row chunks where N allows (measured at 256x192x256: 139 -> 134 us)
             const int zkc = zwin_chunk(h);
-            const dim3 gzw(3 * h->M * ((h->L + 63) / 64), (h->N / zkc + 3) / 4);
+            const dim3 gzw(3 * h->M * ((h->L + 63) / 64), ((h->N + zkc - 1) / zkc + 3) / 4);
             const double* wz = cn->dev + cn->oz;
             h->timer.begin("z_solve", s, &ev);
             if (f32) {
