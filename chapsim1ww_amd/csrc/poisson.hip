@@ -1,10 +1,12 @@
 // Pressure Poisson solve, the MI355X form of FFT99_POIS3D_periodicxz
 // (src/possion3d_FFT99.f90:254-488):
 //
-//   x: real FFT of every (j,k) row          k_fft_x_fwd   (LDS Stockham, 2 rows per complex FFT)
-//   z: complex FFT along k for every (j,kx) k_fft_z       (LDS Stockham, tile of TX kx columns)
+//   x: real FFT of every (j,k) row          k_reg_x_fwd, k_fft256_x_fwd  (2 rows per complex FFT)
+//   z: complex FFT along k for every (j,kx) k_reg_z, k_fft256_z          (tile of 8 kx columns)
 //   y: tridiagonal solve per (kx,kz) line   k_poisson_y   (segmented Thomas, FP64, complex RHS)
-//   z, x inverse transforms                 k_fft_z, k_fft_x_inv
+//   z, x inverse transforms                 k_reg_z, k_reg_x_inv, k_fft256_*
+// (k_fft_x_fwd, k_fft_z, k_fft_x_inv: LDS Stockham, the FP32 spectra of other
+// lengths than 256 and FP64 lengths without a register plan)
 //
 // The spectral array S is complex, layout S[(kz*M + j)*LHP + kx], so rows of
 // kx are contiguous: the x transform writes whole rows, the z transform reads
@@ -302,6 +304,208 @@ __global__ void __launch_bounds__(128) k_fft256_x_inv(const cpx_t<Rl>* __restric
             if (hi) base[(size_t)(M + 1) * 256 + 16 * k2] = ghost == 1 ? val : 0.0;
         }
     }
+}
+
+// ---------------------------------------------------------------------------
+// FP64 transforms of any length with a register plan (fft_dev.hpp): the x and
+// z passes of k_fft_x_fwd, k_fft_z and k_fft_x_inv with the stages' radices
+// chosen at run time by one switch per stage, and no integer division per
+// element.  Bound: HBM, each pass reading and writing its array once.  Against
+// the Stockham stages, which cross LDS once per radix up to 5 with two runtime
+// divisions per butterfly: at 320x150x240 z 79.8 -> 32.5 us (5.7 TB/s), x
+// 64.1 -> 41.0 and 67.1 -> 39.6 us; at 512x256x384 z 603 -> 160, x 416 -> 144
+// and 420 -> 207 us; a solve 338 -> 193 us and 2186 -> 830 us.  Length 256
+// keeps its own kernels: 43 + 37 (x), 37 us (z) against 41 + 42, 38 us here
+// at 256x192x256.
+// ---------------------------------------------------------------------------
+// f(R) for the radix of a stage (uniform over the block)
+template <int NST, class F>
+__device__ __forceinline__ void reg_radix(int rad, F f) {
+    switch (rad) {
+        case 4: f(std::integral_constant<int, 4>{}); return;
+        case 5: f(std::integral_constant<int, 5>{}); return;
+        case 6: f(std::integral_constant<int, 6>{}); return;
+        case 8: f(std::integral_constant<int, 8>{}); return;
+        case 9: f(std::integral_constant<int, 9>{}); return;
+        case 10: f(std::integral_constant<int, 10>{}); return;
+        default: break;
+    }
+    if constexpr (NST == 2) {
+        switch (rad) {
+            case 2: f(std::integral_constant<int, 2>{}); return;
+            case 3: f(std::integral_constant<int, 3>{}); return;
+            case 12: f(std::integral_constant<int, 12>{}); return;
+            case 15: f(std::integral_constant<int, 15>{}); return;
+            case 16: f(std::integral_constant<int, 16>{}); return;
+            default: break;
+        }
+    }
+}
+
+// A transform's elements in LDS, mul apart: after the first stage element
+// q r0 + k at q sA + k, after the middle one q r0 r1 + k at q sB + k.  In x
+// (mul = 1, lanes along the transform) odd strides keep the stages' stores
+// off each other's banks; in z (mul = 8, lanes along kx) any stride does.
+struct RegLds {
+    double2* b;
+    int mul, sA, sB;
+    __device__ __forceinline__ double2& at(int s, int q, int k) const { return b[(q * s + k) * mul]; }
+};
+
+// v = the twiddled inputs of butterfly t (clamped) of the stage of radix R
+// whose inputs are n/R = nb apart: place(r) is the LDS place of input r, step
+// the twiddle exponent of r = 1.  The twiddles are loaded before the barrier
+// that makes the stage before visible.
+template <int R, int DIR, class P>
+__device__ __forceinline__ void reg_gather(double2 (&v)[R], const double2* __restrict__ tw, int step, P place) {
+    double2 w[R];
+#pragma unroll
+    for (int r = 1; r < R; ++r) w[r] = tw[r * step];
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < R; ++r) v[r] = place(r);
+#pragma unroll
+    for (int r = 1; r < R; ++r) v[r] = cmul(v[r], DIR > 0 ? cconj(w[r]) : w[r]);
+    dft_reg<R, DIR>(v);
+}
+
+// The stages of one transform held by T threads (t = the thread's number; all
+// threads of the block call it: barriers).  load(i) gives input element i,
+// last(v, t, nb, R) takes the outputs t + r nb, r < R, of the threads with
+// t < nb (the others hold a copy of the last butterfly's).
+template <int NST, int DIR, class Ld, class Last>
+__device__ __forceinline__ void reg_fft(const RegPlan& p, int t, const RegLds& x, const double2* __restrict__ tw,
+                                        Ld load, Last last) {
+    reg_radix<NST>(p.r[0], [&](auto rc) {
+        constexpr int R = decltype(rc)::value;
+        if (t < p.nb[0]) {
+            double2 v[R];
+#pragma unroll
+            for (int r = 0; r < R; ++r) v[r] = load(t + r * p.nb[0]);
+            dft_reg<R, DIR>(v);
+#pragma unroll
+            for (int r = 0; r < R; ++r) x.at(x.sA, t, r) = v[r];
+        }
+    });
+    if constexpr (NST == 3) {
+        reg_radix<NST>(p.r[1], [&](auto rc) {
+            constexpr int R = decltype(rc)::value;
+            const int tc = min(t, p.nb[1] - 1), q = tc / p.r[0], k = tc - q * p.r[0];
+            double2 v[R];
+            reg_gather<R, DIR>(v, tw, k * p.r[2], [&](int r) { return x.at(x.sA, q + r * p.r[2], k); });
+            __syncthreads();   // every input of this stage has been read
+            if (t < p.nb[1]) {
+#pragma unroll
+                for (int r = 0; r < R; ++r) x.at(x.sB, q, k + r * p.r[0]) = v[r];
+            }
+        });
+    }
+    reg_radix<NST>(p.r[NST - 1], [&](auto rc) {
+        constexpr int R = decltype(rc)::value;
+        const int nb = p.nb[NST - 1], tc = min(t, nb - 1);
+        double2 v[R];
+        reg_gather<R, DIR>(v, tw, tc, [&](int r) { return x.at(NST == 2 ? x.sA : x.sB, r, tc); });
+        last(v, nb, rc);
+    });
+}
+
+// z: 8 kx columns (128 bytes of a row of S) of JB rows j per block
+template <int NST, int DIR>
+__global__ void __launch_bounds__(NST == 2 ? 256 : 1024) k_reg_z(double2* __restrict__ S, int M, int LH, int LHP,
+                                                                RegPlan p, int JB, const double2* __restrict__ tw) {
+    extern __shared__ unsigned char smem_raw[];
+    const int c = threadIdx.x & 7, u = threadIdx.x >> 3;
+    const int jj = (int)(((float)u + 0.5f) * p.Tinv), t = u - jj * p.T;
+    const int j = blockIdx.y * JB + jj, kx = blockIdx.x * 8 + c;   // kx < LHP, a multiple of 8
+    const size_t kst = (size_t)M * LHP;
+    double2* col = S + (size_t)min(j, M - 1) * LHP + kx;
+    const bool ok = j < M && kx < LH;
+    const RegLds x{reinterpret_cast<double2*>(smem_raw) + (size_t)jj * p.n * 8 + c, 8, p.r[0], p.r[0] * p.r[1]};
+    reg_fft<NST, DIR>(p, t, x, tw, [&](int i) { return col[i * kst]; },
+                      [&](auto& v, int nb, auto rc) {
+                          if (!ok || t >= nb) return;
+#pragma unroll
+                          for (int r = 0; r < decltype(rc)::value; ++r) col[(size_t)(t + r * nb) * kst] = v[r];
+                      });
+}
+
+// x forward: pairs of real rows, blockDim.x / T pairs per block
+template <int NST>
+__global__ void __launch_bounds__(256) k_reg_x_fwd(const double* __restrict__ f, double2* __restrict__ S, int nrows,
+                                                   int LHP, RegPlan p, const double2* __restrict__ tw) {
+    extern __shared__ unsigned char smem_raw[];
+    const int T = p.T, L = p.n, PB = blockDim.x / T;
+    const int pr = (int)(((float)threadIdx.x + 0.5f) * p.Tinv), t = threadIdx.x - pr * T;
+    const int ra = (blockIdx.x * PB + pr) * 2;
+    const double* fa = f + (size_t)min(ra, nrows - 1) * L;
+    const double* fb = f + (size_t)min(ra + 1, nrows - 1) * L;
+    double2* Z = reinterpret_cast<double2*>(smem_raw) + (size_t)pr * (L + T);
+    const RegLds x{Z, 1, p.r[0] | 1, (p.r[0] * p.r[1]) | 1};
+    reg_fft<NST, -1>(p, t, x, tw, [&](int i) { return make_double2(fa[i], fb[i]); },
+                     [&](auto& v, int nb, auto rc) {
+                         __syncthreads();   // every input has been read: the outputs in natural order
+                         if (t < nb) {
+#pragma unroll
+                             for (int r = 0; r < decltype(rc)::value; ++r) Z[t + r * nb] = v[r];
+                         }
+                     });
+    __syncthreads();
+    // split the two real rows: A = (Z_k + conj Z_{L-k}) / 2, B = (Z_k - conj Z_{L-k}) / (2i)
+    const int LH = L / 2 + 1;
+    double2* Sa = S + (size_t)ra * LHP;
+    for (int kx = t; kx < LH; kx += T) {
+        const double2 z = Z[kx], zc = Z[kx == 0 ? 0 : L - kx];
+        if (ra < nrows) Sa[kx] = make_double2(0.5 * (z.x + zc.x), 0.5 * (z.y - zc.y));
+        if (ra + 1 < nrows) Sa[LHP + kx] = make_double2(0.5 * (z.y + zc.y), -0.5 * (z.x - zc.x));
+    }
+}
+
+// x inverse: as k_fft_x_inv, ghost planes zero (ghost = 0) or Neumann copies (1)
+template <int NST>
+__global__ void __launch_bounds__(256) k_reg_x_inv(const double2* __restrict__ S, double* __restrict__ dph, int M,
+                                                   int nrows, int LHP, int ghost, RegPlan p,
+                                                   const double2* __restrict__ tw) {
+    extern __shared__ unsigned char smem_raw[];
+    const int T = p.T, L = p.n, PB = blockDim.x / T;
+    const int pr = (int)(((float)threadIdx.x + 0.5f) * p.Tinv), t = threadIdx.x - pr * T;
+    const int ra = (blockIdx.x * PB + pr) * 2;
+    const double2* Sa = S + (size_t)min(ra, nrows - 1) * LHP;
+    const double2* Sb = S + (size_t)min(ra + 1, nrows - 1) * LHP;
+    const RegLds x{reinterpret_cast<double2*>(smem_raw) + (size_t)pr * (L + T), 1, p.r[0] | 1,
+                   (p.r[0] * p.r[1]) | 1};
+    const size_t plane = (size_t)L * (M + 2);
+    reg_fft<NST, 1>(
+        p, t, x, tw,
+        [&](int n) {
+            const bool up = 2 * n > L;
+            const int m = up ? L - n : n;
+            double2 A = Sa[m], B = Sb[m];
+            if (m == 0 || 2 * m == L) A.y = B.y = 0.0;   // b_0 = b_{L/2} = 0 (FFT99 ordering)
+            // Z[m] = A + iB; Z[L-m] = conj(A) + i conj(B)
+            return up ? make_double2(A.x + B.y, B.x - A.y) : make_double2(A.x - B.y, A.y + B.x);
+        },
+        [&](auto& v, int nb, auto rc) {
+            if (t >= nb) return;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int row = ra + h;
+                if (row >= nrows) continue;
+                const int k = row / M, j = row - k * M;
+                double* base = dph + (size_t)k * plane + t;
+                double* o = base + (size_t)(j + 1) * L;
+#pragma unroll
+                for (int r = 0; r < decltype(rc)::value; ++r) o[r * nb] = h ? v[r].y : v[r].x;
+                if (j == 0) {
+#pragma unroll
+                    for (int r = 0; r < decltype(rc)::value; ++r) base[r * nb] = ghost == 1 ? (h ? v[r].y : v[r].x) : 0.0;
+                }
+                if (j == M - 1) {
+                    double* g = base + (size_t)(M + 1) * L;
+#pragma unroll
+                    for (int r = 0; r < decltype(rc)::value; ++r) g[r * nb] = ghost == 1 ? (h ? v[r].y : v[r].x) : 0.0;
+                }
+            }
+        });
 }
 
 // ---- y: tridiagonal solve per (kx, kz) line, FP64 --------------------------
@@ -678,8 +882,47 @@ static int poisson_pass(chs_handle* h, const TI* f, double* dph, int ghost, cpx_
         set_error("poisson: the fused residual transform needs NCL1 = 256");
         return CHS_E_ARG;
     }
+    // FP64, other lengths: register transforms where the length has a plan
+    // (the FP32 spectra keep their Stockham stages and so their roundings)
+    RegPlan rx, rxi, rz;
+    const bool xr = !f32 && !x256 && reg_plan(L, true, &rx) && reg_plan(L, false, &rxi);
+    const bool zr = !f32 && !z256 && reg_plan(N, false, &rz);
+    const int pb = xr ? std::max(1, (rx.nst == 2 ? 128 : 256) / rx.T) : 1;   // row pairs per block
+    const dim3 gxr((nrows + 2 * pb - 1) / (2 * pb)), bxr(pb * (xr ? rx.T : 1));
+    const size_t smxr = xr ? sizeof(double2) * (size_t)pb * (L + rx.T) : 0;
+    const int jb = zr ? std::max(1, 16 / rz.T) : 1;   // rows j per block: 128 threads at least
+    const dim3 gzr(LHP / 8, (M + jb - 1) / jb), bzr(8 * jb * (zr ? rz.T : 1));
+    const size_t smzr = zr ? sizeof(double2) * (size_t)8 * jb * N : 0;
+    auto fft_z_reg = [&](int dir) -> int {
+        if constexpr (!f32) {
+            if (rz.nst == 2 && dir < 0)
+                CHS_LAUNCH((k_reg_z<2, -1>), gzr, bzr, smzr, s, S, M, LH, LHP, rz, jb, twz);
+            else if (rz.nst == 2)
+                CHS_LAUNCH((k_reg_z<2, 1>), gzr, bzr, smzr, s, S, M, LH, LHP, rz, jb, twz);
+            else if (dir < 0)
+                CHS_LAUNCH((k_reg_z<3, -1>), gzr, bzr, smzr, s, S, M, LH, LHP, rz, jb, twz);
+            else
+                CHS_LAUNCH((k_reg_z<3, 1>), gzr, bzr, smzr, s, S, M, LH, LHP, rz, jb, twz);
+        }
+        return CHS_OK;
+    };
+    auto fft_x_reg = [&](int dir) -> int {
+        if constexpr (!f32) {
+            if (rx.nst == 2 && dir < 0)
+                CHS_LAUNCH((k_reg_x_fwd<2>), gxr, bxr, smxr, s, f, S, nrows, LHP, rx, twx);
+            else if (dir < 0)
+                CHS_LAUNCH((k_reg_x_fwd<3>), gxr, bxr, smxr, s, f, S, nrows, LHP, rx, twx);
+            else if (rx.nst == 2)
+                CHS_LAUNCH((k_reg_x_inv<2>), gxr, bxr, smxr, s, S, dph, M, nrows, LHP, ghost, rxi, twx);
+            else
+                CHS_LAUNCH((k_reg_x_inv<3>), gxr, bxr, smxr, s, S, dph, M, nrows, LHP, ghost, rxi, twx);
+        }
+        return CHS_OK;
+    };
     h->timer.begin(rphi ? "resid_fft_x" : "fft_x_fwd", s, &ev);
-    if (rphi != nullptr)
+    if (xr)
+        CHS_TRY(fft_x_reg(-1));
+    else if (rphi != nullptr)
         CHS_LAUNCH((k_fft256_x_fwd_res<Rl>), dim3(8 * ((gx16.x + 7) / 8)), dim3(128), sm16x, s, rphi, (const double*)f, S, M, nrows, LHP,
                    twx, h->dxqi, h->dzqi, h->amph, h->acph, h->apph);
     else if (x256)
@@ -690,7 +933,9 @@ static int poisson_pass(chs_handle* h, const TI* f, double* dph, int ghost, cpx_
     const dim3 gz((LH + ZTX - 1) / ZTX, M);
     const size_t smz = sizeof(cpx_t<Rl>) * (size_t)2 * ZTX * N;
     h->timer.begin("fft_z", s, &ev);
-    if (z256)
+    if (zr)
+        CHS_TRY(fft_z_reg(-1));
+    else if (z256)
         CHS_LAUNCH((k_fft256_z<Rl, ZCB>), gz16, dim3(16 * ZCB), sm16z, s, S, M, LH, LHP, -1, twz);
     else
         CHS_LAUNCH(k_fft_z<Rl>, gz, dim3(256), smz, s, S, N, M, LH, LHP, -1, pz, twz);
@@ -731,13 +976,17 @@ static int poisson_pass(chs_handle* h, const TI* f, double* dph, int ghost, cpx_
     }
     h->timer.end(ev, "poisson_y", s);
     h->timer.begin("fft_z", s, &ev);
-    if (z256)
+    if (zr)
+        CHS_TRY(fft_z_reg(1));
+    else if (z256)
         CHS_LAUNCH((k_fft256_z<Rl, ZCB>), gz16, dim3(16 * ZCB), sm16z, s, S, M, LH, LHP, +1, twz);
     else
         CHS_LAUNCH(k_fft_z<Rl>, gz, dim3(256), smz, s, S, N, M, LH, LHP, +1, pz, twz);
     h->timer.end(ev, "fft_z", s);
     h->timer.begin("fft_x_inv", s, &ev);
-    if (x256)
+    if (xr)
+        CHS_TRY(fft_x_reg(1));
+    else if (x256)
         CHS_LAUNCH(k_fft256_x_inv<Rl>, gx16, dim3(128), sm16x, s, S, dph, M, nrows, LHP, ghost, twx, phf);
     else
         CHS_LAUNCH(k_fft_x_inv<Rl>, gx, dim3(256), smx, s, S, dph, L, M, nrows, LHP, ghost, px, twx);
