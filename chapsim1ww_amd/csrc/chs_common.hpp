@@ -191,6 +191,50 @@ inline int march_chunk_rows(int rows, int nkg, size_t smem, int lds_max, bool fi
     return (rows + nyc - 1) / nyc;
 }
 
+// xz-plane sums in two stages of a fixed order: one block of 256 threads per
+// (row j, chunk of kc z rows) leaves its NM sums in part[(chunk M + j) NM + m],
+// then k_xz_finish adds a row's chunks and scales.  Chunks: about 2048 blocks,
+// at least 4 z rows each, at most what cap values hold.
+inline int xz_chunk(int M, int N, int nm, long cap) {
+    const int nch = (int)std::max(1L, std::min({(long)(N + 3) / 4, (2048L + M - 1) / M, cap / ((long)nm * M)}));
+    return (N + nch - 1) / nch;
+}
+// The block's tile: each XCD walks rows in j order, whose v(j + 1) is the next
+// tile's v(j).  f(i, k) for the cells of the tile this thread sums: lanes
+// along i, the block's remaining threads along k.
+struct XzTile {
+    int j, ch;
+    __device__ __forceinline__ bool pick(int M, int nch) {
+        const int t = xcd_tile(blockIdx.x, gridDim.x);
+        j = t % M;
+        ch = t / M;
+        return t < M * nch;
+    }
+    template <class F>
+    __device__ __forceinline__ void cells(int L, int N, int kc, F f) const {
+        const int Lr = min(256, (L + 63) & ~63), R = 256 / Lr;
+        const int r = threadIdx.x / Lr, i0 = threadIdx.x - r * Lr, k1 = min(N, (ch + 1) * kc);
+        if (r >= R) return;
+        for (int k = ch * kc + r; k < k1; k += R)   // unrolled: 299 -> 342 us (k_mean_xz_io), 110 -> 107 us (k_mean_xz)
+            for (int i = i0; i < L; i += Lr) f(i, k);
+    }
+};
+// The block's sums of acc[0..NM-1] to out (a shuffle tree per wave, then the
+// four waves in order); 256 threads, red: 4 NM doubles of LDS.
+template <int NM>
+__device__ __forceinline__ void xz_block_sums(const double (&acc)[NM], double* red, double* __restrict__ out) {
+#pragma unroll
+    for (int m = 0; m < NM; ++m) {
+        double v = acc[m];
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+        if ((threadIdx.x & 63) == 0) red[(threadIdx.x >> 6) * NM + m] = v;
+    }
+    __syncthreads();
+    const int m = threadIdx.x;
+    if (m < NM) out[m] = (red[m] + red[NM + m]) + (red[2 * NM + m] + red[3 * NM + m]);
+}
+
 struct CnCache;   // truncated-inverse CN stencils of one handle (substep.hip)
 
 }  // namespace chs
@@ -244,7 +288,9 @@ struct chs_handle {
     // the mixed-precision substep's convergence check, fused into its
     // projection and read back without a wait: the largest max|r| / bound
     // since the last reported error and the latest max|r|, max|f| land in
-    // pinned chk_host when chk_ev completes; chk_tol is the latest bound
+    // pinned chk_host[0..2] when chk_ev completes; chk_tol is the latest bound.
+    // chk_host[4], [5]: max|div u| and the CFL rate, written by their reduction
+    // kernel (coherent mapped memory) and read after the stream's sync
     bool chk_pending;
     double chk_tol;
     double* chk_host;

@@ -6,10 +6,9 @@
 //   chs_mean_t      PP_MEAN_T_TG / PP_MEAN_T_Xperiodic_IO
 //                   (src/processing/PP_MEAN_T.f90:322-370, 436-470)
 //   chs_mean_t_reset PP_TMEAN_INI_ZERO_TG / _IO (src/processing/PP_MEAN_T.f90:29-54, 110-319)
-// One block per row j sums its L x N cells in a fixed order (per-thread
-// strided partial sums, then a tree over the block), so every result is
-// deterministic.  The last xz means stay on the device (chs_handle::stats)
-// for the time means.
+// Blocks sum chunks of z rows of a row j and a second pass adds a row's chunks,
+// both in a fixed order, so every result is deterministic.  The last xz means
+// stay on the device (chs_handle::stats) for the time means.
 #include "chs_common.hpp"
 
 namespace chs {
@@ -21,24 +20,28 @@ struct StatGeo {
     int L, M, N;
 };
 
-// Row J = blockIdx.x + 1 of the (L, 0:M+1, N[,3]) io arrays.  Column order
-// as in include/chapsim_gpu.h (chs_mean_xz_io).  The channel has RCCI1 = 1,
-// so v and w's cell averages carry the factor 1.0 the reference multiplies.
-__global__ void __launch_bounds__(128) k_mean_xz_io(StatGeo g, const double* __restrict__ Q,
+// One chunk of z rows of one row of the (L, 0:M+1, N[,3]) io arrays.  Column
+// order as in include/chapsim_gpu.h (chs_mean_xz_io).  The channel has RCCI1 =
+// 1, so v and w's cell averages carry the factor 1.0 the reference multiplies.
+// Bound: HBM, 88 B/cell (11 fields read once).  One block per row left a
+// quarter of the CUs without work and the others with two waves: 976 us at
+// 256x192x256 (1.1 TB/s), in chunks 299 us (3.7 TB/s).
+__global__ void __launch_bounds__(256) k_mean_xz_io(StatGeo g, const double* __restrict__ Q,
                                                     const double* __restrict__ Gf, const double* __restrict__ PR,
                                                     const double* __restrict__ T, const double* __restrict__ RHO,
                                                     const double* __restrict__ H, const double* __restrict__ MU,
-                                                    int thermal, double* __restrict__ out) {
-    __shared__ double red[NIO][128];
-    const int L = g.L, N = g.N, J = blockIdx.x + 1;
-    const int LP = L * (g.M + 2), CS = LP * N;
+                                                    int thermal, int kc, int nch, double* __restrict__ part) {
+    __shared__ double red[4 * NIO];
+    const int L = g.L, N = g.N;
+    XzTile t;
+    if (!t.pick(g.M, nch)) return;
+    const int LP = L * (g.M + 2), CS = LP * N, row = L * (t.j + 1);
     double acc[NIO];
 #pragma unroll
     for (int m = 0; m < NIO; ++m) acc[m] = 0.0;
-    for (int e = threadIdx.x; e < L * N; e += blockDim.x) {
-        const int k = e / L, i = e - k * L;
-        const int ip = i == L - 1 ? 0 : i + 1, kp = k == N - 1 ? 0 : k + 1;
-        const int o = i + L * J + LP * k, oip = o - i + ip, okp = o + LP * (kp - k);
+    t.cells(L, N, kc, [&](int i, int k) {
+        const int o = i + row + LP * k;
+        const int oip = o + (i == L - 1 ? 1 - L : 1), okp = o + (k == N - 1 ? (1 - N) * LP : LP);
         double U[3], G[3];
         G[0] = (Gf[o] + Gf[oip]) * 0.5;
         U[0] = (Q[o] + Q[oip]) * 0.5;
@@ -63,12 +66,12 @@ __global__ void __launch_bounds__(128) k_mean_xz_io(StatGeo g, const double* __r
                 acc[10 + l] += U[m] * U[n];
             }
         if (thermal) {
-            const double t = T[o], d = RHO[o], hh = H[o], v = MU[o];
-            acc[22] += t;
+            const double tt = T[o], d = RHO[o], hh = H[o], v = MU[o];
+            acc[22] += tt;
             acc[23] += d;
             acc[24] += hh;
             acc[25] += v;
-            acc[26] += t * t;
+            acc[26] += tt * tt;
             acc[27] += d * d;
             acc[28] += hh * hh;
             acc[29] += hh * d;
@@ -79,20 +82,17 @@ __global__ void __launch_bounds__(128) k_mean_xz_io(StatGeo g, const double* __r
                 acc[34 + m] += hh * G[m];
             }
         }
-    }
-#pragma unroll
-    for (int m = 0; m < NIO; ++m) red[m][threadIdx.x] = acc[m];
-    __syncthreads();
-    for (int st = blockDim.x / 2; st > 0; st >>= 1) {
-        if ((int)threadIdx.x < st)
-#pragma unroll
-            for (int m = 0; m < NIO; ++m) red[m][threadIdx.x] += red[m][threadIdx.x + st];
-        __syncthreads();
-    }
-    if (threadIdx.x < NIO) {
-        const double VL = 1.0 / (double)(L * N);
-        out[NIO * (J - 1) + threadIdx.x] = red[threadIdx.x][0] * VL;
-    }
+    });
+    xz_block_sums(acc, red, part + (size_t)NIO * (t.ch * g.M + t.j));
+}
+
+// out[e] = scale sum over the chunks of part[c n + e], e < n = 37 M
+__global__ void k_xz_finish(const double* __restrict__ part, int n, int nch, double scale, double* __restrict__ out) {
+    const int e = blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= n) return;
+    double s = 0.0;
+    for (int c = 0; c < nch; ++c) s += part[(size_t)c * n + e];
+    out[e] = s * scale;
 }
 
 // acc = coe3 acc + coe2 val over n values
@@ -123,9 +123,12 @@ int mean_xz_io(chs_handle* h, const chs_thermal_fields* tf, const chs_io_fields*
     const hipStream_t s = h->stream;
     double* xz = xz_of(h, 1);
     const StatGeo g{h->L, h->M, h->N};
-    CHS_LAUNCH(k_mean_xz_io, dim3(h->M), dim3(128), 0, s, g, f->q, f->g, f->pr, thermal ? tf->temperature : nullptr,
-               thermal ? tf->density : nullptr, thermal ? tf->enthalpy : nullptr, thermal ? tf->viscosity : nullptr,
-               thermal, xz);
+    const int kc = xz_chunk(h->M, h->N, NIO, 2L * h->npart), nch = (h->N + kc - 1) / kc, n = NIO * h->M;
+    CHS_LAUNCH(k_mean_xz_io, dim3(8 * ((h->M * nch + 7) / 8)), dim3(256), 0, s, g, f->q, f->g, f->pr,
+               thermal ? tf->temperature : nullptr, thermal ? tf->density : nullptr, thermal ? tf->enthalpy : nullptr,
+               thermal ? tf->viscosity : nullptr, thermal, kc, nch, h->partials);
+    CHS_LAUNCH(k_xz_finish, dim3((n + 255) / 256), dim3(256), 0, s, h->partials, n, nch,
+               1.0 / ((double)h->L * (double)h->N), xz);
     if (out_host) {
         CHS_HIP(hipMemcpyAsync(out_host, xz, (size_t)NIO * h->M * sizeof(double), hipMemcpyDeviceToHost, s));
         CHS_HIP(hipStreamSynchronize(s));

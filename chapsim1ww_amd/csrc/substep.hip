@@ -1155,61 +1155,86 @@ __global__ void __launch_bounds__(256) k_update(Geo g, double cu, double cw, dou
 }
 
 // max |div u| (DIVGCK_tg, src/DIVGCK.f90:33-46) and max CFL rate (CFL_tg,
-// src/CFL.f90:39-53) in one sweep: part[2b] = div, part[2b+1] = cfl.
+// src/CFL.f90:39-53) in one sweep: part[2b] = div, part[2b+1] = cfl.  Tiles of
+// 64 i x 4 k x DVJ rows as k_divg (v's row J+1 of one cell is row J of the
+// next), each XCD walking a contiguous range of them in j order with
+// gridDim.x / 8 blocks.  Bound: HBM, 24 B/cell: at 256x192x256 76 us with one
+// cell per thread and 64-bit index divisions, 61 us (5.0 TB/s) in tiles.
 __global__ void __launch_bounds__(256) k_divgck_cfl(Geo g, const double* __restrict__ Q, double* __restrict__ part) {
-    __shared__ double red[2][256];
-    const size_t ncell = (size_t)g.L * g.M * g.N;
+    __shared__ double red[2][4];
+    const int L = g.L, M = g.M, N = g.N;
+    const int LP = L * (M + 2), CS = LP * N;
+    const int ni = (L + 63) / 64, nk = (N + 3) / 4, ng = (M + DVJ - 1) / DVJ;
+    const int nt = ni * ng * nk, per = (nt + 7) / 8;
+    const int xcd = blockIdx.x % 8, nq = gridDim.x / 8, t1 = min(nt, (xcd + 1) * per);
+    const int li = threadIdx.x & 63, lk = threadIdx.x >> 6;
     double md = 0.0, mc = 0.0;
-    for (size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x; t < ncell; t += (size_t)gridDim.x * blockDim.x) {
-        const int i = t % g.L;
-        const int j = (t / g.L) % g.M;
-        const int k = t / ((size_t)g.L * g.M);
-        const int ip = i == g.L - 1 ? 0 : i + 1, kp = k == g.N - 1 ? 0 : k + 1;
-        const int J = j + 1;
-        const double u0 = Q[qidx(g, 0, i, J, k)], u1 = Q[qidx(g, 0, ip, J, k)];
-        const double v0 = Q[qidx(g, 1, i, J, k)], v1 = Q[qidx(g, 1, i, J + 1, k)];
-        const double w0 = Q[qidx(g, 2, i, J, k)], w1 = Q[qidx(g, 2, i, J, kp)];
-        const double D = (u1 - u0) * g.dxi + (v1 - v0) * g.dyfi[j] * 1.0 + (w1 - w0) * g.dzi * 1.0;
-        const double C = (fabs((u0 + u1) * g.dxi) + fabs((v0 + v1) * g.dyfi[j] * 1.0) + fabs((w0 + w1) * g.dzi * 1.0)) * 0.5;
-        // NaN-propagating maxima: a NaN anywhere makes the result NaN
-        md = nanmax(md, fabs(D));
-        mc = nanmax(mc, C);
-    }
-    red[0][threadIdx.x] = md;
-    red[1][threadIdx.x] = mc;
-    __syncthreads();
-    for (int s = blockDim.x / 2; s > 0; s >>= 1) {
-        if (threadIdx.x < s) {
-            red[0][threadIdx.x] = nanmax(red[0][threadIdx.x], red[0][threadIdx.x + s]);
-            red[1][threadIdx.x] = nanmax(red[1][threadIdx.x], red[1][threadIdx.x + s]);
+    for (int t = xcd * per + (int)blockIdx.x / 8; t < t1; t += nq) {
+        const int it = t % ni, rr = t / ni, jg = rr % ng, kt = rr / ng;
+        // lanes past the grid and rows past M evaluate a cell again
+        const int i = min(it * 64 + li, L - 1), k = min(kt * 4 + lk, N - 1), j0 = jg * DVJ;
+        const int ip = i == L - 1 ? 1 - L : 1, kp = k == N - 1 ? (1 - N) * LP : LP;
+        const double *U = Q + (i + L * (j0 + 1) + LP * k), *V = U + CS, *W = V + CS;
+        double u0[DVJ], u1[DVJ], w0[DVJ], w1[DVJ], v[DVJ + 1];
+#pragma unroll
+        for (int r = 0; r < DVJ; ++r) {
+            const int o = L * (min(j0 + r, M - 1) - j0);
+            u0[r] = U[o];
+            u1[r] = U[o + ip];
+            w0[r] = W[o];
+            w1[r] = W[o + kp];
         }
-        __syncthreads();
+#pragma unroll
+        for (int r = 0; r <= DVJ; ++r) v[r] = V[L * (min(j0 + r, M) - j0)];
+#pragma unroll
+        for (int r = 0; r < DVJ; ++r) {
+            if (j0 + r >= M) break;
+            const double dy = ldc(g.dyfi, j0 + r);
+            const double D = (u1[r] - u0[r]) * g.dxi + (v[r + 1] - v[r]) * dy * 1.0 + (w1[r] - w0[r]) * g.dzi * 1.0;
+            const double C = (fabs((u0[r] + u1[r]) * g.dxi) + fabs((v[r] + v[r + 1]) * dy * 1.0) +
+                              fabs((w0[r] + w1[r]) * g.dzi * 1.0)) * 0.5;
+            // NaN-propagating maxima: a NaN anywhere makes the result NaN
+            md = nanmax(md, fabs(D));
+            mc = nanmax(mc, C);
+        }
     }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        md = nanmax(md, __shfl_xor(md, o));
+        mc = nanmax(mc, __shfl_xor(mc, o));
+    }
+    if (li == 0) {
+        red[0][lk] = md;
+        red[1][lk] = mc;
+    }
+    __syncthreads();
     if (threadIdx.x == 0) {
-        part[2 * blockIdx.x] = red[0][0];
-        part[2 * blockIdx.x + 1] = red[1][0];
+        part[2 * blockIdx.x] = nanmax(nanmax(red[0][0], red[0][1]), nanmax(red[0][2], red[0][3]));
+        part[2 * blockIdx.x + 1] = nanmax(nanmax(red[1][0], red[1][1]), nanmax(red[1][2], red[1][3]));
     }
 }
 
 // xz-mean statistics of PP_MEAN_ZX_FLOW_TG (src/processing/PP_MEAN_ZX.f90:
-// 104-237), first and second moments: one block per row j, out[13 j + m] as the
-// C ABI documents (cell-centred u, v, w sums, p, their products, u p).
+// 104-237), first and second moments: one chunk of z rows of row j per block
+// (xz_chunk), out[13 j + m] as the C ABI documents (cell-centred u, v, w sums,
+// p, their products, u p).  Bound: HBM, 32 B/cell.  One block per row: 186 us
+// at 256x192x256 (2.2 TB/s), in chunks 110 us (3.7 TB/s).
 __global__ void __launch_bounds__(256) k_mean_xz(Geo g, const double* __restrict__ Q, const double* __restrict__ PR,
-                                                 double* __restrict__ out) {
-    __shared__ double red[13][256];
-    const int L = g.L, N = g.N, j = blockIdx.x, J = j + 1;
-    const int LP = L * (g.M + 2), CS = LP * N;
+                                                 int kc, int nch, double* __restrict__ part) {
+    __shared__ double red[4 * 13];
+    const int L = g.L, N = g.N;
+    XzTile t;
+    if (!t.pick(g.M, nch)) return;
+    const int LP = L * (g.M + 2), CS = LP * N, row = L * (t.j + 1);
     double acc[13];
 #pragma unroll
     for (int m = 0; m < 13; ++m) acc[m] = 0.0;
-    for (int e = threadIdx.x; e < L * N; e += blockDim.x) {
-        const int k = e / L, i = e - k * L;
-        const int ip = i == L - 1 ? 0 : i + 1, kp = k == N - 1 ? 0 : k + 1;
-        const int o = i + L * J + LP * k;
+    t.cells(L, N, kc, [&](int i, int k) {
+        const int o = i + row + LP * k;
         double U[3];
-        U[0] = Q[o] + Q[o - i + ip];
+        U[0] = Q[o] + Q[o + (i == L - 1 ? 1 - L : 1)];
         U[1] = Q[CS + o] + Q[CS + o + L];
-        U[2] = Q[2 * CS + o] + Q[2 * CS + o + LP * (kp - k)];
+        U[2] = Q[2 * CS + o] + Q[2 * CS + o + (k == N - 1 ? (1 - N) * LP : LP)];
         const double P = PR[o];
 #pragma unroll
         for (int m = 0; m < 3; ++m) {
@@ -1222,44 +1247,48 @@ __global__ void __launch_bounds__(256) k_mean_xz(Geo g, const double* __restrict
         for (int m = 0; m < 3; ++m)
 #pragma unroll
             for (int n = m; n < 3; ++n) acc[l++] += U[m] * U[n];
-    }
-#pragma unroll
-    for (int m = 0; m < 13; ++m) red[m][threadIdx.x] = acc[m];
-    __syncthreads();
-    for (int st = blockDim.x / 2; st > 0; st >>= 1) {
-        if ((int)threadIdx.x < st)
-#pragma unroll
-            for (int m = 0; m < 13; ++m) red[m][threadIdx.x] += red[m][threadIdx.x + st];
-        __syncthreads();
-    }
-    if (threadIdx.x < 13) {
-        const int m = threadIdx.x;
-        const double VL = 1.0 / (double)(L * N);
-        const double c = m == 3 ? VL : (m >= 4 && m < 10) ? VL * (0.5 * 0.5) : VL * 0.5;
-        out[13 * j + m] = red[m][0] * c;
-    }
+    });
+    xz_block_sums(acc, red, part + (size_t)13 * (t.ch * g.M + t.j));
 }
 
-__global__ void k_reduce_max2_nan(const double* __restrict__ part, int nb, double* __restrict__ out) {
-    __shared__ double red[2][256];
-    double a = 0.0, b = 0.0;
-    for (int i = threadIdx.x; i < nb; i += blockDim.x) {
-        a = nanmax(a, part[2 * i]);
-        b = nanmax(b, part[2 * i + 1]);
+// the rows' chunks added in order, and the reference's scaling
+__global__ void k_mean_xz_finish(const double* __restrict__ part, int n, int nch, double VL, double* __restrict__ out) {
+    const int e = blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= n) return;
+    const int m = e % 13;
+    double s = 0.0;
+    for (int c = 0; c < nch; ++c) s += part[(size_t)c * n + e];
+    out[e] = s * (m == 3 ? VL : (m >= 4 && m < 10) ? VL * (0.5 * 0.5) : VL * 0.5);
+}
+
+// NaN-propagating maxima of nb <= 1024 pairs, one per thread
+__global__ void __launch_bounds__(1024) k_reduce_max2_nan(const double* __restrict__ part, int nb,
+                                                          double* __restrict__ out) {
+    __shared__ double red[2][16];
+    const int i = threadIdx.x;
+    double a = i < nb ? part[2 * i] : 0.0, b = i < nb ? part[2 * i + 1] : 0.0;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        a = nanmax(a, __shfl_xor(a, o));
+        b = nanmax(b, __shfl_xor(b, o));
     }
-    red[0][threadIdx.x] = a;
-    red[1][threadIdx.x] = b;
+    if ((i & 63) == 0) {
+        red[0][i >> 6] = a;
+        red[1][i >> 6] = b;
+    }
     __syncthreads();
-    for (int s = blockDim.x / 2; s > 0; s >>= 1) {
-        if (threadIdx.x < s) {
-            red[0][threadIdx.x] = nanmax(red[0][threadIdx.x], red[0][threadIdx.x + s]);
-            red[1][threadIdx.x] = nanmax(red[1][threadIdx.x], red[1][threadIdx.x + s]);
+    if (i < 64) {
+        a = i < 16 ? red[0][i] : 0.0;
+        b = i < 16 ? red[1][i] : 0.0;
+#pragma unroll
+        for (int o = 8; o > 0; o >>= 1) {
+            a = nanmax(a, __shfl_xor(a, o));
+            b = nanmax(b, __shfl_xor(b, o));
         }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        out[0] = red[0][0];
-        out[1] = red[1][0];
+        if (i == 0) {
+            out[0] = a;
+            out[1] = b;
+        }
     }
 }
 
@@ -1908,17 +1937,17 @@ int divgck_cfl(chs_handle* h, double* div_out, double* cfl_out) {
     CHS_TRY(mixed_check(h, true));
     const Geo g = geo_of(h);
     const hipStream_t s = h->stream;
-    const int nb = 1024;
+    const long nt = (long)((h->L + 63) / 64) * ((h->N + 3) / 4) * ((h->M + DVJ - 1) / DVJ);
+    const int nb = (int)std::min(1024L, 8 * ((nt + 7) / 8));
     hipEvent_t ev;
     h->timer.begin("divgck_cfl", s, &ev);
     CHS_LAUNCH(k_divgck_cfl, dim3(nb), dim3(256), 0, s, g, h->q, h->partials);
-    CHS_LAUNCH(k_reduce_max2_nan, dim3(1), dim3(256), 0, s, h->partials, nb, h->scalars + 1);
+    // straight to pinned host memory: no copy between the kernel and the sync
+    CHS_LAUNCH(k_reduce_max2_nan, dim3(1), dim3(1024), 0, s, h->partials, nb, h->chk_host + 4);
     h->timer.end(ev, "divgck_cfl", s);
-    double host[2];
-    CHS_HIP(hipMemcpyAsync(host, h->scalars + 1, 2 * sizeof(double), hipMemcpyDeviceToHost, s));
     CHS_HIP(hipStreamSynchronize(s));
-    if (div_out) *div_out = host[0];
-    if (cfl_out) *cfl_out = host[1];
+    if (div_out) *div_out = h->chk_host[4];
+    if (cfl_out) *cfl_out = h->chk_host[5];
     return CHS_OK;
 }
 
@@ -1926,7 +1955,10 @@ int mean_xz(chs_handle* h, double* out_host) {
     const Geo g = geo_of(h);
     const hipStream_t s = h->stream;
     // kept on the device for the time means (chs_mean_t)
-    CHS_LAUNCH(k_mean_xz, dim3(h->M), dim3(256), 0, s, g, h->q, h->pr, h->stats);
+    const int kc = xz_chunk(h->M, h->N, 13, 2L * h->npart), nch = (h->N + kc - 1) / kc, n = 13 * h->M;
+    CHS_LAUNCH(k_mean_xz, dim3(8 * ((h->M * nch + 7) / 8)), dim3(256), 0, s, g, h->q, h->pr, kc, nch, h->partials);
+    CHS_LAUNCH(k_mean_xz_finish, dim3((n + 255) / 256), dim3(256), 0, s, h->partials, n, nch,
+               1.0 / ((double)h->L * (double)h->N), h->stats);
     CHS_HIP(hipMemcpyAsync(out_host, h->stats, 13 * (size_t)h->M * sizeof(double), hipMemcpyDeviceToHost, s));
     CHS_HIP(hipStreamSynchronize(s));
     return CHS_OK;
