@@ -5,8 +5,7 @@
 //   k_io_prepare   DENSITY_TIME_DERIVATION(NS) (src/THERM_PROP_UPDATE.f90:
 //                  225-291), DENSITY_Staggered, MU_Staggered and
 //                  VELOCITY_CALC_io (src/MASSFLUX_CALC_IO.f90:82-311)
-//   k_io_divu      DIVG_U_io (src/DIVG.f90:153-259)
-//   k_io_terms     CONVECTION_X/Y/Z_io (src/CONVECTION_X.f90:77-176,
+//   k_io_terms     DIVG_U_io (src/DIVG.f90:153-259), CONVECTION_X/Y/Z_io (src/CONVECTION_X.f90:77-176,
 //                  src/CONVECTION_Y.f90:128-287, src/CONVECTION_Z.f90:115-314),
 //                  VISCOUS_ALL_EXPLT_X/Y/Z_io (src/VISCOUS_X_EXPLICIT_io.f90:
 //                  1-113, src/VISCOUS_Y_EXPLICIT_io.f90:1-99,
@@ -285,17 +284,29 @@ __global__ void __launch_bounds__(256) k_io_prepare_m(IoGeo g, const double* __r
     }
 }
 
-// DIVG_U_io on rows 1..M and the y wrap of its ghost rows
-__global__ void __launch_bounds__(256) k_io_divu(IoGeo g, const double* __restrict__ Q, double* __restrict__ divu) {
+// x / 3.0, correctly rounded: one Newton correction of the product with the
+// rounded reciprocal (the remainder is exact in a fused multiply-add); an
+// infinity or NaN passes as the division would give it
+__device__ __forceinline__ double third(double x) {
+    const double y = 1.0 / 3.0, q = x * y;
+    const double r = fma(fma(-3.0, q, x), y, q);
+    return fabs(x) == __builtin_inf() ? q : r;
+}
+
+// DIVG_U_io (src/DIVG.f90:153-259) at the cell (di, dj, dk) from (IC, JC, KC),
+// formed where the stresses need it instead of read back from an array a pass
+// of its own filled: the velocities around the cell are at hand.
+__device__ __forceinline__ double io_divu_v(const IoGeo& g, double dyfi, double up, double u, double vp, double v,
+                                            double wp, double w) {
 #pragma clang fp contract(off)
-    IO_CELL(g.M + 2, 0);
-    const int J = JT;
-    const int Jr = J == 0 ? M : (J == M + 1 ? 1 : J);
-    const int c = at(IC, Jr, KC);
-    const double DIVX = (Q[at(IP, Jr, KC)] - Q[c]) * g.dxi;
-    const double DIVY = (Q[CS + at(IC, Jr + 1, KC)] - Q[CS + c]) * (ldc(g.dyfi, Jr - 1) * 1.0);
-    const double DIVZ = (Q[2 * CS + at(IC, Jr, KP)] - Q[2 * CS + c]) * (g.dzi * 1.0);
-    divu[at(IC, J, KC)] = (DIVX + DIVY + DIVZ) / 3.0;
+    const double DIVX = (up - u) * g.dxi, DIVY = (vp - v) * (dyfi * 1.0), DIVZ = (wp - w) * (g.dzi * 1.0);
+    return third(DIVX + DIVY + DIVZ);
+}
+template <class A>
+__device__ __forceinline__ double io_divu(const IoGeo& g, const A& Q1, const A& Q2, const A& Q3, int JC, int di,
+                                          int dj, int dk) {
+    return io_divu_v(g, ldc(g.dyfi, max(JC + dj, 1) - 1), Q1(di + 1, dj, dk), Q1(di, dj, dk), Q2(di, dj + 1, dk),
+                     Q2(di, dj, dk), Q3(di, dj, dk + 1), Q3(di, dj, dk));
 }
 
 template <int NT>
@@ -312,7 +323,7 @@ __device__ __forceinline__ double io_block_sum(double v, double* red) {
 }
 
 // Values of one array around the cell held in registers, for the offsets
-// the terms use: MU, MU0, DivU and PR at (0,0,0), (-1,0,0), (0,-1,0),
+// the terms use: MU, MU0, DivU (formed by io_divu) and PR at (0,0,0), (-1,0,0), (0,-1,0),
 // (0,0,-1); MU_STG x-y at (0,0,0), (0,1,0), (1,0,0); x-z at (0,0,0), (0,0,1),
 // (1,0,0); y-z at (0,0,0), (0,1,0), (0,0,1).
 struct IoV4 {
@@ -333,6 +344,21 @@ struct IoVS3 {
     double c, jp, kp;
     __device__ __forceinline__ double operator()(int, int dj, int dk) const { return dj > 0 ? jp : dk > 0 ? kp : c; }
 };
+
+// DivU at the cell and at i-1, j-1, k-1 (on row 1 the last but one is
+// evaluated from in-bounds rows and only enters what the callers discard)
+template <class A>
+__device__ __forceinline__ IoV4 io_divu4(const IoGeo& g, const A& Q1, const A& Q2, const A& Q3, int JC) {
+    return IoV4{io_divu(g, Q1, Q2, Q3, JC, 0, 0, 0), io_divu(g, Q1, Q2, Q3, JC, -1, 0, 0),
+                io_divu(g, Q1, Q2, Q3, JC, 0, -1, 0), io_divu(g, Q1, Q2, Q3, JC, 0, 0, -1)};
+}
+
+// DivU of the cell at offset c of row JC, with the y wrap of its ghost rows
+__device__ __forceinline__ void io_divu_store(const IoGeo& g, int JC, int c, double d, double* __restrict__ DU) {
+    DU[c] = d;
+    if (JC == g.M) DU[c - g.L * g.M] = d;   // row 0
+    if (JC == 1) DU[c + g.L * g.M] = d;     // row M+1
+}
 
 // CONVECTION_X/Y/Z_io at the cell: hx, hy, hz.  hy is evaluated on row 1
 // too (from in-bounds rows); the callers discard it there.
@@ -405,7 +431,7 @@ __device__ __forceinline__ void io_conv(const IoGeo& g, const double* __restrict
 template <int GRAV, class AQ, class AM, class AS1, class AS2, class AS3, class AP>
 __device__ __forceinline__ void io_terms_cell(const IoGeo& g, const AQ& G1, const AQ& G2, const AQ& G3,
                                               const AQ& Q1, const AQ& Q2, const AQ& Q3, const AM& MU,
-                                              const AM& MU0, const AM& DU, const AS1& MS1, const AS2& MS2,
+                                              const AM& MU0, const IoV4& DU, const AS1& MS1, const AS2& MS2,
                                               const AS3& MS3, const AP& PR, int JC, const double* E, double rsg,
                                               const IoParams& p, double tg, double tr, double dt, double adt,
                                               double* h, double* r) {
@@ -547,7 +573,7 @@ __device__ __forceinline__ double io_terms_store(const IoParams& p, const IoGeo&
 template <int GRAV>
 __global__ void __launch_bounds__(256) k_io_terms(IoGeo g, const double* __restrict__ G, const double* __restrict__ Q,
                                                   const double* __restrict__ MU, const double* __restrict__ MU0,
-                                                  const double* __restrict__ DU, const double* __restrict__ MS,
+                                                  double* __restrict__ DU, const double* __restrict__ MS,
                                                   const double* __restrict__ PR, const double* __restrict__ RS,
                                                   double* __restrict__ E, IoParams p, double tg, double tr, double dt,
                                                   double adt, double* __restrict__ inc, double* __restrict__ part,
@@ -572,8 +598,9 @@ __global__ void __launch_bounds__(256) k_io_terms(IoGeo g, const double* __restr
         const double Ev[3] = {E[e], E[NC + e], E[2 * NC + e]};
         const double rsg = GRAV == 0 ? 0.0 : RS[(GRAV - 1) * CS + c];
         double hv[3], rv[3];
+        const IoV4 du = io_divu4(g, A(Q), A(Q + CS), A(Q + 2 * CS), JC);
         io_terms_cell<GRAV>(g, A(G), A(G + CS), A(G + 2 * CS), A(Q), A(Q + CS), A(Q + 2 * CS), A(MU), A(MU0),
-                            A(DU), A(MS), A(MS + CS), A(MS + 2 * CS), A(PR), JC, Ev, rsg, p, tg, tr, dt, adt, hv, rv);
+                            du, A(MS), A(MS + CS), A(MS + 2 * CS), A(PR), JC, Ev, rsg, p, tg, tr, dt, adt, hv, rv);
         const int cg = c + (JC == 1 ? -L : L);
         const double gv[3] = {G[c], G[CS + c], G[2 * CS + c]};
         double glv[3] = {0.0, 0.0, 0.0};
@@ -583,6 +610,7 @@ __global__ void __launch_bounds__(256) k_io_terms(IoGeo g, const double* __restr
             glv[2] = G[2 * CS + cg];
         }
         flow = io_terms_store(p, g, JC, e, NC, hv, rv, E, inc, G0, c, cg, CS, gv, glv);
+        io_divu_store(g, JC, c, du.c, DU);
     }
     const double bs = io_block_sum<256>(flow, red);
     if (threadIdx.x == 0 && threadIdx.y == 0) part[tile] = bs;
@@ -596,18 +624,23 @@ __global__ void __launch_bounds__(256) k_io_terms(IoGeo g, const double* __restr
 // components, IOKR + 2 k rows each: the periodic z neighbours as halo rows),
 // so their stencil reads come from LDS and each value comes from global
 // memory once per block; the ring's next row is loaded while the current one
-// is computed.  MU, MU0, DivU, MU_STG, PR, RHO_STG and EXPLT0 are read from
+// is computed.  DivU comes from the ring's velocities, one evaluation per cell
+// shared through an LDS plane (at 256x192x256 its own pass, 89 us, and this
+// kernel's reads of it go for 616 -> 631 us here; formed three times per cell
+// instead: 729 us; its store kept after the others, since the branches of the
+// wrapped rows before the arithmetic cost 50 registers).  MU, MU0, MU_STG, PR,
+// RHO_STG and EXPLT0 are read from
 // global memory as in k_io_terms.  The mass-flux partial of row j goes to
 // part[kg*M + j].
 // ---------------------------------------------------------------------------
 constexpr int IOKR = 2, IOKP = IOKR + 2;
 
-inline size_t io_terms_m_smem(int L) { return sizeof(double) * ((size_t)3 * 6 * IOKP * L + 16); }
+inline size_t io_terms_m_smem(int L) { return sizeof(double) * ((size_t)3 * 6 * IOKP * L + 16 + (size_t)(IOKR + 1) * L); }
 
 template <int GRAV>
 __global__ void __launch_bounds__(512) k_io_terms_m(IoGeo g, const double* __restrict__ G,
                                                     const double* __restrict__ Q, const double* __restrict__ MU,
-                                                    const double* __restrict__ MU0, const double* __restrict__ DU,
+                                                    const double* __restrict__ MU0, double* __restrict__ DU,
                                                     const double* __restrict__ MS, const double* __restrict__ PR,
                                                     const double* __restrict__ RS, double* __restrict__ E,
                                                     IoParams p, double tg, double tr, double dt, double adt,
@@ -619,6 +652,7 @@ __global__ void __launch_bounds__(512) k_io_terms_m(IoGeo g, const double* __res
     const int PL = IOKP * L, SL = 6 * PL;  // one component / one ring row
     double* ring = sm;
     double* red = sm + 3 * SL;
+    double* dup = red + 16;                // DivU of the row, k0-1 .. k0+IOKR-1
     const int nt = (N / IOKR) * nyc, per = (nt + 7) / 8;
     const int t = (blockIdx.x % 8) * per + blockIdx.x / 8;  // XCD x: tiles x*per .. (x+1)*per-1
     if (t >= nt) return;
@@ -632,16 +666,17 @@ __global__ void __launch_bounds__(512) k_io_terms_m(IoGeo g, const double* __res
     const int kh = rb == 0 ? (k0 == 0 ? N - 1 : k0 - 1) : (k0 + IOKR == N ? 0 : k0 + IOKR);
     const int gc = i + LP * KC, gh = i + LP * kh;                   // global, row 0
     const int lc = (rb + 1) * L + i, lh = (rb == 0 ? 0 : IOKP - 1) * L + i;  // in a ring plane
+    const int ldh = rb == 0 ? i : lc;   // DivU halo: row k0-1, or the own cell once more
     const int ip = i == L - 1 ? 1 - L : 1, im = i == 0 ? L - 1 : -1;
     const int kp = KC == N - 1 ? (1 - N) * LP : LP, km = KC == 0 ? (N - 1) * LP : -LP;
     const double *MS1 = MS, *MS2 = MS + CS, *MS3 = MS + 2 * CS;
     // The values from global memory a step needs besides the ring, loaded one
-    // step ahead: row JC of MU, MU0, DivU, PR (cell, i-1, k-1), MU_STG (the
+    // step ahead: row JC of MU, MU0, PR (cell, i-1, k-1), MU_STG (the
     // cell's x-neighbour and z-neighbour entries), EXPLT0 and RHO_STG, and
-    // row JC+1 of MU_STG x-y and y-z; the j-1 entries of MU, MU0, DivU, PR and
+    // row JC+1 of MU_STG x-y and y-z; the j-1 entries of MU, MU0, PR and
     // the cell entries of MU_STG x-y, y-z carry over from the step before.
     struct Row {
-        double mu[3], mu0[3], du[3], pr[3];  // cell, i-1, k-1
+        double mu[3], mu0[3], pr[3];         // cell, i-1, k-1
         double s1ip, s2[3], s3kp;            // MS1(i+1); MS2 cell, k+1, i+1; MS3(k+1)
         double s1jp, s3jp;                   // MS1, MS3 at row JC+1
         double e[3], rs;
@@ -651,7 +686,6 @@ __global__ void __launch_bounds__(512) k_io_terms_m(IoGeo g, const double* __res
         const int e = i + L * (JL - 1) + L * M * KC;
         r.mu[0] = MU[c], r.mu[1] = MU[c + im], r.mu[2] = MU[c + km];
         r.mu0[0] = MU0[c], r.mu0[1] = MU0[c + im], r.mu0[2] = MU0[c + km];
-        r.du[0] = DU[c], r.du[1] = DU[c + im], r.du[2] = DU[c + km];
         r.pr[0] = PR[c], r.pr[1] = PR[c + im], r.pr[2] = PR[c + km];
         r.s1ip = MS1[c + ip];
         r.s2[0] = MS2[c], r.s2[1] = MS2[c + kp], r.s2[2] = MS2[c + ip];
@@ -675,12 +709,26 @@ __global__ void __launch_bounds__(512) k_io_terms_m(IoGeo g, const double* __res
     Row cur;
     load_row(j0 + 1, cur);
     const int cm = gc + L * j0;  // row JC-1 of the first step
-    double mujm = MU[cm], mu0jm = MU0[cm], dujm = DU[cm], prjm = PR[cm];
+    double mujm = MU[cm], mu0jm = MU0[cm], prjm = PR[cm];
     double s1c = MS1[cm + L], s3c = MS3[cm + L];
     const int nw = blockDim.x >> 6;
     __builtin_amdgcn_s_waitcnt(0xF70);  // nothing above in flight when the loop starts: s_waitcnt vmcnt(0)
     __syncthreads();
     int sM = 0, s0 = 1, sP = 2;
+    // DivU: the row's values (cells and the k0-1 halo row) in an LDS plane of
+    // their own, formed at the end of the step before from the ring and the
+    // arriving v row; the cell's own of this row and of row JC-1 carry over
+    double duc, dujm;
+    {
+        auto R = [&](int q) {
+            return CellRing{ring + q * PL + lc, ring + SL + q * PL + lc, ring + 2 * SL + q * PL + lc, ip, im, L};
+        };
+        dujm = io_divu(g, R(3), R(4), R(5), j0 + 1, 0, -1, 0);
+        duc = io_divu(g, R(3), R(4), R(5), j0 + 1, 0, 0, 0);
+        dup[lc] = duc;
+        dup[ldh] = rb == 0 ? io_divu(g, R(3), R(4), R(5), j0 + 1, 0, 0, -1) : duc;
+    }
+    __syncthreads();
     for (int j = j0; j < j1; ++j) {
         const int JC = j + 1;
         // the next step's row values, then the ring's next row JC+2 (both
@@ -702,7 +750,8 @@ __global__ void __launch_bounds__(512) k_io_terms_m(IoGeo g, const double* __res
                           ip, im, L};
         };
         const IoV4 vmu{cur.mu[0], cur.mu[1], mujm, cur.mu[2]}, vmu0{cur.mu0[0], cur.mu0[1], mu0jm, cur.mu0[2]};
-        const IoV4 vdu{cur.du[0], cur.du[1], dujm, cur.du[2]}, vpr{cur.pr[0], cur.pr[1], prjm, cur.pr[2]};
+        const IoV4 vdu{duc, dup[lc + im], dujm, dup[lc - L]};
+        const IoV4 vpr{cur.pr[0], cur.pr[1], prjm, cur.pr[2]};
         const IoVS1 vs1{s1c, cur.s1jp, cur.s1ip};
         const IoVS2 vs2{cur.s2[0], cur.s2[1], cur.s2[2]};
         const IoVS3 vs3{s3c, cur.s3jp, cur.s3kp};
@@ -714,6 +763,7 @@ __global__ void __launch_bounds__(512) k_io_terms_m(IoGeo g, const double* __res
         const double glv[3] = {JC == 1 ? R(0).m[0] : R(0).p[0], JC == 1 ? R(1).m[0] : R(1).p[0],
                                JC == 1 ? R(2).m[0] : R(2).p[0]};
         double v = io_terms_store(p, g, JC, e, NC, hv, rv, E, inc, G0, c, cg, CS, gv, glv);
+        io_divu_store(g, JC, c, duc, DU);
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
         if ((tid & 63) == 0) red[tid >> 6] = v;
@@ -730,7 +780,18 @@ __global__ void __launch_bounds__(512) k_io_terms_m(IoGeo g, const double* __res
             ring[sM * SL + q * PL + lc] = pn[q];
             ring[sM * SL + q * PL + lh] = ph[q];
         }
-        mujm = cur.mu[0], mu0jm = cur.mu0[0], dujm = cur.du[0], prjm = cur.pr[0];
+        // DivU of row JC+1: u and w of that row are in the ring, v of row JC+2
+        // has just arrived; rb == 0 forms the halo row's too
+        dujm = duc;
+        {
+            const double dy = ldc(g.dyfi, min(JC + 1, M) - 1);
+            const double *U1 = ring + sP * SL + 3 * PL, *V1 = U1 + PL, *W1 = V1 + PL;
+            duc = io_divu_v(g, dy, U1[lc + ip], U1[lc], pn[4], V1[lc], W1[lc + L], W1[lc]);
+            const double dh = io_divu_v(g, dy, U1[ldh + ip], U1[ldh], rb == 0 ? ph[4] : pn[4], V1[ldh], W1[ldh + L], W1[ldh]);
+            dup[lc] = duc;
+            dup[ldh] = dh;
+        }
+        mujm = cur.mu[0], mu0jm = cur.mu0[0], prjm = cur.pr[0];
         s1c = cur.s1jp, s3c = cur.s3jp;
         cur = nxt;
         __syncthreads();
@@ -1565,9 +1626,6 @@ int io_substep(chs_handle* h, const chs_thermal_fields* tf, const chs_io_fields*
     const bool fold = !prm->visimplicit && prm->nflow != 2;
     if (!fold) CHS_HIP(hipMemcpyAsync(f->g0, f->g, 3 * ngh * sizeof(double), hipMemcpyDeviceToDevice, s));
     if (prm->visimplicit) return io_substep_cn(h, f, a, p, ns, dt, talp);   // no DIVG_U_io in that branch
-    h->timer.begin("io_divu", s, &ev);
-    CHS_LAUNCH(k_io_divu, io_grid(h, h->M + 2), dim3(64, 4), 0, s, g, f->q, f->divu);
-    h->timer.end(ev, "io_divu", s);
     // the marching form needs L a power of two with 2L threads in whole
     // waves (at most 512) and its LDS ring on this device; chs_set_cn_solver
     // mode 2 selects the row-tile form
