@@ -509,7 +509,10 @@ int energy_substep(chs_handle* h, chs_props* p, const chs_thermal_fields* tf, in
                            tf->thermcondt + o, nullptr, p->ecnt, s));
     }
     h->timer.end(ev, "energy_props", s);
-    CHS_LAUNCH(k_energy_wall, dim3(64), dim3(256), props_lds_bytes(p), s, t, g, f, p->ecnt);
+    // a lookup chain per thread: one pass over the 2 L N wall cells with up to
+    // two blocks per CU (256x192x256: 64 blocks 30 us, 512 blocks 16)
+    const int nwall = (int)std::min(2L * p->ncu, (2L * h->L * h->N + 255) / 256);
+    CHS_LAUNCH(k_energy_wall, dim3(nwall), dim3(256), props_lds_bytes(p), s, t, g, f, p->ecnt);
     // the counts of lookups outside the table and of surrogate fallbacks to
     // pinned host memory, read by the next call on p (or chs_props_check,
     // chs_props_last_fallback) without a stream sync here
