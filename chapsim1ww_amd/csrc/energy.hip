@@ -104,10 +104,17 @@ __device__ __forceinline__ double energy_update(double rhoh, double rhs, double 
     return fmin(cap, r);
 }
 
+// The substep's counters (cnt[0..3]) cleared for the kernels that follow
+__device__ __forceinline__ void clear_counts(unsigned long long* cnt) {
+    const int t = threadIdx.x + blockDim.x * threadIdx.y;
+    if (blockIdx.x == 0 && t < 4) cnt[t] = 0ull;
+}
+
 // one thread per interior cell in row tiles (64 i x 4 k)
 __global__ void __launch_bounds__(256) k_energy_rhs(EGeo g, EFields f, double rk1, double rk0, double cthecd,
-                                                    double rhoh_cap) {
+                                                    double rhoh_cap, unsigned long long* __restrict__ cnt) {
 #pragma clang fp contract(off)
+    clear_counts(cnt);
     const int L = g.L, M = g.M, N = g.N;
     int it, jt, kt, tile;
     if (!row_tile(L, N, M, &it, &jt, &kt, &tile)) return;
@@ -144,8 +151,10 @@ constexpr int EKR = 4, EKP = EKR + 2;
 inline size_t energy_rhs_m_smem(int L) { return sizeof(double) * (size_t)3 * 3 * EKP * L; }
 
 __global__ void __launch_bounds__(1024) k_energy_rhs_m(EGeo g, EFields f, double rk1, double rk0, double cthecd,
-                                                       double rhoh_cap, int nyc, int jc, int lgL) {
+                                                       double rhoh_cap, int nyc, int jc, int lgL,
+                                                       unsigned long long* __restrict__ cnt) {
 #pragma clang fp contract(off)
+    clear_counts(cnt);
     extern __shared__ double sm[];
     const int L = g.L, M = g.M, N = g.N;
     const int PL = EKP * L, SL = 3 * PL;  // one array / one ring row (H, T, kappa)
@@ -236,39 +245,32 @@ __global__ void __launch_bounds__(1024) k_energy_rhs_m(EGeo g, EFields f, double
     }
 }
 
-constexpr int EPT = 512;   // threads per property block
-
-// cells per thread and pass of k_energy_props (heated substep at 256x192x256:
-// 1 cell 2330 us, 2 cells 2324 us, 4 cells 2310 us, 8 cells 2345 us)
-constexpr int ECELL = 4;
 
 // The lookups of k_energy_props without branches, so that the chains of a
 // thread's cells interleave: the query is clamped into the table (its result
 // is then discarded), ok says whether the value was inside; a NaN passes and
 // gives NaN (as the reference's evaluators do).
 // S_HT (hack: ENTHALPY_UPDATE's |h| < 1e-10 gives T = 1)
-template <int KW>
-__device__ __forceinline__ double ht_nb(const PropTab& t, const double* xh, const int* sh, double hv, bool hack,
-                                        bool& ok) {
+template <int KW, bool WIDE>
+__device__ __forceinline__ double ht_nb(const PropTab& t, const LdsTab<WIDE>& l, double hv, bool hack, bool& ok) {
     const bool nan = hv != hv, in = hv > t.h_lo && hv < t.h_hi;
     ok = nan || in;
     const double hq = in ? hv : t.h_lo;
-    const int i = find_iv<KW>(xh, sh, t.n, t.nbh, t.h_lo, t.hbi, hq);
-    const double4 r = reinterpret_cast<const double4*>(t.rh)[i];
-    double T = cubic_nc(r.x, r.y, r.z, r.w, hq - xh[i]);
+    const int i = find_iv<KW>(l.xh, l.sh, t.n, t.nbh, t.h_lo, t.hbi, hq);
+    const double4 r = l.ht(t, i);
+    double T = cubic_nc(r.x, r.y, r.z, r.w, hq - l.xh[i]);
     if (hack && fabs(hv) < 1.0e-10) T = 1.0;
     return nan ? hv : T;
 }
 
 // the interval of T (clamped) and its record's first double4 (S_TD) or all
 // four (S_TD, S_TM, S_TK, S_TCp)
-template <int KW>
-__device__ __forceinline__ int t_iv_nb(const PropTab& t, const double* xt, const int* st, double tv, bool& ok,
-                                       double& tq) {
+template <int KW, bool WIDE>
+__device__ __forceinline__ int t_iv_nb(const PropTab& t, const LdsTab<WIDE>& l, double tv, bool& ok, double& tq) {
     const bool nan = tv != tv, in = tv > t.t_lo && tv < t.t_hi;
     ok = nan || in;
     tq = in ? tv : t.t_lo;
-    return find_iv<KW>(xt, st, t.n, t.nbt, t.t_lo, t.tbi, tq);
+    return find_iv<KW>(l.xt, l.st, t.n, t.nbt, t.t_lo, t.tbi, tq);
 }
 
 // rotations of the property history on every cell, the property cascade on
@@ -279,14 +281,13 @@ __device__ __forceinline__ int t_iv_nb(const PropTab& t, const double* xt, const
 // one-cell form, so the outputs are unchanged bit for bit).
 // second = 0: the final THERM_PROP_UPDATE lookup is left to the learned
 // surrogate (chs_props_set_mode), which runs after this kernel on h
-template <int KW>
+template <int KW, bool WIDE, int EPT, int ECELL>
 __global__ void __launch_bounds__(EPT) k_energy_props(PropTab t, EGeo g, EFields f,
                                                       unsigned long long* __restrict__ cnt, int second) {
 #pragma clang fp contract(off)
     extern __shared__ unsigned char smem[];
-    const double *xh, *xt;
-    const int *sh, *st;
-    stage_tables(t, smem, xh, xt, sh, st);
+    const LdsTab<WIDE> l = stage_tab<WIDE>(t, smem);
+    const double* xt = l.xt;
     // 32-bit cell offsets (chs_create keeps 3*L*(M+2)*N below 2^31): the
     // row of a cell costs one 32-bit division instead of two 64-bit ones
     const int L = g.L, M = g.M;
@@ -322,16 +323,16 @@ __global__ void __launch_bounds__(EPT) k_energy_props(PropTab t, EGeo g, EFields
             double T1[ECELL];
             bool okh[ECELL];
 #pragma unroll
-            for (int u = 0; u < ECELL; ++u) T1[u] = ht_nb<KW>(t, xh, sh, rh[u] / rho_old[u], true, okh[u]);
+            for (int u = 0; u < ECELL; ++u) T1[u] = ht_nb<KW>(t, l, rh[u] / rho_old[u], true, okh[u]);
             int k1[ECELL];
             double tq[ECELL];
             double4 cd[ECELL];
 #pragma unroll
             for (int u = 0; u < ECELL; ++u) {
                 bool okt;
-                k1[u] = t_iv_nb<KW>(t, xt, st, T1[u], okt, tq[u]);
+                k1[u] = t_iv_nb<KW>(t, l, T1[u], okt, tq[u]);
                 ok1[u] = okh[u] && okt;
-                cd[u] = reinterpret_cast<const double4*>(t.rt)[4 * (size_t)k1[u]];
+                cd[u] = l.td(t, k1[u]);
             }
 #pragma unroll
             for (int u = 0; u < ECELL; ++u) {
@@ -349,8 +350,8 @@ __global__ void __launch_bounds__(EPT) k_energy_props(PropTab t, EGeo g, EFields
         for (int u = 0; u < ECELL; ++u) {
             h2[u] = rh[u] / D1[u];
             bool okh, okt;
-            T2[u] = ht_nb<KW>(t, xh, sh, h2[u], false, okh);
-            k2[u] = t_iv_nb<KW>(t, xt, st, T2[u], okt, tq2[u]);
+            T2[u] = ht_nb<KW>(t, l, h2[u], false, okh);
+            k2[u] = t_iv_nb<KW>(t, l, T2[u], okt, tq2[u]);
             ok2[u] = okh && okt;
         }
 #pragma unroll
@@ -374,7 +375,7 @@ __global__ void __launch_bounds__(EPT) k_energy_props(PropTab t, EGeo g, EFields
                 continue;
             }
             const double4* r4 = reinterpret_cast<const double4*>(t.rt) + 4 * (size_t)k2[u];
-            const double4 cd = r4[0], cm = r4[1], ck = r4[2];
+            const double4 cd = l.td(t, k2[u]), cm = r4[1], ck = r4[2];
             const double dt = tq2[u] - xt[k2[u]];
             double D = cubic_nc(cd.x, cd.y, cd.z, cd.w, dt);
             double Mu = cubic_nc(cm.x, cm.y, cm.z, cm.w, dt);
@@ -396,9 +397,7 @@ __global__ void __launch_bounds__(256) k_energy_wall(PropTab t, EGeo g, EFields 
                                                      unsigned long long* __restrict__ cnt) {
 #pragma clang fp contract(off)
     extern __shared__ unsigned char smem[];
-    const double *xh, *xt;
-    const int *sh, *st;
-    stage_tables(t, smem, xh, xt, sh, st);
+    const LdsTab<false> l = stage_tab<false>(t, smem);
     const int L = g.L, M = g.M;
     const long long LP = (long long)L * (M + 2);
     const long long nw = 2LL * L * g.N;
@@ -421,7 +420,7 @@ __global__ void __launch_bounds__(256) k_energy_wall(PropTab t, EGeo g, EFields 
         }
         f.h[q] = hv;
         double Tt, D, Mu, K, CP;
-        if (!spline_ht(t, xh, sh, hv, Tt, true) || !spline_t(t, xt, st, Tt, D, Mu, K, CP)) {
+        if (!spline_ht(t, l.xh, l.sh, hv, Tt, true) || !spline_t(t, l.xt, l.st, Tt, D, Mu, K, CP)) {
             ++bad;
             continue;
         }
@@ -433,10 +432,6 @@ __global__ void __launch_bounds__(256) k_energy_wall(PropTab t, EGeo g, EFields 
     }
     for (int o = 32; o > 0; o >>= 1) bad += __shfl_xor(bad, o);
     if ((threadIdx.x & 63) == 0 && bad) atomicAdd(cnt, bad);
-}
-
-__global__ void k_zero_u64_e(unsigned long long* c, int n) {
-    if ((int)threadIdx.x < n) c[threadIdx.x] = 0ull;
 }
 
 static const double TGAM_E[4] = {1.0, 8.0 / 15.0, 5.0 / 12.0, 3.0 / 4.0};
@@ -459,7 +454,6 @@ int energy_substep(chs_handle* h, chs_props* p, const chs_thermal_fields* tf, in
     const hipStream_t s = h->stream;
     const double cap = p->rhoh_max + 1.0e-14;   // RHOHmax + REALMIN
     hipEvent_t ev;
-    CHS_LAUNCH(k_zero_u64_e, dim3(1), dim3(64), 0, s, p->ecnt, 4);
     // the marching form needs L a power of two with 4L threads in whole
     // waves (at most 1024) and its LDS ring on this device; chs_set_cn_solver
     // mode 2 selects the row-tile form
@@ -477,21 +471,36 @@ int energy_substep(chs_handle* h, chs_props* p, const chs_thermal_fields* tf, in
         const int nyc = (h->M + jc - 1) / jc;
         (void)hipFuncSetAttribute((const void*)k_energy_rhs_m, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm);
         CHS_LAUNCH(k_energy_rhs_m, dim3(8 * ((nkg * nyc + 7) / 8)), dim3(EKR * L), sm, s, g, f, TGAM_E[ns] * dt,
-                   TROH_E[ns] * dt, cthecd, cap, nyc, jc, __builtin_ctz((unsigned)L));
+                   TROH_E[ns] * dt, cthecd, cap, nyc, jc, __builtin_ctz((unsigned)L), p->ecnt);
     } else {
         CHS_LAUNCH(k_energy_rhs, dim3(row_tile_blocks(h->L, h->N, h->M)), dim3(64, 4), 0, s, g, f, TGAM_E[ns] * dt,
-                   TROH_E[ns] * dt, cthecd, cap);
+                   TROH_E[ns] * dt, cthecd, cap, p->ecnt);
     }
     h->timer.end(ev, "energy_rhs", s);
     const PropTab t = tab_of(p);
     h->timer.begin("energy_props", s, &ev);
-    CHS_TRY(props_lds_attr((const void*)k_energy_wall, p));
+    CHS_TRY(props_lds_attr((const void*)k_energy_wall, props_lds_bytes(p)));
     const bool sur = p->mode == CHS_PROPS_SURROGATE;
+    // with the H -> T and T -> D records in LDS (LdsTab): two cells per thread
+    // of one block per CU; heated time steps at 256x192x256 6760 -> 6531 us (4
+    // cells: 6552), 128^3 1447 -> 1404 (1420), 64^3 317 -> 312 (332)
+    const bool wide = props_lds_wide(p) <= (size_t)p->lds_max;
+    const long ncells = (long)h->L * (h->M + 2) * h->N;
+#define CHS_EPROPS_L(KK, WIDE, EPT, ECELL)                                                                     \
+    do {                                                                                                       \
+        const auto kern = k_energy_props<KK, WIDE, EPT, ECELL>;                                                \
+        const size_t lds = WIDE ? props_lds_wide(p) : props_lds_bytes(p);                                      \
+        const long nblk = (ncells + EPT * ECELL - 1) / (EPT * ECELL);                                          \
+        CHS_TRY(props_lds_attr((const void*)kern, lds));                                                       \
+        CHS_LAUNCH(kern, dim3(props_grid_occ(p, (const void*)kern, EPT, lds, nblk)), dim3(EPT), lds, s, t, g, f, \
+                   p->ecnt, sur ? 0 : 1);                                                                      \
+    } while (0)
 #define CHS_EPROPS(KK)                                                                                         \
     do {                                                                                                       \
-        CHS_TRY(props_lds_attr((const void*)k_energy_props<KK>, p));                                           \
-        CHS_LAUNCH(k_energy_props<KK>, dim3(props_grid_occ(p, (const void*)k_energy_props<KK>, EPT, 1 << 20)),  \
-                   dim3(EPT), props_lds_bytes(p), s, t, g, f, p->ecnt, sur ? 0 : 1);                           \
+        if (wide)                                                                                              \
+            CHS_EPROPS_L(KK, true, 1024, 2);                                                                   \
+        else                                                                                                   \
+            CHS_EPROPS_L(KK, false, 512, 4);                                                                   \
     } while (0)
     switch (p->kwalk) {
         case 2: CHS_EPROPS(2); break;
@@ -500,6 +509,7 @@ int energy_substep(chs_handle* h, chs_props* p, const chs_thermal_fields* tf, in
         default: CHS_EPROPS(0); break;
     }
 #undef CHS_EPROPS
+#undef CHS_EPROPS_L
     if (sur) {
         // THERM_PROP_UPDATE of the interior rows by the surrogate where it is
         // certified (the table elsewhere), on this handle's stream

@@ -4,11 +4,12 @@
 // scaled property table (NIST_SPLINE_H/T, CUBIC_SPLINE,
 // src/Flow_State.f90:916-1014, 1693-1788).
 //
-// Layout: the knots of H and T (16 KB each at 2048 knots) and the bucket
-// starts of the two interval searches are staged in LDS once per persistent
-// block; the spline coefficients are read per cell as one record per interval
-// (32 B for H -> T, 128 B = one cache line for T -> D, M, K, CP), so a cell
-// costs its 8 B of h, its 40 B of outputs and two L2-resident records.
+// Layout: the knots of H and T (16 KB each at 2048 knots), the bucket starts
+// of the two interval searches and, for tables up to about 2100 knots, the
+// H -> T and T -> D coefficients are staged in LDS once per persistent block;
+// the other coefficients are read per cell from one record per interval (128 B
+// = one cache line for T -> D, M, K, CP), so a cell costs its 8 B of h, its
+// 40 B of outputs and an L2-resident record.
 // The reference's four separate bisections over the same T knots collapse
 // into one: they find the same interval.
 #include <algorithm>
@@ -66,31 +67,28 @@ static void bucket_starts(int n, const double* x, int nb, double lo, double bi, 
     }
 }
 
-__global__ void k_zero_u64(unsigned long long* c, int n) {
-    if ((int)threadIdx.x < n) c[threadIdx.x] = 0ull;
+// The two counts of a property update to pinned host memory, and zeros in
+// their place for the next call
+__global__ void k_counts_out(unsigned long long* c, unsigned long long* host) {
+    if (threadIdx.x < 2) {
+        host[threadIdx.x] = c[threadIdx.x];
+        c[threadIdx.x] = 0ull;
+    }
 }
 
-constexpr int PT = 1024;     // threads per lookup block
-constexpr int PCELL = 8;     // cells per thread and chunk (measured: 4 -> 8, 0.252 -> 0.240 ms)
-
-template <int KW>
+// PT threads, PCELL cells per thread and chunk of persistent blocks.  WIDE
+// (LdsTab): bound by the LDS reads of the searches and records and by the
+// gathers of the M, K and CP records; 12.6 M cells 290 -> 267 us a call.
+template <int KW, bool WIDE, int PT, int PCELL>
 __global__ void __launch_bounds__(PT) k_props_table(PropTab t, Rows rw, const double* __restrict__ h,
                                                     double* __restrict__ To, double* __restrict__ rho,
                                                     double* __restrict__ mu, double* __restrict__ kap,
                                                     double* __restrict__ cp, unsigned long long* __restrict__ cnt,
                                                     int count_lookups) {
     extern __shared__ unsigned char smem[];
-    double* xh = reinterpret_cast<double*>(smem);
-    double* xt = xh + t.n;
-    int* sh = reinterpret_cast<int*>(xt + t.n);
-    int* st = sh + t.nbh;
-    for (int e = threadIdx.x; e < t.n; e += blockDim.x) {
-        xh[e] = t.xh[e];
-        xt[e] = t.xt[e];
-    }
-    for (int e = threadIdx.x; e < t.nbh; e += blockDim.x) sh[e] = t.sh[e];
-    for (int e = threadIdx.x; e < t.nbt; e += blockDim.x) st[e] = t.st[e];
-    __syncthreads();
+    const LdsTab<WIDE> l = stage_tab<WIDE>(t, smem);
+    const double *xh = l.xh, *xt = l.xt;
+    constexpr int TC = PCELL < 2 ? 1 : 2;   // cells whose T records are in flight together
     const long long chunk = (long long)PT * PCELL;
     const long long cpr = (rw.rowlen + chunk - 1) / chunk;   // chunks per row
     const long long nch = cpr * rw.nrow;
@@ -108,8 +106,8 @@ __global__ void __launch_bounds__(PT) k_props_table(PropTab t, Rows rw, const do
             in[u] = c < rw.rowlen;
             hv[u] = in[u] ? h[base + c] : 0.0;
         }
-        // S_HT for every cell at once: the H intervals (LDS) and their
-        // coefficient records (L2), loaded together
+        // S_HT for every cell at once: the H intervals and their coefficient
+        // records, loaded together
         int ih[PCELL];
         double4 rr[PCELL];
 #pragma unroll
@@ -117,8 +115,8 @@ __global__ void __launch_bounds__(PT) k_props_table(PropTab t, Rows rw, const do
             // NaN and out-of-range values search at h_lo (a float-to-int
             // conversion of them would be undefined); their results are unused
             const double hq = hv[u] > t.h_lo && hv[u] < t.h_hi ? hv[u] : t.h_lo;
-            ih[u] = find_iv<KW>(xh, sh, t.n, t.nbh, t.h_lo, t.hbi, hq);
-            rr[u] = reinterpret_cast<const double4*>(t.rh)[ih[u]];
+            ih[u] = find_iv<KW>(xh, l.sh, t.n, t.nbh, t.h_lo, t.hbi, hq);
+            rr[u] = l.ht(t, ih[u]);
         }
         double tv[PCELL];
         bool okh[PCELL];
@@ -131,19 +129,21 @@ __global__ void __launch_bounds__(PT) k_props_table(PropTab t, Rows rw, const do
         // S_TD/TM/TK/TCp two cells at a time: both cells' T records are
         // loaded before either is evaluated
 #pragma unroll
-        for (int u0 = 0; u0 < PCELL; u0 += 2) {
-            int kt[2];
-            double4 rq[2][4];
+        for (int u0 = 0; u0 < PCELL; u0 += TC) {
+            int kt[TC];
+            double4 rq[TC][4];
 #pragma unroll
-            for (int v = 0; v < 2; ++v) {
+            for (int v = 0; v < TC; ++v) {
                 const double tq = tv[u0 + v] > t.t_lo && tv[u0 + v] < t.t_hi ? tv[u0 + v] : t.t_lo;
-                kt[v] = find_iv<KW>(xt, st, t.n, t.nbt, t.t_lo, t.tbi, tq);
+                kt[v] = find_iv<KW>(xt, l.st, t.n, t.nbt, t.t_lo, t.tbi, tq);
                 const double4* q = reinterpret_cast<const double4*>(t.rt) + 4 * (size_t)kt[v];
-#pragma unroll
-                for (int m = 0; m < 4; ++m) rq[v][m] = q[m];
+                rq[v][0] = l.td(t, kt[v]);
+                rq[v][1] = q[1];
+                rq[v][2] = q[2];
+                rq[v][3] = cp ? q[3] : q[2];
             }
 #pragma unroll
-            for (int v = 0; v < 2; ++v) {
+            for (int v = 0; v < TC; ++v) {
                 const int u = u0 + v;
                 // THERM_PROP_UPDATE leaves |h| < 1e-10 (and cells past the row) as they are
                 if (!in[u] || fabs(hv[u]) < 1.0e-10) continue;
@@ -185,17 +185,35 @@ __global__ void __launch_bounds__(PT) k_props_table(PropTab t, Rows rw, const do
     }
 }
 
+// Calls of fewer cells than a chunk of 8 per thread of 1024 would spread over
+// the CUs run one cell per thread: 4,096 cells 53 -> 33 us a call, 262,144
+// 65 -> 39, 1,048,576 69 -> 59; 2,097,152 70 against 78 (with the same host path)
+constexpr long long PSMALL = 3ll << 19;
+
 int props_table_launch(chs_props* p, const double* h, Rows rw, double* T, double* rho, double* mu, double* kap,
                        double* cp, unsigned long long* cnt, int count_lookups, hipStream_t stream) {
-    const long long chunk = (long long)PT * PCELL;
-    const long long nch = ((rw.rowlen + chunk - 1) / chunk) * rw.nrow;
-    if (nch == 0) return CHS_OK;
+    const long long cells = rw.rowlen * rw.nrow;
+    if (cells == 0) return CHS_OK;
+    const bool wide = props_lds_wide(p) <= (size_t)p->lds_max;
+#define CHS_PROPS_L(KK, WIDE, PT, PCELL)                                                                         \
+    do {                                                                                                         \
+        const auto kern = k_props_table<KK, WIDE, PT, PCELL>;                                                    \
+        const size_t lds = WIDE ? props_lds_wide(p) : props_lds_bytes(p);                                        \
+        const long long chunk = (long long)PT * PCELL;                                                           \
+        const long long nch = ((rw.rowlen + chunk - 1) / chunk) * rw.nrow;                                       \
+        CHS_TRY(props_lds_attr((const void*)kern, lds));                                                         \
+        const int grid = props_grid_occ(p, (const void*)kern, PT, lds, nch);                                     \
+        CHS_LAUNCH(kern, dim3(grid), dim3(PT), lds, stream, tab_of(p), rw, h, T, rho, mu, kap, cp, cnt,          \
+                   count_lookups);                                                                               \
+    } while (0)
 #define CHS_PROPS_K(KK)                                                                                          \
     do {                                                                                                         \
-        CHS_TRY(props_lds_attr((const void*)k_props_table<KK>, p));                                              \
-        const int grid = props_grid_occ(p, (const void*)k_props_table<KK>, PT, nch);                             \
-        CHS_LAUNCH(k_props_table<KK>, dim3(grid), dim3(PT), props_lds_bytes(p), stream, tab_of(p), rw, h, T, rho, \
-                   mu, kap, cp, cnt, count_lookups);                                                             \
+        if (cells < PSMALL)                                                                                      \
+            CHS_PROPS_L(KK, false, 256, 1);                                                                      \
+        else if (wide)                                                                                           \
+            CHS_PROPS_L(KK, true, 1024, 8);                                                                      \
+        else                                                                                                     \
+            CHS_PROPS_L(KK, false, 1024, 8);                                                                     \
     } while (0)
     switch (p->kwalk) {
         case 2: CHS_PROPS_K(2); break;
@@ -204,6 +222,7 @@ int props_table_launch(chs_props* p, const double* h, Rows rw, double* T, double
         default: CHS_PROPS_K(0); break;
     }
 #undef CHS_PROPS_K
+#undef CHS_PROPS_L
     return CHS_OK;
 }
 
@@ -335,18 +354,22 @@ int props_create(int n, const double* H, const double* T, const double* D, const
     p->xt = p->xh + n;
     p->sh = reinterpret_cast<int*>(p->xt + n);
     p->st = p->sh + p->nbh;
-    if (hipMalloc((void**)&p->counters, 8 * sizeof(unsigned long long)) != hipSuccess ||
-        hipHostMalloc((void**)&p->ecnt_host, 2 * sizeof(unsigned long long), hipHostMallocDefault) != hipSuccess) {
+    if (hipMalloc((void**)&p->counters, 12 * sizeof(unsigned long long)) != hipSuccess ||
+        hipHostMalloc((void**)&p->ecnt_host, 4 * sizeof(unsigned long long),
+                      hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
         set_error("chs_props_create: allocation of the counters failed");
         return fail(CHS_E_NOMEM);
     }
     p->ecnt = p->counters + 4;
-    p->ecnt_host[0] = p->ecnt_host[1] = 0;
+    p->ucnt = p->counters + 8;
+    for (int q = 0; q < 4; ++q) p->ecnt_host[q] = 0;
     if (hipEventCreateWithFlags(&p->ecnt_ev, hipEventDisableTiming) != hipSuccess) {
         set_error("chs_props_create: event creation failed");
         return fail(CHS_E_HIP);
     }
-    if (hipMemcpy(p->rh, p->hrh.data(), p->hrh.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess ||
+    const unsigned long long zeros[12] = {};
+    if (hipMemcpy(p->counters, zeros, sizeof(zeros), hipMemcpyHostToDevice) != hipSuccess ||
+        hipMemcpy(p->rh, p->hrh.data(), p->hrh.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(p->rt, p->hrt.data(), p->hrt.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(p->xh, H, n * sizeof(double), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(p->xt, T, n * sizeof(double), hipMemcpyHostToDevice) != hipSuccess ||
@@ -415,13 +438,12 @@ int props_update(chs_props* p, int mode, const double* h, long long nrow, long l
     if (nrow == 0 || rowlen == 0) return CHS_OK;
     CHS_CHECK(h && T && rho && mu && kap, CHS_E_ARG, "chs_therm_prop_update: NULL array");
     Rows rw{nrow, rowlen, nrow > 1 ? stride : rowlen};
-    CHS_LAUNCH(k_zero_u64, dim3(1), dim3(64), 0, p->stream, p->counters, 4);
     if (mode == CHS_PROPS_TABLE)
-        CHS_TRY(props_table_launch(p, h, rw, T, rho, mu, kap, cp, p->counters, 0, p->stream));
+        CHS_TRY(props_table_launch(p, h, rw, T, rho, mu, kap, cp, p->ucnt, 0, p->stream));
     else
-        CHS_TRY(mlp_update(p, h, rw, T, rho, mu, kap, cp, p->counters, p->stream));
-    unsigned long long host[2] = {0, 0};
-    CHS_HIP(hipMemcpyAsync(host, p->counters, 2 * sizeof(unsigned long long), hipMemcpyDeviceToHost, p->stream));
+        CHS_TRY(mlp_update(p, h, rw, T, rho, mu, kap, cp, p->ucnt, p->stream));
+    unsigned long long* host = p->ecnt_host + 2;
+    CHS_LAUNCH(k_counts_out, dim3(1), dim3(64), 0, p->stream, p->ucnt, host);
     CHS_HIP(hipStreamSynchronize(p->stream));
     if (n_fallback) *n_fallback = (long long)host[1];
     if (host[0]) {

@@ -2,6 +2,8 @@
 // the learned surrogate (mlp.hip).
 #pragma once
 
+#include <type_traits>
+
 #include "chs_common.hpp"
 
 namespace chs {
@@ -27,7 +29,8 @@ struct chs_props {
     int* st = nullptr;         // T bucket -> first candidate interval [nbt]
     double* rh = nullptr;      // [n][4]: T, b, c, d of the H -> T spline
     double* rt = nullptr;      // [n][16]: (y, b, c, d) of T -> D, M, K, CP
-    unsigned long long* counters = nullptr;   // [4] device counters
+    unsigned long long* counters = nullptr;   // device counters: [4] training and certification, [4] ecnt, [4] ucnt
+    unsigned long long* ucnt = nullptr;       // those of chs_therm_prop_update, zero between calls
     // host copies used by the surrogate's certification
     std::vector<double> hH, hT, hrh, hrt;
     // learned surrogate (mlp.hip)
@@ -37,8 +40,8 @@ struct chs_props {
     int mode = 0;
     long long last_fallback = 0;
     // the energy substep's range check, read without a stream sync: its
-    // device counters (after the four of the other calls), their pinned host
-    // copy, the event that follows the copy, and a resolved count not yet
+    // device counters, their pinned host
+    // copy (ecnt_host[0..1]; [2..3]: that of ucnt), the event that follows the copy, and a resolved count not yet
     // reported
     unsigned long long* ecnt = nullptr;
     unsigned long long* ecnt_host = nullptr;
@@ -65,14 +68,17 @@ int energy_range_check(chs_props* p, const char* who);
 inline size_t props_lds_bytes(const chs_props* p) {
     return sizeof(double) * 2 * (size_t)p->n + sizeof(int) * ((size_t)p->nbh + p->nbt);
 }
+// and with the H -> T and T -> D coefficient records staged too (LdsTab<true>)
+inline size_t props_lds_wide(const chs_props* p) {
+    return sizeof(double) * 9 * (size_t)p->n + sizeof(unsigned short) * ((size_t)p->nbh + p->nbt);
+}
 
 // Blocks of a persistent lookup kernel of `threads` threads with the staged
 // tables in LDS: as many as are resident at once on the device (registers and
 // LDS), at most `want`.
-inline int props_grid_occ(const chs_props* p, const void* kernel, int threads, long long want) {
+inline int props_grid_occ(const chs_props* p, const void* kernel, int threads, size_t lds, long long want) {
     int per = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, threads, props_lds_bytes(p)) != hipSuccess ||
-        per < 1)
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, threads, lds) != hipSuccess || per < 1)
         per = 1;
     const long long g = (long long)p->ncu * per;
     return (int)(want < g ? want : g);
@@ -80,8 +86,7 @@ inline int props_grid_occ(const chs_props* p, const void* kernel, int threads, l
 
 // Allow a lookup kernel the staged tables' LDS when they exceed the default
 // 64 KB per block (props_create has checked them against the device limit).
-inline int props_lds_attr(const void* kernel, const chs_props* p) {
-    const size_t b = props_lds_bytes(p);
+inline int props_lds_attr(const void* kernel, size_t b) {
     if (b > 65536) {
         hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)b);
         if (e != hipSuccess) {
@@ -96,7 +101,8 @@ inline int props_lds_attr(const void* kernel, const chs_props* p) {
 // result of the reference's bisection (NIST_SLEVAL_*, src/Flow_State.f90:
 // 1050-1061).  A bucket gives the first candidate; short walks make it exact
 // whatever the rounding of the bucket index.
-__device__ __forceinline__ int find_interval(const double* x, const int* start, int n, int nb, double lo,
+template <class Ix>
+__device__ __forceinline__ int find_interval(const double* x, const Ix* start, int n, int nb, double lo,
                                              double bi, double u) {
     int b = (int)((u - lo) * bi);
     b = b < 0 ? 0 : (b >= nb ? nb - 1 : b);
@@ -110,8 +116,8 @@ __device__ __forceinline__ int find_interval(const double* x, const int* start, 
 // back (the rounding of the bucket index) and K forward, K being one more
 // than the most knots any bucket holds (props_create checks it), so that the
 // searches of several cells interleave.
-template <int K>
-__device__ __forceinline__ int find_interval_k(const double* x, const int* start, int n, int nb, double lo,
+template <int K, class Ix>
+__device__ __forceinline__ int find_interval_k(const double* x, const Ix* start, int n, int nb, double lo,
                                                double bi, double u) {
     int b = (int)((u - lo) * bi);
     b = b < 0 ? 0 : (b >= nb ? nb - 1 : b);
@@ -122,8 +128,8 @@ __device__ __forceinline__ int find_interval_k(const double* x, const int* start
     return i;
 }
 
-template <int K>
-__device__ __forceinline__ int find_iv(const double* x, const int* start, int n, int nb, double lo, double bi,
+template <int K, class Ix>
+__device__ __forceinline__ int find_iv(const double* x, const Ix* start, int n, int nb, double lo, double bi,
                                        double u) {
     if constexpr (K > 0)
         return find_interval_k<K>(x, start, n, nb, lo, bi, u);
@@ -164,6 +170,66 @@ inline PropTab tab_of(const chs_props* p) {
     t.sh = p->sh;
     t.st = p->st;
     return t;
+}
+
+// The table as a lookup block holds it in LDS: the knots and bucket starts of
+// both searches and, WIDE, the coefficient records of H -> T (its values are
+// the T knots) and T -> D.  A record read from L2 is two 16-byte gathers whose
+// 64 lanes touch 64 cache lines, one line a cycle: ten of them a cell (H -> T,
+// D, M, K, CP) took 271 us of texture addressing at 12.6 M cells.  LDS serves
+// 64 scattered doubles in some ten cycles, and 2048 knots leave room for two of
+// the five records (156 KB, one block of 1024 threads per CU).
+template <bool WIDE>
+struct LdsTab {
+    using Ix = std::conditional_t<WIDE, unsigned short, int>;
+    const double *xh, *xt;       // knots
+    const double *hb, *ty, *tb;  // WIDE: b, c, d of H -> T; values and b, c, d of T -> D
+    const Ix *sh, *st;
+    // record i of H -> T, record k of T -> D: (y, b, c, d)
+    __device__ __forceinline__ double4 ht(const PropTab& t, int i) const {
+        if constexpr (WIDE)
+            return make_double4(xt[i], hb[3 * i], hb[3 * i + 1], hb[3 * i + 2]);
+        else
+            return reinterpret_cast<const double4*>(t.rh)[i];
+    }
+    __device__ __forceinline__ double4 td(const PropTab& t, int k) const {
+        if constexpr (WIDE)
+            return make_double4(ty[k], tb[3 * k], tb[3 * k + 1], tb[3 * k + 2]);
+        else
+            return reinterpret_cast<const double4*>(t.rt)[4 * (size_t)k];
+    }
+};
+
+// Stage the table (all threads of the block; ends with a barrier):
+// props_lds_wide() or props_lds_bytes() bytes.
+template <bool WIDE>
+__device__ __forceinline__ LdsTab<WIDE> stage_tab(const PropTab& t, unsigned char* smem) {
+    using Ix = typename LdsTab<WIDE>::Ix;
+    double* a = reinterpret_cast<double*>(smem);
+    double *b = a + t.n, *e = b + t.n;
+    double *hb = nullptr, *ty = nullptr, *tb = nullptr;
+    if constexpr (WIDE) {
+        hb = e;
+        ty = hb + 3 * t.n;
+        tb = ty + t.n;
+        e = tb + 3 * t.n;
+    }
+    Ix *c = reinterpret_cast<Ix*>(e), *d = c + t.nbh;
+    for (int q = threadIdx.x; q < t.n; q += blockDim.x) {
+        a[q] = t.xh[q];
+        b[q] = t.xt[q];
+        if constexpr (WIDE) {
+            const double4 r = reinterpret_cast<const double4*>(t.rh)[q];
+            const double4 s = reinterpret_cast<const double4*>(t.rt)[4 * (size_t)q];
+            hb[3 * q] = r.y, hb[3 * q + 1] = r.z, hb[3 * q + 2] = r.w;
+            ty[q] = s.x;
+            tb[3 * q] = s.y, tb[3 * q + 1] = s.z, tb[3 * q + 2] = s.w;
+        }
+    }
+    for (int q = threadIdx.x; q < t.nbh; q += blockDim.x) c[q] = (Ix)t.sh[q];
+    for (int q = threadIdx.x; q < t.nbt; q += blockDim.x) d[q] = (Ix)t.st[q];
+    __syncthreads();
+    return LdsTab<WIDE>{a, b, hb, ty, tb, c, d};
 }
 
 // S_HT (NIST_SLEVAL_HT, src/Flow_State.f90:1015-1070): false when h leaves
@@ -236,27 +302,6 @@ __device__ __forceinline__ bool lookup_cell(const PropTab& t, const double* xh, 
     if (!spline_t<KW>(t, xt, st, tv, D, Mu, K, CP)) return false;
     T = tv;
     return true;
-}
-
-// Stage the search tables of t in LDS (all threads of the block; ends with a
-// barrier).  Layout: xh[n] xt[n] sh[nbh] st[nbt], props_lds_bytes() bytes.
-__device__ __forceinline__ void stage_tables(const PropTab& t, unsigned char* smem, const double*& xh,
-                                             const double*& xt, const int*& sh, const int*& st) {
-    double* a = reinterpret_cast<double*>(smem);
-    double* b = a + t.n;
-    int* c = reinterpret_cast<int*>(b + t.n);
-    int* d = c + t.nbh;
-    for (int e = threadIdx.x; e < t.n; e += blockDim.x) {
-        a[e] = t.xh[e];
-        b[e] = t.xt[e];
-    }
-    for (int e = threadIdx.x; e < t.nbh; e += blockDim.x) c[e] = t.sh[e];
-    for (int e = threadIdx.x; e < t.nbt; e += blockDim.x) d[e] = t.st[e];
-    __syncthreads();
-    xh = a;
-    xt = b;
-    sh = c;
-    st = d;
 }
 
 }  // namespace chs
