@@ -176,19 +176,48 @@ inline unsigned row_tile_blocks(int L, int N, int nj) {
 }
 
 // Rows per y chunk of a kernel that marches along y with an LDS ring, one
-// block per group of k rows (nkg groups) and chunk of rows: about one block
-// per CU (256 on MI355X), or, with fill, one for each block that the ring's
-// LDS (smem bytes of lds_max) lets a CU hold, at most four; chunks of at
-// least 4 rows, none empty.
+// block per group of k rows (nkg groups) and chunk of rows.  A CU holds one
+// block, or, with fill, as many as the ring's LDS lets it (smem bytes of
+// lds_max), at most four; each XCD's 32 CUs take an eighth of the blocks in
+// rounds.  The chunks (of at least 4 rows, none empty) are those with the
+// fewest row steps, rounds x (rows of a chunk + 3 to fill the ring): a round
+// that is nearly empty costs as much as a full one (a tg time step at
+// 200x150x200: 6 chunks, 300 blocks 2089 us, 5 chunks, 250 blocks 1851 us).
 // A march shorter than MARCH_MIN rows (small grids) loses to the row-tile
 // kernels, which need no ring fill: measured at 64^3, FP64 substep 74.9 ->
 // 71.1 us, heated substep 122.1 -> 111.3 us (4-row chunks); at 128^3 (8 and
 // 16 rows) the marching kernels win (244 against 251 us, 492 against 533 us).
+// Threads past the block's last cell (n cells, whole waves) repeat that cell:
+// same loads, same stores of the same values; live says whose sums count.
+struct MarchLane {
+    int tid;
+    bool live;
+};
+__device__ __forceinline__ MarchLane march_lane(int n) {
+    const int t = threadIdx.x;
+    return MarchLane{t < n ? t : n - 1, t < n};
+}
+inline unsigned march_threads(int n) { return (unsigned)((n + 63) & ~63); }
+// tid / L and tid % L of a block's thread (L need not be a power of two)
+__device__ __forceinline__ void march_split(int tid, int L, int& r, int& i) {
+    r = (int)(((float)tid + 0.5f) / (float)L);
+    i = tid - r * L;
+}
 constexpr int MARCH_MIN = 8;
 inline int march_chunk_rows(int rows, int nkg, size_t smem, int lds_max, bool fill) {
     const int bpc = fill ? std::max(1, std::min(4, (int)((size_t)lds_max / std::max<size_t>(smem, 1)))) : 1;
-    const int nyc = std::max(1, std::min(rows / 4, (256 * bpc + nkg - 1) / nkg));
-    return (rows + nyc - 1) / nyc;
+    int best = rows;
+    long cost = -1;
+    for (int nyc = 1; nyc <= std::max(1, rows / 4); ++nyc) {
+        const int jc = (rows + nyc - 1) / nyc;
+        const long per = ((long)nkg * ((rows + jc - 1) / jc) + 7) / 8;   // blocks of an XCD
+        const long c = (per + 32 * bpc - 1) / (32 * bpc) * (jc + 3);
+        if (cost < 0 || c < cost) {
+            cost = c;
+            best = jc;
+        }
+    }
+    return best;
 }
 
 // xz-plane sums in two stages of a fixed order: one block of 256 threads per

@@ -140,22 +140,22 @@ __global__ void __launch_bounds__(256) k_energy_rhs(EGeo g, EFields f, double rk
 
 // ---------------------------------------------------------------------------
 // k_energy_rhs_m: k_energy_rhs marching along y, as k_rhs_xm: a block owns
-// EKR = 4 consecutive k rows of every x line and a chunk of rows, one cell
-// of each row per thread (4L threads).  LDS holds a ring of the rows JC-1,
+// EKR consecutive k rows (4, or 2 for lines beyond 256) of every x line and a
+// chunk of rows, one cell of each row per thread (EKR L threads).  LDS holds a ring of the rows JC-1,
 // JC, JC+1 of H, T and kappa (EKR + 2 k rows each); the mass fluxes, RHOH
 // and RHS0 of a row are loaded one step ahead in registers, G0 and G of v at
 // the cell carried from the step before.
 // ---------------------------------------------------------------------------
-constexpr int EKR = 4, EKP = EKR + 2;
+inline size_t energy_rhs_m_smem(int L, int EKR) { return sizeof(double) * (size_t)3 * 3 * (EKR + 2) * L; }
 
-inline size_t energy_rhs_m_smem(int L) { return sizeof(double) * (size_t)3 * 3 * EKP * L; }
-
+template <int EKR>
 __global__ void __launch_bounds__(1024) k_energy_rhs_m(EGeo g, EFields f, double rk1, double rk0, double cthecd,
-                                                       double rhoh_cap, int nyc, int jc, int lgL,
+                                                       double rhoh_cap, int nyc, int jc,
                                                        unsigned long long* __restrict__ cnt) {
 #pragma clang fp contract(off)
     clear_counts(cnt);
     extern __shared__ double sm[];
+    constexpr int EKP = EKR + 2;
     const int L = g.L, M = g.M, N = g.N;
     const int PL = EKP * L, SL = 3 * PL;  // one array / one ring row (H, T, kappa)
     double* ring = sm;
@@ -165,7 +165,8 @@ __global__ void __launch_bounds__(1024) k_energy_rhs_m(EGeo g, EFields f, double
     const int kg = t / nyc;
     const int j0 = (t - kg * nyc) * jc, j1 = min(M, j0 + jc);
     const int k0 = kg * EKR;
-    const int tid = threadIdx.x, r = tid >> lgL, IC = tid & (L - 1);
+    int r, IC;
+    march_split(march_lane(EKR * L).tid, L, r, IC);
     const int KC = k0 + r;
     const int LP = L * (M + 2), CS = LP * N;
     // one halo value per thread: the k0-1 row (r == 0), the k0+EKR row
@@ -454,24 +455,23 @@ int energy_substep(chs_handle* h, chs_props* p, const chs_thermal_fields* tf, in
     const hipStream_t s = h->stream;
     const double cap = p->rhoh_max + 1.0e-14;   // RHOHmax + REALMIN
     hipEvent_t ev;
-    // the marching form needs L a power of two with 4L threads in whole
-    // waves (at most 1024) and its LDS ring on this device; chs_set_cn_solver
-    // mode 2 selects the row-tile form
-    const int L = h->L;
-    const bool march = h->cn_mode != 2 && (L & (L - 1)) == 0 && L >= 16 && EKR * L <= 1024 && h->N % EKR == 0 &&
-                       energy_rhs_m_smem(L) <= (size_t)h->lds_max &&
-                       (h->cn_mode == 3 ||
-                        march_chunk_rows(h->M, h->N / EKR, energy_rhs_m_smem(L), h->lds_max, false) >= MARCH_MIN);
+    // the marching form: EKR k rows of whole x lines, one cell per thread (at
+    // most 1024) and the LDS ring on this device; chs_set_cn_solver mode 2
+    // selects the row-tile form
+    const int L = h->L, ekr = L <= 256 ? 4 : 2;
+    const size_t smr = energy_rhs_m_smem(L, ekr);
+    const bool march = h->cn_mode != 2 && L >= 16 && ekr * L <= 1024 && h->N % ekr == 0 && smr <= (size_t)h->lds_max &&
+                       (h->cn_mode == 3 || march_chunk_rows(h->M, h->N / ekr, smr, h->lds_max, false) >= MARCH_MIN);
     h->timer.begin("energy_rhs", s, &ev);
     if (march) {
-        const int nkg = h->N / EKR;
-        const size_t sm = energy_rhs_m_smem(L);
+        const int nkg = h->N / ekr;
         // one block per CU: filling the LDS (two per CU at 128^3) measured no faster
-        const int jc = march_chunk_rows(h->M, nkg, sm, h->lds_max, false);
+        const int jc = march_chunk_rows(h->M, nkg, smr, h->lds_max, false);
         const int nyc = (h->M + jc - 1) / jc;
-        (void)hipFuncSetAttribute((const void*)k_energy_rhs_m, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm);
-        CHS_LAUNCH(k_energy_rhs_m, dim3(8 * ((nkg * nyc + 7) / 8)), dim3(EKR * L), sm, s, g, f, TGAM_E[ns] * dt,
-                   TROH_E[ns] * dt, cthecd, cap, nyc, jc, __builtin_ctz((unsigned)L), p->ecnt);
+        const auto kern = ekr == 4 ? k_energy_rhs_m<4> : k_energy_rhs_m<2>;
+        (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smr);
+        CHS_LAUNCH(kern, dim3(8 * ((nkg * nyc + 7) / 8)), dim3(march_threads(ekr * L)), smr, s, g, f, TGAM_E[ns] * dt,
+                   TROH_E[ns] * dt, cthecd, cap, nyc, jc, p->ecnt);
     } else {
         CHS_LAUNCH(k_energy_rhs, dim3(row_tile_blocks(h->L, h->N, h->M)), dim3(64, 4), 0, s, g, f, TGAM_E[ns] * dt,
                    TROH_E[ns] * dt, cthecd, cap, p->ecnt);

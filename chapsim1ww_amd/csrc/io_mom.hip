@@ -645,7 +645,7 @@ __global__ void __launch_bounds__(512) k_io_terms_m(IoGeo g, const double* __res
                                                     const double* __restrict__ RS, double* __restrict__ E,
                                                     IoParams p, double tg, double tr, double dt, double adt,
                                                     double* __restrict__ inc, double* __restrict__ part,
-                                                    double* __restrict__ G0, int nyc, int jc, int lgL) {
+                                                    double* __restrict__ G0, int nyc, int jc) {
 #pragma clang fp contract(off)
     extern __shared__ double sm[];
     const int L = g.L, M = g.M, N = g.N;
@@ -659,7 +659,10 @@ __global__ void __launch_bounds__(512) k_io_terms_m(IoGeo g, const double* __res
     const int kg = t / nyc;
     const int j0 = (t - kg * nyc) * jc, j1 = min(M, j0 + jc);
     const int k0 = kg * IOKR;
-    const int tid = threadIdx.x, rb = tid >> lgL, i = tid & (L - 1);
+    const int tid = threadIdx.x;
+    const MarchLane ml = march_lane(IOKR * L);
+    int rb, i;
+    march_split(ml.tid, L, rb, i);
     const int KC = k0 + rb;
     const int LP = L * (M + 2), CS = LP * N, NC = L * M * N;
     // the cell's halo row: k0-1 (rb == 0) or k0+IOKR (rb == 1)
@@ -764,6 +767,7 @@ __global__ void __launch_bounds__(512) k_io_terms_m(IoGeo g, const double* __res
                                JC == 1 ? R(2).m[0] : R(2).p[0]};
         double v = io_terms_store(p, g, JC, e, NC, hv, rv, E, inc, G0, c, cg, CS, gv, glv);
         io_divu_store(g, JC, c, duc, DU);
+        v = ml.live ? v : 0.0;
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
         if ((tid & 63) == 0) red[tid >> 6] = v;
@@ -1626,11 +1630,11 @@ int io_substep(chs_handle* h, const chs_thermal_fields* tf, const chs_io_fields*
     const bool fold = !prm->visimplicit && prm->nflow != 2;
     if (!fold) CHS_HIP(hipMemcpyAsync(f->g0, f->g, 3 * ngh * sizeof(double), hipMemcpyDeviceToDevice, s));
     if (prm->visimplicit) return io_substep_cn(h, f, a, p, ns, dt, talp);   // no DIVG_U_io in that branch
-    // the marching form needs L a power of two with 2L threads in whole
-    // waves (at most 512) and its LDS ring on this device; chs_set_cn_solver
-    // mode 2 selects the row-tile form
+    // the marching form: IOKR k rows of whole x lines, one cell per thread (at
+    // most 512) and the LDS ring on this device; chs_set_cn_solver mode 2
+    // selects the row-tile form
     const int L = h->L;
-    const bool march = h->cn_mode != 2 && (L & (L - 1)) == 0 && L >= 32 && 2 * L <= 512 && h->N % IOKR == 0 &&
+    const bool march = h->cn_mode != 2 && L >= 32 && IOKR * L <= 512 && h->N % IOKR == 0 &&
                        io_terms_m_smem(L) <= (size_t)h->lds_max && (long)(h->N / IOKR) * h->M <= 2L * h->npart &&
                        (h->cn_mode == 3 ||
                         march_chunk_rows(h->M, h->N / IOKR, io_terms_m_smem(L), h->lds_max, true) >= MARCH_MIN);
@@ -1645,14 +1649,13 @@ int io_substep(chs_handle* h, const chs_thermal_fields* tf, const chs_io_fields*
         const int nyc = (h->M + jc - 1) / jc;
         nbt = (long)nkg * h->M;
         const dim3 gm(8 * ((nkg * nyc + 7) / 8));
-        const int lgL = __builtin_ctz((unsigned)L);
 #define IO_TERMS_M(GR)                                                                                             \
     do {                                                                                                           \
         (void)hipFuncSetAttribute((const void*)k_io_terms_m<GR>, hipFuncAttributeMaxDynamicSharedMemorySize,     \
                                   (int)sm);                                                                        \
-        CHS_LAUNCH(k_io_terms_m<GR>, gm, dim3(2 * L), sm, s, g, a.g, a.q, a.mu, a.mu0, a.divu, a.ms, a.pr, a.rs,     \
+        CHS_LAUNCH(k_io_terms_m<GR>, gm, dim3(march_threads(IOKR * L)), sm, s, g, a.g, a.q, a.mu, a.mu0, a.divu, a.ms, a.pr, a.rs,     \
                    a.explt0, p, TGAM_IO[ns], TROH_IO[ns], dt, talp * dt, h->rhs, h->partials,                      \
-                   fold ? f->g0 : nullptr, nyc, jc, lgL);                                                          \
+                   fold ? f->g0 : nullptr, nyc, jc);                                                          \
     } while (0)
         switch (prm->gravdir) {
             case 1: IO_TERMS_M(1); break;

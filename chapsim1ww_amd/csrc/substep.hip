@@ -489,8 +489,9 @@ __global__ void __launch_bounds__(CPT == 1 ? 1024 : 512) k_rhs_xm(Geo g, RkCoef 
     const int j0 = (t - kg * nyc) * jc, j1 = min(M, j0 + jc);
     const int k0 = kg * KR;
     const int tid = threadIdx.x;
+    const MarchLane ml = march_lane(RB * L);
     int rb, i;
-    divmod_row(tid, L, lgL, 1.0f / (float)L, rb, i);
+    march_split(ml.tid, L, rb, i);
     const int LP = L * (M + 2), CS = LP * N, LMN = L * M * N;
     // The thread's cells (k rows rb + u*RB) and one halo row: k0-1 (rb == 0),
     // k0+KR (rb == RB-1), or, for the rows between, its first cell once more
@@ -616,6 +617,7 @@ __global__ void __launch_bounds__(CPT == 1 ? 1024 : 512) k_rhs_xm(Geo g, RkCoef 
             }
             v += double(g.mc == 0 ? rhs[0] : rhs[2]) / dyfj / 1.0;
         }
+        v = ml.live ? v : 0.0;
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
         if ((tid & 63) == 0) red[tid >> 6] = v;
@@ -1695,9 +1697,10 @@ int rk3_substep(chs_handle* h, int ns, double dt) {
     CnStencils* cn = nullptr;
     CHS_TRY(cn_stencils_locked(h, facoe, &cn));
     const bool use_st = stencil_path(h, *cn);
-    // the mixed form's FP32 stencils run where NCL3 is a multiple of 64; its
-    // other grids keep the precision they have always had, FP64 stencils
-    const bool f32_ok = h->precision == CHS_MIXED && h->N % 64 == 0;
+    // the mixed form's FP32 stencils run where NCL3 is a multiple of 64 and
+    // NCL1 one of 16; its other grids keep the precision they have always had,
+    // FP64 stencils
+    const bool f32_ok = h->precision == CHS_MIXED && h->N % 64 == 0 && h->L % 16 == 0;
     bool f32 = false;
     // 1. RHS + x solve
     {
@@ -1711,11 +1714,11 @@ int rk3_substep(chs_handle* h, int ns, double dt) {
         const int kr = use_st ? krs : KR;
         const int nblk = h->M * (h->N / kr);
         const dim3 grx(((nblk + 7) / 8) * 8);
-        // y-marching form: XM_CPT cells of each row per thread (whole waves)
-        // and its LDS ring on this device
+        // y-marching form: XM_CPT cells of each row per thread and its LDS ring
+        // on this device
         // (cn_mode 3: wherever it fits; the mixed form marches for its FP32
         // stencils; FP64 otherwise where the chunks have MARCH_MIN rows)
-        const bool use_xm = use_st && (h->cn_mode == 0 || h->cn_mode == 3) && (KRS / XM_CPT) * h->L % 64 == 0 &&
+        const bool use_xm = use_st && (h->cn_mode == 0 || h->cn_mode == 3) &&
                             (KRS / XM_CPT) * h->L <= (XM_CPT == 1 ? 1024 : 512) &&
                             rhs_xm_smem(h->L, cn->KWx) <= (size_t)h->lds_max &&
                             (h->cn_mode == 3 || f32_ok ||
@@ -1737,7 +1740,7 @@ int rk3_substep(chs_handle* h, int ns, double dt) {
     do {                                                                                                         \
         (void)hipFuncSetAttribute((const void*)k_rhs_xm<KX, XM_PD, XM_CPT, float>,                                \
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm);                          \
-        CHS_LAUNCH((k_rhs_xm<KX, XM_PD, XM_CPT, float>), gm, dim3((KRS / XM_CPT) * h->L), sm, s, g, rk, h->cvisc, \
+        CHS_LAUNCH((k_rhs_xm<KX, XM_PD, XM_CPT, float>), gm, dim3(march_threads((KRS / XM_CPT) * h->L)), sm, s, g, rk, h->cvisc, \
                    h->q, h->pr, h->h0f, rf, h->partials, wx, lgL, nyc, jc);                                      \
     } while (0)
             switch (cn->KWx) {
@@ -1757,7 +1760,7 @@ int rk3_substep(chs_handle* h, int ns, double dt) {
     do {                                                                                               \
         (void)hipFuncSetAttribute((const void*)k_rhs_xm<KX, XM_PD, XM_CPT>, hipFuncAttributeMaxDynamicSharedMemorySize, \
                                   (int)sm);                                                            \
-        CHS_LAUNCH((k_rhs_xm<KX, XM_PD, XM_CPT>), gm, dim3((KRS / XM_CPT) * h->L), sm, s, g, rk, h->cvisc, h->q, h->pr, h->convh0,  \
+        CHS_LAUNCH((k_rhs_xm<KX, XM_PD, XM_CPT>), gm, dim3(march_threads((KRS / XM_CPT) * h->L)), sm, s, g, rk, h->cvisc, h->q, h->pr, h->convh0,  \
                    h->rhs, h->partials, wx, lgL, nyc, jc);                                             \
     } while (0)
             switch (cn->KWx) {
