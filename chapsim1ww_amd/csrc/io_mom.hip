@@ -1219,21 +1219,31 @@ struct IoCnCoef {
     const double *amvr, *apvr; // AMVR, APVR (NND2, 3)
 };
 
-// MOMFA1_X_io / MOMFA2_Z_io / MOMFA3_Y_io (src/MOMFA_io.f90:51-377) for one
-// component IDR: the coefficients of each line are formed on load from the
-// properties, then the segmented solver; DIR 0 = x (cyclic, lines (j, k)),
-// 2 = z (cyclic, lines (i, j)), 1 = y (non-cyclic, lines (i, k), zero
-// boundary values).  The x pass subtracts DPGRNS from the NFLOW component
-// (rows it applies to); the y pass adds the result to G from row N2I.
+// MOMFA1_X_io / MOMFA2_Z_io / MOMFA3_Y_io (src/MOMFA_io.f90:51-377) for the
+// component IDR = blockIdx.y + 1 (a direction's three components depend on
+// nothing of each other, so they share a launch: 3 launches for 9, whose last
+// rounds of blocks fill up); the coefficients of each line are formed on load
+// from the properties, then the segmented solver; DIR 0 = x (cyclic, lines
+// (j, k)), 2 = z (cyclic, lines (i, j)), 1 = y (non-cyclic, lines (i, k),
+// zero boundary values).  The x pass subtracts DPGRNS from the NFLOW
+// component (rows it applies to); the y pass adds the result to G from row
+// N2I and keeps the values it found as G0 (src/SOLVERRK3_MOM_IO.f90:15).
+// Bound: HBM, 32 B/cell and component (y: 48), in 128-byte pieces of 16 lines
+// and in the phases that small blocks overlap.  All components, one launch
+// and solve per component before: 160x96x120 x 125 -> 63, z 62 -> 44, y 128
+// and a copy of G to G0 of 20 -> 65 us; 256x192x256 x 684 -> 348, z 504 ->
+// 285, y 645 + 120 -> 524 us.
 template <int MS, int DIR>
-__global__ void __launch_bounds__(1024) k_io_cn(IoGeo g, int idr, int sub_dpg, const double* __restrict__ MU,
-                                               const double* __restrict__ MSTG, const double* __restrict__ RS,
-                                               double* __restrict__ R, double* __restrict__ Gc,
-                                               const double* __restrict__ dpg, IoCnCoef cf, int LPB, int P) {
+__global__ void __launch_bounds__(512, DIR == 1 ? 4 : 1) k_io_cn(IoGeo g, int nflow, const double* __restrict__ MU,
+                                              const double* __restrict__ MSTG, const double* __restrict__ RS,
+                                              double* __restrict__ R0, double* __restrict__ G, double* __restrict__ G0,
+                                              const double* __restrict__ dpg, IoCnCoef cf, int LPB, int P) {
 #pragma clang fp contract(off)
     extern __shared__ unsigned char smem[];
     const int L = g.L, M = g.M, N = g.N;
     const int LP = L * (M + 2), CS = LP * N;
+    const int idr = blockIdx.y + 1;
+    double* R = R0 + (size_t)(idr - 1) * L * M * N;
     const int n = DIR == 0 ? L : (DIR == 2 ? N : M);
     const int nlines = DIR == 0 ? M * N : (DIR == 2 ? L * M : L * N);
     const int ll = threadIdx.x % LPB, seg = threadIdx.x / LPB;
@@ -1246,92 +1256,70 @@ __global__ void __launch_bounds__(1024) k_io_cn(IoGeo g, int idr, int sub_dpg, c
         else { li = line % L; lk = line / L; }
     }
     const double* RSc = RS + (size_t)(idr - 1) * CS;
-    const double dp = sub_dpg ? *dpg : 0.0;
+    const double dp = DIR == 0 && idr == nflow ? *dpg : 0.0;
     // wall-row coefficients of u, w in y that TDMA_COEF sets aside
     // (src/TDMA_COEF.f90:86-96)
     const double amvr1 = 4.0 / (2.0 / ldc(g.dyci, 1) + 1.0 / ldc(g.dyfi, 0)) * (2.0 * ldc(g.dyfi, 0));
     const double apvrn = 4.0 / (2.0 / ldc(g.dyci, M - 1) + 1.0 / ldc(g.dyfi, M - 1)) * (2.0 * ldc(g.dyfi, M - 1));
     double a[MS], b[MS], c[MS], d[MS];
-    // x and z: branch-free over the rows (rows past n form row n - 1's
-    // coefficients, invalid lines those of line 0, and become identity rows
-    // after), so the loads of all rows are issued before the first wait; y
-    // skips them (its wall-row branches split the loads anyway, and the
-    // clamped form measured slower there)
+    // The thread's rows share their neighbours: RHO_STG of rows first-1 ..
+    // first+MS and the MS+1 viscosities between them are loaded once each
+    // (MU from first-1 for the component along the line, MU_STG from first
+    // for the others), all before the first wait; cyclic lines are whole
+    // segments, y rows past the ghost row M + 1 repeat it.
+    const int first = seg * MS;
+    const bool own = idr == (DIR == 0 ? 1 : DIR == 2 ? 3 : 2);   // the component along the lines
+    const double* X = own ? MU : MSTG + (size_t)(DIR == 0 ? idr - 2 : DIR == 2 ? (idr == 1 ? 1 : 2) : idr - 1) * CS;
+    const int st = DIR == 0 ? 1 : DIR == 2 ? LP : L;             // from row to row in the ghost-aware arrays
+    const int row0 = DIR == 0 ? L * lj + LP * lk : DIR == 2 ? li + L * lj : li + L + LP * lk;   // row 0 of the line
+    const int sr = DIR == 0 ? 1 : DIR == 2 ? L * M : L;          // the same in R
+    const int rr0 = DIR == 0 ? L * (lj - 1) + L * M * lk : DIR == 2 ? li + L * (lj - 1) : li + L * M * lk;
+    auto at = [&](int m) {   // offset of row m = -1 .. n of the line
+        return row0 + st * (DIR == 1 ? min(m, n) : (m < 0 ? n - 1 : m >= n ? m - n : m));
+    };
+    double rs[MS + 2], x[MS + 1];
+    double m0 = 0.0, m1 = 0.0, mM = 0.0, mP = 0.0;   // MU of the wall rows (y lines of u and w)
+    if (DIR == 1 && !own && seg == 0) {
+        m0 = MU[at(-1)];
+        m1 = MU[at(0)];
+    }
+    if (DIR == 1 && !own && first + MS >= n && first < n) {
+        mM = MU[at(n - 1)];
+        mP = MU[at(n)];
+    }
+#pragma unroll
+    for (int l = 0; l < MS + 2; ++l) rs[l] = RSc[at(first - 1 + l)];
+#pragma unroll
+    for (int l = 0; l < MS + 1; ++l) x[l] = X[at(first - (own ? 1 : 0) + l)];
+#pragma unroll
+    for (int l = 0; l < MS; ++l) d[l] = R[rr0 + sr * min(first + l, n - 1)];
 #pragma unroll
     for (int l = 0; l < MS; ++l) {
-        if (DIR == 1 && !(valid && seg * MS + l < n)) {
-            a[l] = 0.0; b[l] = 1.0; c[l] = 0.0; d[l] = 0.0;
-            continue;
-        }
-        const int m = min(seg * MS + l, n - 1);
-        const int IC = DIR == 0 ? m : li, JC = DIR == 1 ? m + 1 : lj, KC = DIR == 2 ? m : lk;
-        const int cc = IC + L * JC + LP * KC;
-        const int e = IC + L * (JC - 1) + L * M * KC;
-        double AMU, APU, am, ap, ac;
-        if (DIR == 0) {
-            const int IM = IC == 0 ? L - 1 : IC - 1, IP = IC == L - 1 ? 0 : IC + 1;
-            const int cm = cc - IC + IM, cp = cc - IC + IP;
-            // u: MU at (IM, IC), coefficient c1; v, w: MU_STG(., 1 | 2) at (IC, IP), c2
-            const bool u = idr == 1;
-            const double* X = u ? MU : MSTG + (size_t)(idr - 2) * CS;
-            const double k = u ? cf.c1 : cf.c2;
-            AMU = -k * X[u ? cm : cc];
-            APU = -k * X[u ? cc : cp];
-            am = AMU / RSc[cm];
-            ap = APU / RSc[cp];
-            ac = 1.0 - (AMU + APU) / RSc[cc];
-        } else if (DIR == 2) {
-            const int KM = KC == 0 ? N - 1 : KC - 1, KP = KC == N - 1 ? 0 : KC + 1;
-            const int cm = cc + LP * (KM - KC), cp = cc + LP * (KP - KC);
-            // w: MU at (KM, KC), c1; u, v: MU_STG(., 2 | 3) at (KC, KP), c2
-            const bool w = idr == 3;
-            const double* X = w ? MU : MSTG + (size_t)(idr == 1 ? 1 : 2) * CS;
-            const double k = w ? cf.c1 : cf.c2;
-            AMU = -k * X[w ? cm : cc] * 1.0;
-            APU = -k * X[w ? cc : cp] * 1.0;
-            am = AMU / RSc[cm];
-            ap = APU / RSc[cp];
-            ac = 1.0 - (AMU + APU) / RSc[cc];
+        double AMU, APU;
+        if (DIR != 1) {
+            const double k = own ? cf.c1 : cf.c2;
+            AMU = -k * x[l];
+            APU = -k * x[l + 1];
+            a[l] = AMU / rs[l];
+            c[l] = APU / rs[l + 2];
         } else {
-            const int cm = cc - L, cp = cc + L;   // rows 0 and M + 1 are the ghost rows
-            const double amv = cf.amvr[(idr - 1) * (M + 1) + JC - 1], apv = cf.apvr[(idr - 1) * (M + 1) + JC - 1];
-            const double* FM = MSTG + (size_t)(idr - 1) * CS;
-            if (idr == 1 || idr == 3) {
-                if (JC == 1) {
-                    const double MUQT = (MU[cc] + MU[cm]) * 0.5;
-                    AMU = -cf.c2 * amvr1 * MUQT;
-                    APU = -cf.c2 * apv * FM[cp];
-                    am = 0.0;
-                    ap = APU / RSc[cp];
-                } else if (JC == M) {
-                    const double MUQT = (MU[cc] + MU[cp]) * 0.5;
-                    AMU = -cf.c2 * amv * FM[cc];
-                    APU = -cf.c2 * apvrn * MUQT;
-                    am = AMU / RSc[cm];
-                    ap = 0.0;
-                } else {
-                    AMU = -cf.c2 * amv * FM[cc];
-                    APU = -cf.c2 * apv * FM[cp];
-                    am = AMU / RSc[cm];
-                    ap = APU / RSc[cp];
-                }
-                ac = 1.0 - (AMU + APU) / RSc[cc];
-            } else {
-                AMU = -cf.c1 * amv * MU[cm];
-                APU = -cf.c1 * apv * MU[cc];
-                am = AMU / RSc[cm];
-                ap = APU / RSc[JC == 1 ? cp : cc];
-                ac = 1.0 - (AMU + APU) / RSc[cc];
+            const int JC = min(first + l, n - 1) + 1;
+            const double k = own ? cf.c1 : cf.c2;
+            AMU = -k * cf.amvr[(idr - 1) * (M + 1) + JC - 1] * x[l];
+            APU = -k * cf.apvr[(idr - 1) * (M + 1) + JC - 1] * x[l + 1];
+            if (!own) {
+                if (JC == 1) AMU = -k * amvr1 * ((m1 + m0) * 0.5);
+                if (JC == M) APU = -k * apvrn * ((mM + mP) * 0.5);
             }
+            a[l] = !own && JC == 1 ? 0.0 : AMU / rs[l];
+            c[l] = !own && JC == M ? 0.0 : APU / (own && JC > 1 ? rs[l + 1] : rs[l + 2]);
         }
-        a[l] = am;
-        b[l] = ac;
-        c[l] = ap;
-        d[l] = (DIR == 0 && (idr != 2 || JC >= 2)) ? R[e] - dp : R[e];
+        b[l] = 1.0 - (AMU + APU) / rs[l + 1];
+        if (DIR == 0 && (idr != 2 || lj >= 2)) d[l] -= dp;
     }
 #pragma unroll
     for (int l = 0; l < MS; ++l) {
-        if (!(valid && seg * MS + l < n)) {
+        if (!(valid && first + l < n)) {
             a[l] = 0.0; b[l] = 1.0; c[l] = 0.0; d[l] = 0.0;
         }
     }
@@ -1346,20 +1334,30 @@ __global__ void __launch_bounds__(1024) k_io_cn(IoGeo g, int idr, int sub_dpg, c
     }
     seg_solve<MS, double>(a, b, c, d, LPB, P, ll, seg, valid, DIR != 1, smem);
     if (!valid) return;
+    if (DIR == 1) {
+        // rows of G loaded together (row n - 1 again past the end)
+        double* Gc = G + (size_t)(idr - 1) * CS + li + LP * lk;
+        double* Gc0 = G0 + (size_t)(idr - 1) * CS + li + LP * lk;
+        double go[MS];
+#pragma unroll
+        for (int l = 0; l < MS; ++l) go[l] = Gc[L * (min(seg * MS + l, n - 1) + 1)];
+#pragma unroll
+        for (int l = 0; l < MS; ++l) {
+            const int JC = seg * MS + l + 1;
+            if (JC > n) continue;
+            Gc0[L * JC] = go[l];
+            if (JC >= (idr == 2 ? 2 : 1)) Gc[L * JC] = d[l] + go[l];
+        }
+        if (seg == 0) Gc0[0] = Gc[0];   // the ghost rows, which no solve changes
+        if (seg == P - 1) Gc0[L * (M + 1)] = Gc[L * (M + 1)];
+        return;
+    }
 #pragma unroll
     for (int l = 0; l < MS; ++l) {
         const int m = seg * MS + l;
         if (m >= n) continue;
-        const int IC = DIR == 0 ? m : li, JC = DIR == 1 ? m + 1 : lj, KC = DIR == 2 ? m : lk;
-        const int e = IC + L * (JC - 1) + L * M * KC;
-        if (DIR == 1) {
-            if (JC >= (idr == 2 ? 2 : 1)) {
-                const int cc = IC + L * JC + LP * KC;
-                Gc[cc] = d[l] + Gc[cc];
-            }
-        } else {
-            R[e] = d[l];
-        }
+        const int IC = DIR == 0 ? m : li, JC = lj, KC = DIR == 2 ? m : lk;
+        R[IC + L * (JC - 1) + L * M * KC] = d[l];
     }
 }
 
@@ -1367,35 +1365,63 @@ __global__ void __launch_bounds__(1024) k_io_cn(IoGeo g, int idr, int sub_dpg, c
 // first copies its LPB rows of RHS, of the viscosity the component uses (MU
 // for u, MU_STG for v and w) and of RHO_STG with coalesced loads into LDS
 // (row stride L + 1: the lanes of a wave, LPB lines x consecutive segments,
-// then fall on distinct banks), forms the coefficients from there exactly as
-// k_io_cn<MS, 0> does, solves, and writes the rows back through LDS.
+// then fall on distinct banks; four elements of each array in flight per
+// thread), forms the coefficients from there exactly as k_io_cn<MS, 0> does, solves, and writes the rows back through LDS.
 inline size_t io_cn_x_smem(int L, int LPB, int P) {
-    return std::max(sizeof(double) * 3 * (size_t)LPB * (L + 1), seg_smem_bytes<double>(LPB, P));
+    return std::max(sizeof(double) * 3 * (size_t)LPB * (L + 1), seg_smem_bytes<double>(LPB, P, true));
 }
 
 template <int MS>
-__global__ void __launch_bounds__(1024) k_io_cn_x(IoGeo g, int idr, int sub_dpg, const double* __restrict__ MU,
-                                                 const double* __restrict__ MSTG, const double* __restrict__ RS,
-                                                 double* __restrict__ R, const double* __restrict__ dpg, IoCnCoef cf,
-                                                 int LPB, int P) {
+__global__ void __launch_bounds__(512) k_io_cn_x(IoGeo g, int nflow, const double* __restrict__ MU,
+                                                const double* __restrict__ MSTG, const double* __restrict__ RS,
+                                                double* __restrict__ R0, const double* __restrict__ dpg, IoCnCoef cf,
+                                                int LPB, int P) {
 #pragma clang fp contract(off)
     extern __shared__ unsigned char smem[];
     const int L = g.L, M = g.M, N = g.N;
     const int LP = L * (M + 2), CS = LP * N, RL = L + 1;
+    const int idr = blockIdx.y + 1;
+    double* R = R0 + (size_t)(idr - 1) * L * M * N;
     const int nlines = M * N, line0 = blockIdx.x * LPB;
     double* sR = reinterpret_cast<double*>(smem);
     double* sX = sR + LPB * RL;
     double* sS = sX + LPB * RL;
     const double* X = idr == 1 ? MU : MSTG + (size_t)(idr - 2) * CS;  // MU for u, MU_STG(., 1 | 2) for v | w
     const double* RSc = RS + (size_t)(idr - 1) * CS;
-    for (int e = threadIdx.x; e < LPB * L; e += blockDim.x) {
-        const int ll = e / L, i = e - ll * L, line = line0 + ll;
-        if (line < nlines) {
-            const int lj = line % M + 1, lk = line / M;
-            const int cc = i + L * lj + LP * lk, ee = i + L * (lj - 1) + L * M * lk;
-            sR[ll * RL + i] = R[ee];
-            sX[ll * RL + i] = X[cc];
-            sS[ll * RL + i] = RSc[cc];
+    // (row l2, column i) of the staged rows' element e, and the row's line
+    const int j00 = line0 % M, k00 = line0 / M;
+    const float Linv = 1.0f / (float)L;
+    auto elem = [&](int e, int& l2, int& i, int& lj, int& lk) {
+        l2 = (int)(((float)e + 0.5f) * Linv);   // e < 2^13
+        i = e - l2 * L;
+        lj = j00 + min(l2, nlines - 1 - line0);
+        lk = k00;
+        while (lj >= M) {
+            lj -= M;
+            ++lk;
+        }
+    };
+    // EB elements of the three arrays in flight per thread (elements past the
+    // last repeat it, rows past the last line repeat that line's)
+    constexpr int EB = 4;
+    const int ne = LPB * L;
+    for (int e0 = threadIdx.x; e0 < ne; e0 += EB * blockDim.x) {
+        int o[EB];
+        double vr[EB], vx[EB], vs[EB];
+#pragma unroll
+        for (int q = 0; q < EB; ++q) {
+            int l2, i, lj, lk;
+            elem(min(e0 + q * (int)blockDim.x, ne - 1), l2, i, lj, lk);
+            o[q] = l2 * RL + i;
+            vr[q] = R[i + L * lj + L * M * lk];
+            vx[q] = X[i + L * (lj + 1) + LP * lk];
+            vs[q] = RSc[i + L * (lj + 1) + LP * lk];
+        }
+#pragma unroll
+        for (int q = 0; q < EB; ++q) {
+            sR[o[q]] = vr[q];
+            sX[o[q]] = vx[q];
+            sS[o[q]] = vs[q];
         }
     }
     __syncthreads();
@@ -1403,29 +1429,30 @@ __global__ void __launch_bounds__(1024) k_io_cn_x(IoGeo g, int idr, int sub_dpg,
     const int line = line0 + ll;
     const bool valid = line < nlines;
     const int lj = valid ? line % M + 1 : 1;
-    const double dp = sub_dpg ? *dpg : 0.0;
+    const double dp = idr == nflow && (idr != 2 || lj >= 2) ? *dpg : 0.0;
     const double* xr = sX + ll * RL;
     const double* sr = sS + ll * RL;
-    double a[MS], b[MS], c[MS], d[MS];
+    const int first = seg * MS, xo = first - (idr == 1 ? 1 : 0);   // whole segments: MS divides L
+    const double kc = idr == 1 ? cf.c1 : cf.c2;
+    double a[MS], b[MS], c[MS], d[MS], rs[MS + 2], x[MS + 1];
+    auto wrap = [&](int m) { return m < 0 ? L - 1 : m >= L ? m - L : m; };
+#pragma unroll
+    for (int l = 0; l < MS + 2; ++l) rs[l] = sr[wrap(first - 1 + l)];
+#pragma unroll
+    for (int l = 0; l < MS + 1; ++l) x[l] = xr[wrap(xo + l)];
 #pragma unroll
     for (int l = 0; l < MS; ++l) {
-        const int m = seg * MS + l;
-        a[l] = 0.0; b[l] = 1.0; c[l] = 0.0; d[l] = 0.0;
-        if (!valid || m >= L) continue;
-        const int IM = m == 0 ? L - 1 : m - 1, IP = m == L - 1 ? 0 : m + 1;
-        double AMU, APU;
-        if (idr == 1) {
-            AMU = -cf.c1 * xr[IM];
-            APU = -cf.c1 * xr[m];
-        } else {
-            AMU = -cf.c2 * xr[m];
-            APU = -cf.c2 * xr[IP];
+        const double AMU = -kc * x[l], APU = -kc * x[l + 1];
+        a[l] = AMU / rs[l];
+        c[l] = APU / rs[l + 2];
+        b[l] = 1.0 - (AMU + APU) / rs[l + 1];
+        d[l] = sR[ll * RL + first + l] - dp;
+    }
+#pragma unroll
+    for (int l = 0; l < MS; ++l) {
+        if (!valid) {
+            a[l] = 0.0; b[l] = 1.0; c[l] = 0.0; d[l] = 0.0;
         }
-        a[l] = AMU / sr[IM];
-        c[l] = APU / sr[IP];
-        b[l] = 1.0 - (AMU + APU) / sr[m];
-        const double rv = sR[ll * RL + m];
-        d[l] = (idr != 2 || lj >= 2) ? rv - dp : rv;
     }
     __syncthreads();   // the staged rows are read: seg_solve reuses the LDS
     seg_solve<MS, double>(a, b, c, d, LPB, P, ll, seg, valid, true, smem);
@@ -1438,9 +1465,10 @@ __global__ void __launch_bounds__(1024) k_io_cn_x(IoGeo g, int idr, int sub_dpg,
         }
     }
     __syncthreads();
-    for (int e = threadIdx.x; e < LPB * L; e += blockDim.x) {
-        const int l2 = e / L, i = e - l2 * L, ln = line0 + l2;
-        if (ln < nlines) R[i + L * (ln % M) + L * M * (ln / M)] = sR[l2 * RL + i];
+    for (int e = threadIdx.x; e < ne; e += blockDim.x) {
+        int l2, i, rj, rk;
+        elem(e, l2, i, rj, rk);
+        if (line0 + l2 < nlines) R[i + L * rj + L * M * rk] = sR[l2 * RL + i];
     }
 }
 
@@ -1513,19 +1541,29 @@ int io_prepare(chs_handle* h, const chs_thermal_fields* tf, const chs_io_fields*
     return CHS_OK;
 }
 
-// launch one factorised line solve of the RK-CN branch
+// launch one direction's line solves of the RK-CN branch, all components
 template <int DIR>
-static int io_cn_launch(chs_handle* h, const IoGeo& g, int idr, int sub_dpg, const IoArrays& a, double* R,
-                        double* Gc, const IoCnCoef& cf) {
+static int io_cn_launch(chs_handle* h, const IoGeo& g, int nflow, const IoArrays& a, const IoCnCoef& cf) {
     const int n = DIR == 0 ? h->L : (DIR == 2 ? h->N : h->M);
     const int nlines = DIR == 0 ? h->M * h->N : (DIR == 2 ? h->L * h->M : h->L * h->N);
     int MS = 0, P = 0, LPB = 0;
-    // x lines are contiguous in memory: few lines per block (8) put a wave's
-    // lanes on consecutive segments of the same lines, so its loads coalesce
     CHS_CHECK(tdma_seg_config(n, DIR != 1, &MS, &P, &LPB, 1024, DIR == 0), CHS_E_ARG,
               "chs_solverrk3_mom_io: no segmented solver layout for a line length of " + std::to_string(n));
-    const dim3 grid((nlines + LPB - 1) / LPB), block(LPB * P);
-    const size_t sm = seg_smem_bytes<double>(LPB, P);
+    // 8-row segments wherever they fit (4 or 12 rows for cyclic lines that only
+    // those divide).  x lines are contiguous in memory: 8 lines per block put a
+    // wave's lanes on consecutive segments of the same lines; y and z: 16 lines
+    // (128-byte accesses), more for short lines.  Small blocks, so that one's
+    // loads overlap another's reduced systems: at 160x96x120 per component
+    // z 15.6 (32 lines: 16.4, 8: 19.6), y 22.7 (32: 29.7, 8: 31.1) us; x with
+    // 4 lines 30.6 against 26.2 us.
+    if (DIR == 1 || (n % 8 == 0 && n >= 16)) {
+        MS = 8;
+        P = (n + 7) / 8;
+    }
+    while (LPB > (DIR == 0 ? 8 : 16) && LPB * P > 128) LPB /= 2;
+    while (LPB > 2 && LPB * P > 512) LPB /= 2;
+    const dim3 grid((nlines + LPB - 1) / LPB, 3), block(LPB * P);
+    const size_t sm = seg_smem_bytes<double>(LPB, P, DIR != 1);
     const hipStream_t s = h->stream;
     const char* nm = DIR == 0 ? "io_cn_x" : (DIR == 2 ? "io_cn_z" : "io_cn_y");
     hipEvent_t ev;
@@ -1533,9 +1571,8 @@ static int io_cn_launch(chs_handle* h, const IoGeo& g, int idr, int sub_dpg, con
     const size_t smx = io_cn_x_smem(h->L, LPB, P);
     if (DIR == 0 && h->cn_mode != 2 && smx <= 65536) {
 #define IO_CN_X(MSV) \
-    CHS_LAUNCH((k_io_cn_x<MSV>), grid, block, smx, s, g, idr, sub_dpg, a.mu, a.ms, a.rs, R, h->scalars, cf, LPB, P)
+    CHS_LAUNCH((k_io_cn_x<MSV>), grid, block, smx, s, g, nflow, a.mu, a.ms, a.rs, h->rhs, h->scalars, cf, LPB, P)
         switch (MS) {
-            case 16: IO_CN_X(16); break;
             case 12: IO_CN_X(12); break;
             case 4: IO_CN_X(4); break;
             default: IO_CN_X(8); break;
@@ -1543,13 +1580,13 @@ static int io_cn_launch(chs_handle* h, const IoGeo& g, int idr, int sub_dpg, con
 #undef IO_CN_X
     } else {
 #define IO_CN(MSV) \
-    CHS_LAUNCH((k_io_cn<MSV, DIR>), grid, block, sm, s, g, idr, sub_dpg, a.mu, a.ms, a.rs, R, Gc, h->scalars, cf, LPB, P)
-        switch (MS) {
-            case 16: IO_CN(16); break;
-            case 12: IO_CN(12); break;
-            case 4: IO_CN(4); break;
-            default: IO_CN(8); break;
-        }
+    CHS_LAUNCH((k_io_cn<MSV, DIR>), grid, block, sm, s, g, nflow, a.mu, a.ms, a.rs, h->rhs, a.g, a.g0, h->scalars, cf, LPB, P)
+        if (DIR == 1 || MS == 8)
+            IO_CN(8);
+        else if (MS == 12)
+            IO_CN((DIR == 1 ? 8 : 12));
+        else
+            IO_CN((DIR == 1 ? 8 : 4));
 #undef IO_CN
     }
     h->timer.end(ev, nm, s);
@@ -1569,7 +1606,6 @@ static int io_substep_cn(chs_handle* h, const chs_io_fields* f, const IoArrays& 
     const IoGeo g = io_geo(h);
     const dim3 gi = io_grid(h, h->M);
     const long nb = io_tiles(h, h->M);
-    const size_t ncell = (size_t)h->L * h->M * h->N;
     hipEvent_t ev;
     h->timer.begin("io_terms_cn", s, &ev);
 #define IO_TERMS_CN(GR)                                                                                          \
@@ -1590,14 +1626,9 @@ static int io_substep_cn(chs_handle* h, const chs_io_fields* f, const IoArrays& 
     const IoCnCoef cx{FACOE * 4.0 / 3.0 * h->dxqi, FACOE * h->dxqi, h->amvr, h->apvr};
     const IoCnCoef cz{FACOE * 4.0 / 3.0 * h->dzqi, FACOE * h->dzqi, h->amvr, h->apvr};
     const IoCnCoef cy{FACOE * 4.0 / 3.0, FACOE, h->amvr, h->apvr};
-    const size_t CS = (size_t)h->L * (h->M + 2) * h->N;
-    for (int idr = 1; idr <= 3; ++idr) {
-        double* R = h->rhs + (size_t)(idr - 1) * ncell;
-        double* Gc = a.g + (size_t)(idr - 1) * CS;
-        CHS_TRY(io_cn_launch<0>(h, g, idr, p.nflow == idr, a, R, Gc, cx));
-        CHS_TRY(io_cn_launch<2>(h, g, idr, 0, a, R, Gc, cz));
-        CHS_TRY(io_cn_launch<1>(h, g, idr, 0, a, R, Gc, cy));
-    }
+    CHS_TRY(io_cn_launch<0>(h, g, p.nflow, a, cx));
+    CHS_TRY(io_cn_launch<2>(h, g, p.nflow, a, cz));
+    CHS_TRY(io_cn_launch<1>(h, g, p.nflow, a, cy));
     CHS_LAUNCH(k_io_massflux, io_grid(h, h->M + 2), dim3(64, 4), 0, s, g, a.g, nullptr, h->scalars, p.nflow);
     h->timer.begin("io_divg", s, &ev);
     CHS_LAUNCH(k_io_divg, gi, dim3(64, 4), 0, s, g, a.g, nullptr, a.drhodtp, 1.0 / dt / talp, h->rhsllphi);
@@ -1624,11 +1655,12 @@ int io_substep(chs_handle* h, const chs_thermal_fields* tf, const chs_io_fields*
     const double talp = TGAM_IO[ns] + TROH_IO[ns];
     hipEvent_t ev;
     IoParams p{prm->thermal, prm->nflow, prm->flowdrvtp, prm->gravdir, prm->cfgv, prm->f_a};
-    // G0 = G (src/SOLVERRK3_MOM_IO.f90:15): a copy in the RK-CN branch and for
-    // NFLOW = 2; otherwise k_io_terms writes G0 and G + RHS ("fold"), the mass
+    // G0 = G (src/SOLVERRK3_MOM_IO.f90:15): a copy for NFLOW = 2, written by
+    // the y solves in the RK-CN branch; otherwise k_io_terms writes G0 and G + RHS ("fold"), the mass
     // flux pass disappears and k_io_update takes DPGRNS off
     const bool fold = !prm->visimplicit && prm->nflow != 2;
-    if (!fold) CHS_HIP(hipMemcpyAsync(f->g0, f->g, 3 * ngh * sizeof(double), hipMemcpyDeviceToDevice, s));
+    if (!fold && !prm->visimplicit)
+        CHS_HIP(hipMemcpyAsync(f->g0, f->g, 3 * ngh * sizeof(double), hipMemcpyDeviceToDevice, s));
     if (prm->visimplicit) return io_substep_cn(h, f, a, p, ns, dt, talp);   // no DIVG_U_io in that branch
     // the marching form: IOKR k rows of whole x lines, one cell per thread (at
     // most 512) and the LDS ring on this device; chs_set_cn_solver mode 2

@@ -1785,7 +1785,9 @@ int rk3_substep(chs_handle* h, int ns, double dt) {
             const int P = h->L / XMS;
             const int nthr = XLPB * P;
             const size_t sm = std::max(sizeof(double) * (3 * KR * (size_t)(h->L + 1) + (size_t)nthr),
-                                       seg_smem_bytes<double>(XLPB, P));
+                                       seg_smem_bytes<double>(XLPB, P, true));
+            if (sm > 65536)
+                (void)hipFuncSetAttribute((const void*)k_rhs_x, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm);
             CHS_LAUNCH(k_rhs_x, grx, dim3(nthr), sm, s, g, rk, h->cvisc, h->q, h->pr, h->convh0, h->rhs, h->partials,
                        xa, xb, xc, lgL);
         }
@@ -1831,8 +1833,9 @@ int rk3_substep(chs_handle* h, int ns, double dt) {
             return CHS_E_ARG;
         }
         const int nlines = 3 * h->L * h->M;
+        while (LPB > 16 && LPB * Pz > 128) LPB /= 2;   // small blocks overlap their phases
         const dim3 gz((nlines + LPB - 1) / LPB), bz(LPB * Pz);
-        const size_t smz = seg_smem_bytes<double>(LPB, Pz);
+        const size_t smz = seg_smem_bytes<double>(LPB, Pz, true);
         const int usedpg = 1;
         if (!use_st) {
         h->timer.begin("z_solve", s, &ev);

@@ -9,11 +9,11 @@
 namespace chs {
 
 // Segmented solver: LPB lines per block, P = ceil(n / MS) segments per line.
-template <int MS>
+template <int MS, bool CYC>
 __global__ void __launch_bounds__(1024) k_tdma_seg(const double* __restrict__ A, const double* __restrict__ B,
                                                    const double* __restrict__ Cc, double* __restrict__ Rr,
                                                    const double* __restrict__ bc, int n, int nlines,
-                                                   long long es, long long ls, int LPB, int P, int cyclic) {
+                                                   long long es, long long ls, int LPB, int P) {
     extern __shared__ unsigned char smem[];
     const int tid = threadIdx.x;
     // consecutive lanes take consecutive lines, also where the rows are the
@@ -46,7 +46,7 @@ __global__ void __launch_bounds__(1024) k_tdma_seg(const double* __restrict__ A,
             d[l] = 0.0;
         }
     }
-    if (!cyclic && valid) {
+    if (!CYC && valid) {
         // the end rows take the boundary values BC(line,1:2) (TDMAIJJ_nonCYC.f90:93-97,108-113)
         if (seg == 0) {
             if (bc) d[0] = d[0] - a[0] * bc[line];
@@ -63,7 +63,7 @@ __global__ void __launch_bounds__(1024) k_tdma_seg(const double* __restrict__ A,
                 }
         }
     }
-    seg_solve<MS, double>(a, b, c, d, LPB, P, ll, seg, valid, cyclic != 0, smem);
+    seg_solve<MS, double>(a, b, c, d, LPB, P, ll, seg, valid, CYC, smem);
     if (valid) {
 #pragma unroll
         for (int l = 0; l < MS; ++l) {
@@ -263,14 +263,15 @@ int tdma_launch(const double* a, const double* b, const double* c, double* r, co
     //     reduced systems have no serial sweep: 500x192 8.3 (15.2), 2000x504
     //     20.0 (20.1), rows contiguous 500x192 6.9 (20.3), 20000x504 144 (287);
     //     only a whole grid's contiguous lines of whole 12-row segments stay
-    //     with k_tdma_seg: 65536x192 120 against 148 us
+    //     with k_tdma_seg: 65536x192 110 against 148 us, 40000x360 at 12 x 16
+    //     (two blocks per CU; 12 x 32: 170) 132 us
     const bool grid_lines = nlines >= 32768, lines_contig = ls == 1;
     int MS = 8, LPB = 0;
     const int p12 = (n + 11) / 12;   // 12 x 32: blocks whose waves fill a CU's 16 (one block of 9 would leave 7 idle)
     if (lines_contig && grid_lines && ((p12 >= 4 && p12 <= 16) || (p12 >= 28 && p12 <= 32)) &&
         (!cyclic || n % 12 == 0)) {
         MS = 12;
-        LPB = 32;
+        LPB = cyclic && p12 > 16 ? 16 : 32;
     } else if (cyclic) {
         const int p = (n - 1 + MS - 1) / MS;
         LPB = es == 1 ? lines_per_block(p, 64, 2, 64)
@@ -291,11 +292,13 @@ int tdma_launch(const double* a, const double* b, const double* c, double* r, co
     const int P = (n + MS - 1) / MS;
     if (LPB > 0 && P * LPB <= 1024) {
         const dim3 grid((nlines + LPB - 1) / LPB), block(LPB * P);
-        const size_t sm = seg_smem_bytes<double>(LPB, P);
-        if (MS == 12)
-            CHS_LAUNCH(k_tdma_seg<12>, grid, block, sm, s, a, b, c, r, bc, n, nlines, es, ls, LPB, P, cyclic);
+        const size_t sm = seg_smem_bytes<double>(LPB, P, cyclic != 0);
+        if (cyclic)
+            CHS_LAUNCH((k_tdma_seg<12, true>), grid, block, sm, s, a, b, c, r, bc, n, nlines, es, ls, LPB, P);
+        else if (MS == 12)
+            CHS_LAUNCH((k_tdma_seg<12, false>), grid, block, sm, s, a, b, c, r, bc, n, nlines, es, ls, LPB, P);
         else
-            CHS_LAUNCH(k_tdma_seg<8>, grid, block, sm, s, a, b, c, r, bc, n, nlines, es, ls, LPB, P, cyclic);
+            CHS_LAUNCH((k_tdma_seg<8, false>), grid, block, sm, s, a, b, c, r, bc, n, nlines, es, ls, LPB, P);
         return CHS_OK;
     }
     const int bs = 256;
