@@ -204,20 +204,24 @@ __device__ __forceinline__ void march_split(int tid, int L, int& r, int& i) {
     i = tid - r * L;
 }
 constexpr int MARCH_MIN = 8;
-inline int march_chunk_rows(int rows, int nkg, size_t smem, int lds_max, bool fill) {
-    const int bpc = fill ? std::max(1, std::min(4, (int)((size_t)lds_max / std::max<size_t>(smem, 1)))) : 1;
+// rows per chunk: ncol columns of blocks, bpc blocks to a CU, fill rows' worth
+// of a chunk's start-up
+inline int chunk_rows(int rows, long ncol, int bpc, int fill) {
     int best = rows;
     long cost = -1;
     for (int nyc = 1; nyc <= std::max(1, rows / 4); ++nyc) {
         const int jc = (rows + nyc - 1) / nyc;
-        const long per = ((long)nkg * ((rows + jc - 1) / jc) + 7) / 8;   // blocks of an XCD
-        const long c = (per + 32 * bpc - 1) / (32 * bpc) * (jc + 3);
+        const long per = (ncol * ((rows + jc - 1) / jc) + 7) / 8;   // blocks of an XCD
+        const long c = (per + 32 * bpc - 1) / (32 * bpc) * (jc + fill);
         if (cost < 0 || c < cost) {
             cost = c;
             best = jc;
         }
     }
     return best;
+}
+inline int march_chunk_rows(int rows, int nkg, size_t smem, int lds_max, bool fill) {
+    return chunk_rows(rows, nkg, fill ? std::max(1, std::min(4, (int)((size_t)lds_max / std::max<size_t>(smem, 1)))) : 1, 3);
 }
 
 // xz-plane sums in two stages of a fixed order: one block of 256 threads per

@@ -888,8 +888,9 @@ __global__ void __launch_bounds__(64) k_y_window(Geo g, const TR* __restrict__ R
         for (int e = threadIdx.x; e < (jn - j0) * W; e += blockDim.x) sw[e] = wy[((size_t)c * M + j0) * W + e];
         __syncthreads();
         if (!valid) return;
-        if (c == 1 && ch == 0) {
-            // v's row-1 right-hand side: the u increment on j = 1 (row 0 of u's solve)
+        if (c == 1 && j0 <= KW) {
+            // v's row-1 right-hand side: the u increment on j = 1 (row 0 of u's
+            // solve), for every chunk whose window reaches row 0
             const TR* Ru = R2 + (size_t)k * LM + i;
 #pragma unroll
             for (int m = KW; m < W; ++m) du0 += wy[m] * double(Ru[(size_t)(m - KW) * L]);
@@ -996,6 +997,184 @@ __global__ void __launch_bounds__(256) k_z_window(Geo g, const T* __restrict__ R
 #pragma unroll
             for (int m = 0; m < W - 1; ++m) win[m] = win[m + 1];
             win[W - 1] = rn[u];
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// k_zy_window: the z and the y window in one pass.  A block owns ZYK
+// consecutive k and pr of the rows of j of all components and i tiles of 64
+// (the same rows for every k tile, so that the blocks of an XCD, which runs
+// neighbouring k tiles together, march the same rows and find each other's k
+// halo in their L2).  Row j of RHS with KZ halo rows of k either side goes
+// through a double-buffered LDS plane (loaded two rows ahead in registers),
+// each thread forms the z solve of its CK cells from there and pushes it into
+// their register windows of 2 KY + 1 rows, from which the y solve of row
+// j - KY leaves.  RHS2 is not written and read back (48 of 120 B/cell) and
+// two launches become one; the expressions and their order are k_z_window's
+// and k_y_window's.  Bound: HBM; at 256x192x256 129 + 187 -> 220 us (4.4 TB/s
+// of 78 B/cell, the windows' fill included), mixed 60 + 164 -> 176 us.  CK =
+// 2 cells per thread where the windows fit (KY <= 8), 1 at KY = 12; 1 at KY =
+// 8 249 us, 8 k rows per block 258 us.
+// ---------------------------------------------------------------------------
+constexpr int ZYK = 16;
+inline size_t zy_smem(int rows, int KZ, int KY, size_t tsize) {
+    return sizeof(double) * (size_t)rows * (2 * KY + 1) + 2 * tsize * (size_t)(ZYK + 2 * KZ) * 64;
+}
+
+template <int KZ, int KY, int CK, class T = double>
+__global__ void __launch_bounds__(64 * ZYK / CK) k_zy_window(Geo g, const T* __restrict__ R, double* __restrict__ Q,
+                                                            const double* __restrict__ dpg, double xone, int use_dpg,
+                                                            const double* __restrict__ wz,
+                                                            const double* __restrict__ wy, int np, int pr) {
+    constexpr int TZ = ZYK / CK, NR = ZYK + 2 * KZ, PL = (NR + TZ - 1) / TZ, W = 2 * KY + 1, WZ = 2 * KZ + 1;
+    extern __shared__ double sw[];   // the rows' weights [j1 - j0][W], then two planes [NR][64]
+    const int L = g.L, M = g.M, N = g.N, LM = L * M;
+    const int ntx = (L + 63) / 64, nkt = (N + ZYK - 1) / ZYK;
+    const int t = xcd_tile(blockIdx.x, gridDim.x);
+    if (t >= np * nkt) return;
+    const int kt = t % nkt, piece = t / nkt;
+    const int lane = threadIdx.x & 63, tz = threadIdx.x >> 6;
+    T* pl = reinterpret_cast<T*>(sw + (size_t)min(pr, M) * W);
+    // this thread's rows of the plane (past the last: that one again) and their offsets in RHS
+    int lr[PL], rk[PL];
+#pragma unroll
+    for (int u = 0; u < PL; ++u) {
+        const int r = min(tz + TZ * u, NR - 1);
+        const int k = (kt * ZYK - KZ + r) % N;
+        lr[u] = r * 64 + lane;
+        rk[u] = LM * (k < 0 ? k + N : k);
+    }
+    T w[WZ];
+#pragma unroll
+    for (int m = 0; m < WZ; ++m) w[m] = T(wz[m]);
+    auto put = [&](int b, const T(&x)[PL], T D) {
+#pragma unroll
+        for (int u = 0; u < PL; ++u) pl[b * NR * 64 + lr[u]] = x[u] - D;
+    };
+    auto zrow = [&](int b, T(&z)[CK]) {
+        const T* p = pl + b * NR * 64 + (tz * CK) * 64 + lane;
+#pragma unroll
+        for (int q = 0; q < CK; ++q) z[q] = T(0.0);
+#pragma unroll
+        for (int m = 0; m < WZ + CK - 1; ++m) {
+            const T v = p[m * 64];
+#pragma unroll
+            for (int q = 0; q < CK; ++q)
+                if (m - q >= 0 && m - q < WZ) z[q] += w[m - q] * v;
+        }
+    };
+    auto corr = [&](int cc) { return T((use_dpg && cc == g.mc) ? dpg[0] * xone : 0.0); };
+    // the piece's rows, segment by segment of one (component, i tile)
+    const int r1 = min(3 * ntx * M, (piece + 1) * pr);
+    for (int r0 = piece * pr; r0 < r1;) {
+        const int col = r0 / M, c = col / ntx, it = col - c * ntx;
+        const int j0 = r0 - col * M, j1 = min(M, j0 + r1 - r0);
+        r0 += j1 - j0;
+        const int i = min(it * 64 + lane, L - 1);
+        __syncthreads();   // the weights and planes of the segment before are read
+        for (int e = threadIdx.x; e < (j1 - j0) * W; e += 64 * TZ) sw[e] = wy[(c * M + j0) * W + e];
+        auto load = [&](const T* Rc, int j, T(&x)[PL]) {
+            const int o = i + L * min(j, M - 1);
+#pragma unroll
+            for (int u = 0; u < PL; ++u) x[u] = Rc[rk[u] + o];
+        };
+        T x[PL];
+        double du0[CK];
+#pragma unroll
+        for (int q = 0; q < CK; ++q) du0[q] = 0.0;
+        if (c == 1 && j0 <= KY) {
+            // v's row-1 right-hand side: the u increment on j = 1 (row 0 of u's
+            // solve), for every segment whose window reaches row 0
+            const T D = corr(0);
+            load(R, 0, x);
+#pragma unroll 1
+            for (int j = 0; j <= KY; ++j) {
+                put(j & 1, x, D);
+                load(R, j + 1, x);
+                __syncthreads();   // the other plane was last read two rows ago
+                T z[CK];
+                zrow(j & 1, z);
+                const double wj = wy[KY + j];
+#pragma unroll
+                for (int q = 0; q < CK; ++q) du0[q] += wj * double(z[q]);
+            }
+            __syncthreads();
+        }
+        const T D = corr(c);
+        const T* Rc = R + (size_t)c * LM * N;
+        // the thread's cells of Q (cells past the grid: the last row's, not stored)
+        bool ok[CK];
+        double* Qc[CK];
+#pragma unroll
+        for (int q = 0; q < CK; ++q) {
+            const int k = kt * ZYK + tz * CK + q;
+            ok[q] = it * 64 + lane < L && k < N;
+            Qc[q] = Q + qidx(g, c, i, 1, min(k, N - 1));
+        }
+        double win[CK][W];
+#pragma unroll
+        for (int q = 0; q < CK; ++q)
+#pragma unroll
+            for (int m = 0; m < W; ++m) win[q][m] = 0.0;
+        const int js = max(0, j0 - KY);
+        load(Rc, js, x);
+        put(0, x, D);
+        load(Rc, js + 1, x);
+        double qn[CK];
+#pragma unroll
+        for (int q = 0; q < CK; ++q) qn[q] = Qc[q][L * j0];
+        __syncthreads();
+        // row jr through plane b: into the windows; row jr - KY leaves
+        auto step = [&](int jr, int b) {
+            put(b ^ 1, x, D);
+            load(Rc, jr + 2, x);
+            const int j = jr - KY;
+            double qv[CK];
+#pragma unroll
+            for (int q = 0; q < CK; ++q) {
+                qv[q] = qn[q];
+                qn[q] = Qc[q][L * min(max(j + 1, j0), M - 1)];
+            }
+            T z[CK];
+            zrow(b, z);
+#pragma unroll
+            for (int q = 0; q < CK; ++q) {
+#pragma unroll
+                for (int m = 0; m < W - 1; ++m) win[q][m] = win[q][m + 1];
+                win[q][W - 1] = jr >= M ? 0.0 : (c == 1 && jr == 0) ? du0[q] : double(z[q]);
+            }
+            if (j >= j0 && j < j1) {
+                const double* wr = sw + (j - j0) * W;
+                double acc[CK];
+#pragma unroll
+                for (int q = 0; q < CK; ++q) acc[q] = 0.0;
+#pragma unroll
+                for (int m = 0; m < W; ++m) {
+                    const double wm = wr[m];
+#pragma unroll
+                    for (int q = 0; q < CK; ++q) acc[q] += wm * win[q][m];
+                }
+#pragma unroll
+                for (int q = 0; q < CK; ++q)
+                    if (ok[q] && !(c == 1 && j == 0)) Qc[q][L * j] = acc[q] + qv[q];
+            }
+            __syncthreads();
+        };
+        // steps in fours (register names of the windows rotate); those past
+        // the last row leave nothing
+        for (int jr = js; jr < j1 + KY; jr += 4) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) step(jr + u, u & 1);
+        }
+#pragma unroll
+        for (int q = 0; q < CK; ++q) {
+            if (!ok[q]) continue;
+            if (j0 == 0) {
+                Qc[q][-L] = 0.0;
+                if (c == 1) Qc[q][0] = 0.0;
+            }
+            if (j1 == M) Qc[q][L * M] = 0.0;
         }
     }
 }
@@ -1702,6 +1881,7 @@ int rk3_substep(chs_handle* h, int ns, double dt) {
     // FP64 stencils
     const bool f32_ok = h->precision == CHS_MIXED && h->N % 64 == 0 && h->L % 16 == 0;
     bool f32 = false;
+    bool zy = false;   // the z and y solves in one pass
     // 1. RHS + x solve
     {
         const double COE = -facoe * h->dxqi;
@@ -1803,7 +1983,48 @@ int rk3_substep(chs_handle* h, int ns, double dt) {
         const double za = RMC2, zc = RMC2, zb = 1.0 - zc - za;
         const double xone = 1.0 / (xa + xb + xc);
         const int usedpg0 = 1;
-        if (use_st) {
+        // the z and y windows in one pass: pieces of zpr rows of the 3 ntx M of a
+        // k tile, about one block per CU (its registers leave room for one of
+        // 8 waves; two measured 233 against 220 us).  Every piece also marches
+        // 2 KW rows to fill its windows, so short pieces lose to the two
+        // kernels: a step at 128x80x128 (15 rows) 470 / 455 us, 128x100x128 (19)
+        // 533 / 528, 96x80x160 (20) 446 / 453, 200x40x160 (20) 457 / 491,
+        // 160x96x120 (27) 603 / 601, 128x128x128 (24) 597 / 679.
+        const int zkt = (h->N + ZYK - 1) / ZYK, zrows = 3 * ((h->L + 63) / 64) * h->M;
+        const int zpr = (zrows + std::max(1, 256 / zkt) - 1) / std::max(1, 256 / zkt);
+        zy = use_st && cn->KWz <= 8 && cn->KW <= 12 && (h->cn_mode == 3 || zpr >= 20) &&
+             zy_smem(std::min(zpr, h->M), cn->KWz, cn->KW, sizeof(double)) <= (size_t)h->lds_max;
+        if (zy) {
+            const double *wz = cn->dev + cn->oz, *wy = cn->dev + cn->oy;
+            const int np = (zrows + zpr - 1) / zpr;
+            const dim3 gzy((unsigned)(8 * ((np * zkt + 7) / 8)));
+            h->timer.begin("zy_solve", s, &ev);
+#define CHS_ZY(KZ, KY, CK, T)                                                                                     \
+    do {                                                                                                          \
+        const size_t sm = zy_smem(std::min(zpr, h->M), KZ, KY, sizeof(T));                                                              \
+        if (sm > 65536)                                                                                           \
+            (void)hipFuncSetAttribute((const void*)k_zy_window<KZ, KY, CK, T>,                                    \
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm);                       \
+        CHS_LAUNCH((k_zy_window<KZ, KY, CK, T>), gzy, dim3(64 * ZYK / CK), sm, s, g,                              \
+                   reinterpret_cast<const T*>(h->rhs), h->q, h->scalars, xone, usedpg0, wz, wy, np, zpr);          \
+    } while (0)
+#define CHS_ZYK(KZ, T)                                                                                            \
+    do {                                                                                                          \
+        if (cn->KW == 4) CHS_ZY(KZ, 4, 2, T);                                                                     \
+        else if (cn->KW == 8) CHS_ZY(KZ, 8, 2, T);                                                                \
+        else CHS_ZY(KZ, 12, 1, T);                                                                                \
+    } while (0)
+            if (f32) {
+                if (cn->KWz == 4) CHS_ZYK(4, float);
+                else CHS_ZYK(8, float);
+            } else {
+                if (cn->KWz == 4) CHS_ZYK(4, double);
+                else CHS_ZYK(8, double);
+            }
+#undef CHS_ZYK
+#undef CHS_ZY
+            h->timer.end(ev, "zy_solve", s);
+        } else if (use_st) {
             const int zkc = zwin_chunk(h);
             const dim3 gzw(3 * h->M * ((h->L + 63) / 64), ((h->N + zkc - 1) / zkc + 3) / 4);
             const double* wz = cn->dev + cn->oz;
@@ -1849,7 +2070,9 @@ int rk3_substep(chs_handle* h, int ns, double dt) {
         }
     }
     // 3. y solves + Q update + BC_WALL_Q
-    if (use_st) {
+    if (zy) {
+        // done with the z solves
+    } else if (use_st) {
         const int yjc = ywin_chunk(h);
         const int nch = (h->M + yjc - 1) / yjc;
         const dim3 gy(h->N * ((h->L + 63) / 64), 3, nch), by(64);
