@@ -75,6 +75,10 @@ __global__ void k_counts_out(unsigned long long* c, unsigned long long* host) {
         c[threadIdx.x] = 0ull;
     }
 }
+int props_counts_out(unsigned long long* c, unsigned long long* host, hipStream_t s) {
+    CHS_LAUNCH(k_counts_out, dim3(1), dim3(64), 0, s, c, host);
+    return CHS_OK;
+}
 
 // PT threads, PCELL cells per thread and chunk of persistent blocks.  WIDE
 // (LdsTab): bound by the LDS reads of the searches and records and by the
@@ -443,7 +447,7 @@ int props_update(chs_props* p, int mode, const double* h, long long nrow, long l
     else
         CHS_TRY(mlp_update(p, h, rw, T, rho, mu, kap, cp, p->ucnt, p->stream));
     unsigned long long* host = p->ecnt_host + 2;
-    CHS_LAUNCH(k_counts_out, dim3(1), dim3(64), 0, p->stream, p->ucnt, host);
+    CHS_TRY(props_counts_out(p->ucnt, host, p->stream));
     CHS_HIP(hipStreamSynchronize(p->stream));
     if (n_fallback) *n_fallback = (long long)host[1];
     if (host[0]) {
