@@ -84,17 +84,20 @@ static const double TROH_IO[4] = {0.0, 0.0, -17.0 / 60.0, -5.0 / 12.0};
 // VELOCITY_CALC_io with BC_WALL_Q_io; one thread per cell of rows 0..M+1.
 // Every array is distinct (restrict): all loads can be issued before the
 // first store.
-__global__ void __launch_bounds__(256) k_io_prepare(IoGeo g, const double* __restrict__ D,
-                                                    const double* __restrict__ D0, const double* __restrict__ V,
-                                                    const double* __restrict__ V0, const double* __restrict__ G,
-                                                    const double* __restrict__ G0, double* __restrict__ drhodtp,
-                                                    double* __restrict__ rs, double* __restrict__ ms,
-                                                    double* __restrict__ q, double* __restrict__ drhoi, int thermal,
-                                                    double ca, double cb, double cd, int nj, int j0) {
+__device__ __forceinline__ void io_prepare_cell(const IoGeo& g, const double* __restrict__ D,
+                                                const double* __restrict__ D0, const double* __restrict__ V,
+                                                const double* __restrict__ V0, const double* __restrict__ G,
+                                                const double* __restrict__ G0, double* __restrict__ drhodtp,
+                                                double* __restrict__ rs, double* __restrict__ ms,
+                                                double* __restrict__ q, double* __restrict__ drhoi, int thermal,
+                                                double ca, double cb, double cd, int IC, int J, int KC) {
 #pragma clang fp contract(off)
-    IO_CELL(nj, j0);   // rows j0 .. j0+nj-1 of 0..M+1
-    const int J = JT;   // ghost-aware row 0..M+1
-    const int c = at(IC, J, KC);
+    const int L = g.L, M = g.M, N = g.N;
+    const int IP = IC == L - 1 ? 0 : IC + 1, IM = IC == 0 ? L - 1 : IC - 1;
+    const int KP = KC == N - 1 ? 0 : KC + 1, KM = KC == 0 ? N - 1 : KC - 1;
+    const int LP = L * (M + 2), CS = LP * N;
+    auto at = [&](int i, int j, int k) { return i + L * j + LP * k; };
+    const int c = at(IC, J, KC);   // J: ghost-aware row 0..M+1
     double r1, r2, r3;
     if (thermal) {
         // Every branch below only selects values: the ghost rows evaluate
@@ -177,12 +180,25 @@ __global__ void __launch_bounds__(256) k_io_prepare(IoGeo g, const double* __res
     }
 }
 
+__global__ void __launch_bounds__(256) k_io_prepare(IoGeo g, const double* __restrict__ D,
+                                                    const double* __restrict__ D0, const double* __restrict__ V,
+                                                    const double* __restrict__ V0, const double* __restrict__ G,
+                                                    const double* __restrict__ G0, double* __restrict__ drhodtp,
+                                                    double* __restrict__ rs, double* __restrict__ ms,
+                                                    double* __restrict__ q, double* __restrict__ drhoi, int thermal,
+                                                    double ca, double cb, double cd) {
+    IO_CELL(g.M + 2, 0);
+    io_prepare_cell(g, D, D0, V, V0, G, G0, drhodtp, rs, ms, q, drhoi, thermal, ca, cb, cd, IC, JT, KC);
+}
+
 // k_io_prepare (thermal = 1) on the rows 2..M, marching along y: a thread
 // owns the column (IC, KC) of a chunk of rows.  There, Jw = Jr = J and Jm =
 // J-1, and the row J-1 parts of RHO_STG y and MU_STG x-y, y-z are the row
 // parts of the step before (the same expressions), so they carry over in
 // registers with v of G and G0 at J; the values of row J+1 are loaded one
-// step ahead.  Rows 0, 1 and M+1 (wrap and wall rows) are k_io_prepare's.
+// step ahead.  Rows 0, 1 and M+1 (wrap and wall rows) are the first
+// ne blocks', a cell per thread as in k_io_prepare (two launches of their own
+// took 11 us at 128^3).  Bound: HBM, 171 B/cell: 460 us at 256x192x256.
 struct PrepRow {
     double d, dim, dkm, d0, d0im, d0km;              // RHO at the cell, i-1, k-1; RHO0 likewise
     double v, vim, vkm, vimkm, v0, v0im, v0km, v0imkm;  // MU, MU0 at the cell, i-1, k-1, i-1 k-1
@@ -195,12 +211,20 @@ __global__ void __launch_bounds__(256) k_io_prepare_m(IoGeo g, const double* __r
                                                       const double* __restrict__ G0, double* __restrict__ drhodtp,
                                                       double* __restrict__ rs, double* __restrict__ ms,
                                                       double* __restrict__ q, double* __restrict__ drhoi, double ca,
-                                                      double cb, double cd, int nyc, int jc) {
+                                                      double cb, double cd, int nyc, int jc, int ne) {
 #pragma clang fp contract(off)
     const int L = g.L, M = g.M, N = g.N;
     const int ni = (L + 63) / 64, nk = (N + 3) / 4;
+    if ((int)blockIdx.x < ne) {
+        const int e = blockIdx.x, r = e / (ni * nk);
+        const int IC = e % ni * 64 + threadIdx.x, KC = e / ni % nk * 4 + threadIdx.y;
+        if (r < 3 && IC < L && KC < N)
+            io_prepare_cell(g, D, D0, V, V0, G, G0, drhodtp, rs, ms, q, drhoi, 1, ca, cb, cd, IC, r < 2 ? r : M + 1, KC);
+        return;
+    }
     const int nt = ni * nk * nyc, per = (nt + 7) / 8;
-    const int t = (blockIdx.x % 8) * per + blockIdx.x / 8;  // XCD x: tiles x*per .. (x+1)*per-1
+    const int bid = blockIdx.x - ne;                // ne: a multiple of 8
+    const int t = (bid % 8) * per + bid / 8;        // XCD x: tiles x*per .. (x+1)*per-1
     if (t >= nt) return;
     const int it = t % ni, kt = (t / ni) % nk, yc = t / (ni * nk);
     const int IC = it * 64 + threadIdx.x, KC = kt * 4 + threadIdx.y;
@@ -1519,23 +1543,20 @@ int io_prepare(chs_handle* h, const chs_thermal_fields* tf, const chs_io_fields*
     const double ca = TGAM_IO[ns] + TROH_IO[ns], cb = TROH_IO[ns], cd = TGAM_IO[ns] - 2.0;
     const IoGeo g = io_geo(h);
     const long ncol = (long)((h->L + 63) / 64) * ((h->N + 3) / 4);
-    // the marching form takes three launches: on grids of fewer than 4096
-    // row tiles (64^3: 1056) one row-tile launch is faster (13.3 against
-    // 20.4 us); at 128^3 (8320) the march wins (98.0 against 101.0 us)
+    // on grids of fewer than 4096 row tiles (64^3: 1056) the row tiles are
+    // faster (13.3 against 20.4 us with the march and its edge rows apart); at
+    // 128^3 (8320) the march wins (86 against 101 us)
     if (prm->thermal && h->M >= 3 && h->cn_mode != 2 && (h->cn_mode == 3 || ncol * (h->M + 2) >= 4096)) {
-        // rows 2..M marching (about 8 blocks per CU), rows 0, 1 and M+1 in row tiles
+        // rows 2..M marching (about 8 blocks per CU), rows 0, 1 and M+1 a cell per thread
         int nyc = (int)std::max(1L, std::min((long)(h->M - 1) / 4, (2048 + ncol - 1) / ncol));
         const int jc = (h->M - 1 + nyc - 1) / nyc;
         nyc = (h->M - 1 + jc - 1) / jc;
-        CHS_LAUNCH(k_io_prepare_m, dim3((unsigned)(8 * ((ncol * nyc + 7) / 8))), dim3(64, 4), 0, s, g, a.rho,
-                   a.rho0, a.mu, a.mu0, a.g, a.g0, a.drhodtp, a.rs, a.ms, a.q, drhoi, ca, cb, cd, nyc, jc);
-        CHS_LAUNCH(k_io_prepare, io_grid(h, 2), dim3(64, 4), 0, s, g, a.rho, a.rho0, a.mu, a.mu0, a.g, a.g0,
-                   a.drhodtp, a.rs, a.ms, a.q, drhoi, prm->thermal, ca, cb, cd, 2, 0);
-        CHS_LAUNCH(k_io_prepare, io_grid(h, 1), dim3(64, 4), 0, s, g, a.rho, a.rho0, a.mu, a.mu0, a.g, a.g0,
-                   a.drhodtp, a.rs, a.ms, a.q, drhoi, prm->thermal, ca, cb, cd, 1, h->M + 1);
+        const int ne = (int)(8 * ((3 * ncol + 7) / 8));
+        CHS_LAUNCH(k_io_prepare_m, dim3((unsigned)(ne + 8 * ((ncol * nyc + 7) / 8))), dim3(64, 4), 0, s, g, a.rho,
+                   a.rho0, a.mu, a.mu0, a.g, a.g0, a.drhodtp, a.rs, a.ms, a.q, drhoi, ca, cb, cd, nyc, jc, ne);
     } else {
         CHS_LAUNCH(k_io_prepare, io_grid(h, h->M + 2), dim3(64, 4), 0, s, g, a.rho, a.rho0, a.mu, a.mu0, a.g,
-                   a.g0, a.drhodtp, a.rs, a.ms, a.q, drhoi, prm->thermal, ca, cb, cd, h->M + 2, 0);
+                   a.g0, a.drhodtp, a.rs, a.ms, a.q, drhoi, prm->thermal, ca, cb, cd);
     }
     h->timer.end(ev, "io_prepare", s);
     return CHS_OK;
