@@ -1612,24 +1612,16 @@ static void thomas_ld(int n, const ld* a, const ld* b, const ld* c, ld* x) {
     for (int i = n - 2; i >= 0; --i) x[i] = gg[i] - h[i] * x[i + 1];
 }
 
-// Smallest K whose dropped tail sum_{|m|>K} |row_m| is <= tol * sum |row|
-static int trunc_width(const std::vector<ld>& row, int centre, bool cyclic) {
-    const int n = (int)row.size();
-    ld tot = 0;
-    for (ld v : row) tot += fabsl(v);
-    for (int K = 0; K <= KMAX; ++K) {
-        ld tail = 0;
-        for (int m = 0; m < n; ++m) {
-            int d = m - centre;
-            if (cyclic) {
-                d = ((d % n) + n) % n;
-                if (d > n / 2) d -= n;
-            }
-            if (d > K || d < -K) tail += fabsl(row[m]);
-        }
-        if (tail <= 1e-17L * tot) return K;
-    }
-    return KMAX + 1;
+// Smallest K <= KMAX whose dropped tail is <= 1e-17 of the row's absolute sum:
+// s[d], d = 0..KMAX: the absolute sum of the row's entries at distance d,
+// beyond: that of the entries further off.  KMAX + 1 if there is none.
+static int trunc_width(const ld* s, ld beyond) {
+    ld tot = beyond;
+    for (int d = 0; d <= KMAX; ++d) tot += s[d];
+    if (!(beyond <= 1e-17L * tot)) return KMAX + 1;   // NaN too
+    int K = KMAX;
+    for (ld tail = beyond; K > 0 && tail + s[K] <= 1e-17L * tot; --K) tail += s[K];
+    return K;
 }
 
 // Inverse of the constant cyclic system (a, b, c) of size n, row 0: the
@@ -1651,55 +1643,147 @@ static int cyclic_stencil(int n, double a, double b, double c, std::vector<doubl
     std::vector<ld> v(n);
     for (int i = 0; i < n; ++i) v[i] = x[i] - fact * u[i];
     // symmetric circulant (a == c): row 0 of the inverse = column 0
-    const int K = trunc_width(v, 0, true);
+    ld sd[KMAX + 1] = {}, beyond = 0;
+    for (int i = 0; i < n; ++i) {
+        const int d = std::min(i, n - i);
+        (d <= KMAX ? sd[d] : beyond) += fabsl(v[i]);
+    }
+    const int K = trunc_width(sd, beyond);
     if (K > KMAX) return K;
     w.assign(2 * K + 1, 0.0);
     for (int m = -K; m <= K; ++m) w[m + K] = (double)v[((m % n) + n) % n];
     return K;
 }
 
+// Device weights with the pinned buffer they are uploaded from, sized for the
+// widest windows; used: recorded after the upload and after each substep that
+// read dev.
+struct CnBuf {
+    double *dev = nullptr, *host = nullptr;
+    hipEvent_t used = nullptr;
+};
+
 struct CnStencils {
     double facoe = -1.0;
     int Kx = -1, Kz = -1, Ky = -1, KW = 4, KWz = 4, KWx = 4;
     bool ok = false;
-    double* dev = nullptr;   // wx[2KWx+1] | wz[2KWz+1] | wy[3][M][2KW+1], zero-padded windows
+    CnBuf buf;               // (ok only)
+    double* dev = nullptr;   // buf.dev: wx[2KWx+1] | wz[2KWz+1] | wy[3][M][2KW+1], zero-padded windows
     size_t ox = 0, oz = 0, oy = 0;
-    std::vector<double> host;   // the uploaded values (kept alive for the stream-ordered copy)
-    hipEvent_t used = nullptr;  // recorded after the last substep that read dev
 };
 
 // The stencils of the last few FACOE values of one handle.  Entries are
-// evicted oldest first; an evicted entry's device memory is freed once its
-// last-use event has completed (never while a queued substep may read it).
+// evicted oldest first; an evicted entry's buffers serve a later one once
+// their last-use event has completed (never while a queued substep may read
+// them).  A run that changes DT with its CFL number brings three new values a
+// step: allocating and freeing for each waited for the GPU (a step of its own
+// DT, with the cost of the inverses: 64^3 1244 -> 270, 256x192x256 11254 -> 2981 us).
 struct CnCache {
-    std::list<CnStencils> live;   // list: entries keep their addresses
-    std::vector<std::pair<double*, hipEvent_t>> retired;
+    std::list<CnStencils> live;   // list: entries keep their addresses; at most 8
+    std::vector<CnBuf> retired;
 };
 
-static void reap_retired(CnCache& c, bool wait) {
-    for (size_t i = 0; i < c.retired.size();) {
-        auto& r = c.retired[i];
-        const bool done = r.second == nullptr || (wait ? hipEventSynchronize(r.second) == hipSuccess
-                                                       : hipEventQuery(r.second) == hipSuccess);
-        if (!done) {
-            ++i;
+static void free_buf(CnBuf& b) {
+    if (b.dev) (void)hipFree(b.dev);
+    if (b.host) (void)hipHostFree(b.host);
+    if (b.used) (void)hipEventDestroy(b.used);
+    b = CnBuf{};
+}
+
+// Buffers of n doubles: retired ones that are free again, else new ones, but
+// no more than 4 are left waiting (then the oldest is waited for).
+static int take_buf(CnCache& c, size_t n, CnBuf* out) {
+    for (size_t i = 0; i <= c.retired.size(); ++i) {
+        const bool wait = i == c.retired.size();
+        if (wait && i < 4) break;
+        const size_t r = wait ? 0 : i;
+        if ((wait ? hipEventSynchronize(c.retired[r].used) : hipEventQuery(c.retired[r].used)) != hipSuccess) {
+            (void)hipGetLastError();   // not ready, or recorded into a graph: not to be reused
             continue;
         }
-        if (r.first) (void)hipFree(r.first);
-        if (r.second) (void)hipEventDestroy(r.second);
-        c.retired.erase(c.retired.begin() + i);
+        *out = c.retired[r];
+        c.retired.erase(c.retired.begin() + (long)r);
+        return CHS_OK;
     }
+    CnBuf b;
+    hipError_t e = hipMalloc((void**)&b.dev, n * sizeof(double));
+    if (e == hipSuccess) e = hipHostMalloc((void**)&b.host, n * sizeof(double), hipHostMallocDefault);
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&b.used, hipEventDisableTiming);
+    if (e != hipSuccess) {
+        free_buf(b);
+        set_error(std::string("CN stencil buffers: ") + hipGetErrorString(e));
+        return CHS_E_HIP;
+    }
+    *out = b;
+    return CHS_OK;
 }
 
 void release_stencils(chs_handle* h) {
     std::lock_guard<std::mutex> lk(h->cn_mu);
     CnCache* c = h->cn_cache;
     if (!c) return;
-    for (auto& e : c->live) c->retired.push_back({e.dev, e.used});
-    c->live.clear();
-    reap_retired(*c, true);
+    for (auto& e : c->live)
+        if (e.dev) c->retired.push_back(e.buf);
+    for (auto& b : c->retired) {
+        (void)hipEventSynchronize(b.used);
+        free_buf(b);
+    }
     delete c;
     h->cn_cache = nullptr;
+}
+
+// Rows of the inverse of component c's y system, distances up to KMAX, to
+// ent[j][KMAX + m] (0 outside the rows); returns the largest truncation width.
+// Column by column as a Thomas solve of a unit vector, with the elimination
+// shared and the sweep down the column cut where what is left can no longer
+// reach the kept entries (1e-48 of the diagonal; 1e-40 is enough for the weights
+// to be those of the full solves to the last bit on wall-refined rows of up to
+// 360).  A column costs its own width instead of NCL2 rows: 2.4 -> 0.2 ms of
+// host time a value of FACOE at NCL2 = 192, 304 -> 117 us at 64.
+static int y_inverse_rows(const chs_handle* h, double facoe, int c, std::vector<double>& ent) {
+    const int M = h->M;
+    std::vector<ld> a(M), den(M), hh(M), gg(M), s((size_t)M * (KMAX + 1), 0), beyond(M, 0);
+    for (int j = 0; j < M; ++j) {
+        const int o = c * (M + 1) + j;
+        const ld b = (ld)(1.0 - facoe * h->h_acvr[o]);
+        const ld cc = j == M - 1 ? (ld)0 : (ld)(-facoe * h->h_apvr[o]);
+        a[j] = j == 0 ? (ld)0 : (ld)(-facoe * h->h_amvr[o]);
+        den[j] = j == 0 ? b : b - a[j] * hh[j - 1];
+        hh[j] = cc / den[j];
+    }
+    constexpr int W = 2 * KMAX + 1;
+    ent.assign((size_t)M * W, 0.0);
+    for (int m = 0; m < M; ++m) {
+        auto put = [&](int j, ld x) {   // entry (j, m) of the inverse
+            const int d = std::abs(j - m);
+            if (d <= KMAX) {
+                ent[(size_t)j * W + KMAX + (m - j)] = (double)x;
+                s[(size_t)j * (KMAX + 1) + d] += fabsl(x);
+            } else {
+                beyond[j] += fabsl(x);
+            }
+        };
+        gg[m] = 1 / den[m];
+        const ld eps = 1e-48L * fabsl(gg[m]), eps_up = 1e-25L * fabsl(gg[m]);   // up: the sums' digits
+        int e = m;
+        while (e < M - 1 && (e - m < KMAX || fabsl(gg[e]) > eps)) {
+            ++e;
+            gg[e] = (0 - a[e] * gg[e - 1]) / den[e];
+        }
+        ld x = gg[e];
+        put(e, x);
+        for (int j = e - 1; j >= m; --j) {
+            x = gg[j] - hh[j] * x;
+            put(j, x);
+        }
+        for (int j = m - 1; j >= 0 && (m - j <= KMAX || fabsl(x) > eps_up); --j) {
+            x = 0 - hh[j] * x;
+            put(j, x);
+        }
+    }
+    int K = 0;
+    for (int j = 0; j < M; ++j) K = std::max(K, trunc_width(s.data() + (size_t)j * (KMAX + 1), beyond[j]));
+    return K;
 }
 
 // Stencils for FACOE (the caller holds h->cn_mu): from the handle's cache, or
@@ -1713,7 +1797,6 @@ static int cn_stencils_locked(chs_handle* h, double facoe, CnStencils** out) {
             *out = &c;
             return CHS_OK;
         }
-    reap_retired(cache, false);
     CnStencils st;
     st.facoe = facoe;
     const int M = h->M;
@@ -1721,73 +1804,48 @@ static int cn_stencils_locked(chs_handle* h, double facoe, CnStencils** out) {
     const double xa = COE, xc = COE, xb = 1.0 - xc - xa;
     const double RMC2 = 1.0 * (-facoe * h->dzqi);
     const double za = RMC2, zc = RMC2, zb = 1.0 - zc - za;
-    std::vector<double> wx, wz;
+    std::vector<double> wx, wz, wy[3];
     st.Kx = cyclic_stencil(h->L, xa, xb, xc, wx);
     st.Kz = cyclic_stencil(h->N, za, zb, zc, wz);
-    // y: full inverse of each component's non-cyclic system (rows j = 0..M-1)
-    std::vector<std::vector<ld>> inv(3 * (size_t)M);
-    const std::vector<double>&amvr = h->h_amvr, &acvr = h->h_acvr, &apvr = h->h_apvr;
-    int Ky = 0;
-    for (int c = 0; c < 3; ++c) {
-        std::vector<ld> a(M), b(M), cc(M), col(M);
-        for (int j = 0; j < M; ++j) {
-            const int o = c * (M + 1) + j;
-            b[j] = (ld)(1.0 - facoe * acvr[o]);
-            cc[j] = (ld)(-facoe * apvr[o]);
-            a[j] = (ld)(-facoe * amvr[o]);
-        }
-        a[0] = 0;
-        cc[M - 1] = 0;
-        for (int j = 0; j < M; ++j) inv[c * M + j].assign(M, 0);
-        for (int m = 0; m < M; ++m) {  // column m of the inverse
-            std::fill(col.begin(), col.end(), (ld)0);
-            col[m] = 1;
-            thomas_ld(M, a.data(), b.data(), cc.data(), col.data());
-            for (int j = 0; j < M; ++j) inv[c * M + j][m] = col[j];
-        }
-        for (int j = 0; j < M; ++j) Ky = std::max(Ky, trunc_width(inv[c * M + j], j, false));
-    }
-    st.Ky = Ky;
+    st.Ky = 0;
+    for (int c = 0; c < 3; ++c) st.Ky = std::max(st.Ky, y_inverse_rows(h, facoe, c, wy[c]));
     auto window = [](int K) { return K <= 4 ? 4 : K <= 8 ? 8 : K <= 12 ? 12 : 16; };
-    st.KW = window(Ky);
+    st.KW = window(st.Ky);
     st.KWz = window(st.Kz);
     st.KWx = window(st.Kx);
     // a periodic window must not wrap onto itself: 2*KW + 1 <= the line length
     st.ok = st.Kx <= KMAX && st.Kz <= KMAX && st.Ky <= KMAX && 2 * st.KWx + 1 <= h->L &&
             2 * st.KWz + 1 <= h->N;
     if (st.ok) {
+        constexpr int WM = 2 * KMAX + 1;
         const int W = 2 * st.KW + 1;
-        Ky = st.KW;
         const size_t nwx = 2 * (size_t)st.KWx + 1, nwz = 2 * (size_t)st.KWz + 1;
-        std::vector<double>& buf = st.host;
-        buf.assign(nwx + nwz + 3 * (size_t)M * W, 0.0);
+        const size_t n = nwx + nwz + 3 * (size_t)M * W;
+        CHS_TRY(take_buf(cache, WM * (2 + 3 * (size_t)M), &st.buf));
+        st.dev = st.buf.dev;
         st.ox = 0;
         st.oz = nwx;
         st.oy = nwx + nwz;
-        std::copy(wx.begin(), wx.end(), buf.begin() + (st.KWx - st.Kx));
-        std::copy(wz.begin(), wz.end(), buf.begin() + st.oz + (st.KWz - st.Kz));
+        double* buf = st.buf.host;
+        std::fill(buf, buf + n, 0.0);
+        std::copy(wx.begin(), wx.end(), buf + (st.KWx - st.Kx));
+        std::copy(wz.begin(), wz.end(), buf + st.oz + (st.KWz - st.Kz));
         for (int c = 0; c < 3; ++c)
-            for (int j = 0; j < M; ++j)
-                for (int m = -Ky; m <= Ky; ++m) {
-                    const int jm = j + m;
-                    if (jm >= 0 && jm < M && m >= -st.Ky && m <= st.Ky)
-                        buf[st.oy + ((size_t)c * M + j) * W + (m + Ky)] = (double)inv[c * M + j][jm];
-                }
-        CHS_HIP(hipMalloc((void**)&st.dev, buf.size() * sizeof(double)));
-        hipError_t e = hipEventCreateWithFlags(&st.used, hipEventDisableTiming);
-        if (e == hipSuccess)
-            e = hipMemcpyAsync(st.dev, buf.data(), buf.size() * sizeof(double), hipMemcpyHostToDevice, h->stream);
+            for (int j = 0; j < M; ++j) {
+                const double* row = wy[c].data() + (size_t)j * WM + KMAX;
+                std::copy(row - st.Ky, row + st.Ky + 1, buf + st.oy + ((size_t)c * M + j) * W + (st.KW - st.Ky));
+            }
+        hipError_t e = hipMemcpyAsync(st.dev, buf, n * sizeof(double), hipMemcpyHostToDevice, h->stream);
+        if (e == hipSuccess) e = hipEventRecord(st.buf.used, h->stream);
         if (e != hipSuccess) {
             (void)hipStreamSynchronize(h->stream);
-            (void)hipFree(st.dev);
-            if (st.used) (void)hipEventDestroy(st.used);
+            free_buf(st.buf);
             set_error(std::string("CN stencil upload: ") + hipGetErrorString(e));
             return CHS_E_HIP;
         }
     }
     if (cache.live.size() >= 8) {
-        CnStencils& old = cache.live.front();
-        cache.retired.push_back({old.dev, old.used});
+        if (cache.live.front().dev) cache.retired.push_back(cache.live.front().buf);
         cache.live.pop_front();
     }
     cache.live.push_back(std::move(st));
@@ -2116,7 +2174,7 @@ int rk3_substep(chs_handle* h, int ns, double dt) {
         h->timer.end(ev, "y_solve", s);
     }
     if (lk.owns_lock()) {
-        if (cn->used) CHS_HIP(hipEventRecord(cn->used, s));
+        if (cn->dev) CHS_HIP(hipEventRecord(cn->buf.used, s));
         lk.unlock();
     }
     // 4. DIVG
