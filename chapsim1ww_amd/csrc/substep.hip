@@ -449,6 +449,11 @@ inline size_t rhs_xm_smem(int L, int KX, size_t tsize = sizeof(double)) {
     return ((b + 7) & ~(size_t)7) + sizeof(double) * ((size_t)(KRS + 1) * L + 16);
 }
 
+constexpr int KRL = 2;   // k rows per block beyond L = 256 (AL)
+inline size_t rhs_xml_smem(int L) {
+    return sizeof(double) * ((size_t)(9 * (KRL + 2) + KRL + 1) * L + 16);
+}
+
 // four consecutive values (16-byte aligned for float, 32 for double)
 __device__ __forceinline__ void store4(double* dst, const double* v) {
     reinterpret_cast<double2*>(dst)[0] = make_double2(v[0], v[1]);
@@ -461,26 +466,34 @@ __device__ __forceinline__ void store4(float* dst, const float* v) {
 // T: the compute type of the cells' right-hand sides, the LDS ring and the x
 // solve (double: the FP64 form; float: the mixed form's FP32 stencils, whose
 // RHS and CONVH0 are stored in FP32).  Q and PR stay FP64 in HBM.
-template <int KX, int PD, int CPT, class T = double>
+//
+// AL, with KRM = 2 k rows: lines beyond 256 values, whose ring leaves no LDS
+// for the x-solve rows.  They take the ring's row J-1, free once every thread
+// has formed its RHS, and leave it before the row J+2 arrives there: two more
+// barriers a row.  Bound: HBM, as below 256; the row tiles read each value of
+// Q nine times through L2 (512x256x384: 1690 us, here 1216, 4.3 TB/s).
+template <int KX, int PD, int CPT, class T = double, int KRM = KRS, bool AL = false>
 __global__ void __launch_bounds__(CPT == 1 ? 1024 : 512) k_rhs_xm(Geo g, RkCoef rk, double cvisc, const double* __restrict__ Q,
                                                const double* __restrict__ PR, T* __restrict__ H0,
                                                T* __restrict__ RHS, double* __restrict__ part,
                                                const double* __restrict__ wx, int lgL, int nyc, int jc) {
-    static_assert(KRS % CPT == 0 && KRS / CPT >= 2, "CPT cells per thread, a low and a high halo row");
-    constexpr int RB = KRS / CPT;  // thread rows
+    static_assert(KRM % CPT == 0 && KRM / CPT >= 2, "CPT cells per thread, a low and a high halo row");
+    static_assert(!AL || (CPT == 1 && PD == 1 && sizeof(T) == 8), "the shared row: one FP64 cell per thread");
+    constexpr int RB = KRM / CPT;  // thread rows
     extern __shared__ double smd[];
     T* sm = reinterpret_cast<T*>(smd);
     // the pressure values stay FP64 (the gradient of a large common level)
     using TP = double;
-    constexpr int KR = KRS, KP = XM_KP, W = 2 * KX + 1;
+    constexpr int KR = KRM, KP = KRM + 2, W = 2 * KX + 1;
     const int L = g.L, M = g.M, N = g.N;
     const int PL = KP * L;            // one component of one ring row
     const int SL = 3 * PL;            // one ring row (u, v, w)
     T* ring = sm;                     // 3 ring rows
     const int LS = L + 2 * KX, Q4 = LS >> 2;
-    T* xr = sm + 3 * SL;              // 3*KR x-solve rows (row_pos layout)
-    TP* pln = reinterpret_cast<TP*>(smd + (sizeof(T) * (size_t)(9 * KP * L + 3 * KR * LS) + 7) / 8);   // PR row J, k0-1 .. k0+KR-1
-    double* red = smd + (sizeof(T) * (size_t)(9 * KP * L + 3 * KR * LS) + 7) / 8 + (KR + 1) * L;
+    T* xr = sm + 3 * SL;              // 3*KR x-solve rows (row_pos layout); AL: the ring's row J-1
+    const int xs = AL ? 0 : 3 * KR * LS;
+    TP* pln = reinterpret_cast<TP*>(smd + (sizeof(T) * (size_t)(9 * KP * L + xs) + 7) / 8);   // PR row J, k0-1 .. k0+KR-1
+    double* red = smd + (sizeof(T) * (size_t)(9 * KP * L + xs) + 7) / 8 + (KR + 1) * L;
     const int nt = (N / KR) * nyc;
     const int per = (nt + 7) / 8;
     const int t = (blockIdx.x % 8) * per + blockIdx.x / 8;  // XCD x: tiles x*per .. (x+1)*per-1
@@ -607,6 +620,10 @@ __global__ void __launch_bounds__(CPT == 1 ? 1024 : 512) k_rhs_xm(Geo g, RkCoef 
             T conv[3], rhs[3];
             rhs_cell<RColT<T>, T, RColT<TP>>(g, rk, cvisc, rc, U, V, Wc, P, n, h0[u], conv, rhs);
             const int ci = i + L * j + L * M * kc[u];
+            if constexpr (AL) {
+                xr = ring + sM * SL;
+                __syncthreads();   // row J-1 has been read
+            }
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
                 if (c != 1 || j != 0) H0[ci + c * LMN] = conv[c];
@@ -628,23 +645,25 @@ __global__ void __launch_bounds__(CPT == 1 ? 1024 : 512) k_rhs_xm(Geo g, RkCoef 
             for (int o = 8; o > 0; o >>= 1) bs += __shfl_xor(bs, o);
             if (tid == 0) part[kg * M + j] = bs;
         }
-        // row J+2 replaces row J-1 in the ring, PR row J+1 replaces row J
-        // (both free since the barrier), before the RHS stores are issued
+        if constexpr (!AL) {
+            // row J+2 replaces row J-1 in the ring, PR row J+1 replaces row J
+            // (both free since the barrier), before the RHS stores are issued
 #pragma unroll
-        for (int c = 0; c < 3; ++c) {
+            for (int c = 0; c < 3; ++c) {
+#pragma unroll
+                for (int u = 0; u < CPT; ++u) {
+                    ring[sM * SL + c * PL + lc[u]] = pa.q[u][c];
+                    h0[u][c] = pa.h[u][c];
+                }
+                ring[sM * SL + c * PL + lh] = pa.qh[c];
+            }
 #pragma unroll
             for (int u = 0; u < CPT; ++u) {
-                ring[sM * SL + c * PL + lc[u]] = pa.q[u][c];
-                h0[u][c] = pa.h[u][c];
+                pln[lc[u]] = pa.p[u];
+                pm[u] = pc[u];
             }
-            ring[sM * SL + c * PL + lh] = pa.qh[c];
+            pln[lph] = pa.ph;
         }
-#pragma unroll
-        for (int u = 0; u < CPT; ++u) {
-            pln[lc[u]] = pa.p[u];
-            pm[u] = pc[u];
-        }
-        pln[lph] = pa.ph;
         // x stencil of the 3*KR rows, 4 outputs per work item
         for (int e = tid; e < 3 * KR * L4; e += blockDim.x) {
             int cr, g4;
@@ -665,6 +684,24 @@ __global__ void __launch_bounds__(CPT == 1 ? 1024 : 512) k_rhs_xm(Geo g, RkCoef 
             }
             T* dst = RHS + (c * LMN + 4 * g4 + L * (j + M * (k0 + rr)));
             store4(dst, o4);
+        }
+        if constexpr (AL) {
+            __syncthreads();   // the x-solve rows have been read
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+#pragma unroll
+                for (int u = 0; u < CPT; ++u) {
+                    ring[sM * SL + c * PL + lc[u]] = pa.q[u][c];
+                    h0[u][c] = pa.h[u][c];
+                }
+                ring[sM * SL + c * PL + lh] = pa.qh[c];
+            }
+#pragma unroll
+            for (int u = 0; u < CPT; ++u) {
+                pln[lc[u]] = pa.p[u];
+                pm[u] = pc[u];
+            }
+            pln[lph] = pa.ph;
         }
         if (PD == 2) pa = pb;
         __syncthreads();
@@ -1950,7 +1987,7 @@ int rk3_substep(chs_handle* h, int ns, double dt) {
         // k halo rows per output) ran 1.3% slower (0.452 vs 0.446 ms)
         const int krs = KRS;
         const int kr = use_st ? krs : KR;
-        const int nblk = h->M * (h->N / kr);
+        int nblk = h->M * (h->N / kr);
         const dim3 grx(((nblk + 7) / 8) * 8);
         // y-marching form: XM_CPT cells of each row per thread and its LDS ring
         // on this device
@@ -1961,6 +1998,17 @@ int rk3_substep(chs_handle* h, int ns, double dt) {
                             rhs_xm_smem(h->L, cn->KWx) <= (size_t)h->lds_max &&
                             (h->cn_mode == 3 || f32_ok ||
                              xm_chunk(h, rhs_xm_smem(h->L, cn->KWx), true) >= MARCH_MIN);
+        // lines beyond 256 values: two k rows per block, the x-solve rows in the
+        // ring, where the chunks have 12 rows (three more fill the ring): a step
+        // at 288x96x128 (24 rows) 1056 -> 1032 us, 320x128x160 1847 -> 1764,
+        // 512x128x128 2291 -> 2045, 512x256x384 14150 -> 12750; 384x64x64 (8
+        // rows) 498 -> 508
+        const size_t sml = rhs_xml_smem(h->L);
+        const bool use_xml = use_st && !use_xm && (h->cn_mode == 0 || h->cn_mode == 3) && KRL * h->L <= 1024 &&
+                             sml <= (size_t)h->lds_max && (long)h->M * (h->N / KRL) <= h->npart &&
+                             (h->cn_mode == 3 ||
+                              (h->L > 256 && march_chunk_rows(h->M, h->N / KRL, sml, h->lds_max, true) >= 12));
+        if (use_xml) nblk = h->M * (h->N / KRL);
         // the mixed form's FP32 stencils: RHS, the x solve and the z solve in
         // FP32 (RHS and RHS2 stored as float in the first half of the FP64
         // buffers), CONVH0 kept in FP32 (h0f); the y elimination stays FP64
@@ -2008,6 +2056,25 @@ int rk3_substep(chs_handle* h, int ns, double dt) {
                 default: CHS_RHSXM(16); break;
             }
 #undef CHS_RHSXM
+        } else if (use_xml) {
+            const int jc = march_chunk_rows(h->M, h->N / KRL, sml, h->lds_max, true);
+            const int nkb = h->N / KRL, nyc = (h->M + jc - 1) / jc;
+            const dim3 gm(8 * ((nkb * nyc + 7) / 8));
+            const double* wx = cn->dev + cn->ox;
+#define CHS_RHSXML(KX)                                                                                           \
+    do {                                                                                                         \
+        const auto kern = k_rhs_xm<KX, 1, 1, double, KRL, true>;                                                 \
+        (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sml);      \
+        CHS_LAUNCH(kern, gm, dim3(march_threads(KRL * h->L)), sml, s, g, rk, h->cvisc, h->q, h->pr, h->convh0,   \
+                   h->rhs, h->partials, wx, lgL, nyc, jc);                                                       \
+    } while (0)
+            switch (cn->KWx) {
+                case 4: CHS_RHSXML(4); break;
+                case 8: CHS_RHSXML(8); break;
+                case 12: CHS_RHSXML(12); break;
+                default: CHS_RHSXML(16); break;
+            }
+#undef CHS_RHSXML
         } else if (use_st) {
             const size_t sm = sizeof(double) * (3 * (size_t)krs * (size_t)(h->L + 2 * cn->KWx) + 4);
             const double* wx = cn->dev + cn->ox;
