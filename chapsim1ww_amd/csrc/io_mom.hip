@@ -436,17 +436,6 @@ __device__ __forceinline__ void io_conv_a(const IoGeo& g, const A& G1, const A& 
     }
 }
 
-// The global-array form, as the RK-CN terms kernel calls it (c = (IC, JC, KC)).
-__device__ __forceinline__ void io_conv(const IoGeo& g, const double* __restrict__ G, const double* __restrict__ Q,
-                                        int IC, int IP, int IM, int JC, int KC, int KP, int KM, double& hx,
-                                        double& hy, double& hz) {
-    const int L = g.L, LP = L * (g.M + 2), CS = LP * g.N;
-    const int c = IC + L * JC + LP * KC, ip = IP - IC, im = IM - IC, kp = (KP - KC) * LP, km = (KM - KC) * LP;
-    io_conv_a(g, cell_acc(G, c, ip, im, kp, km, L), cell_acc(G + CS, c, ip, im, kp, km, L),
-              cell_acc(G + 2 * CS, c, ip, im, kp, km, L), cell_acc(Q, c, ip, im, kp, km, L),
-              cell_acc(Q + CS, c, ip, im, kp, km, L), cell_acc(Q + 2 * CS, c, ip, im, kp, km, L), JC, hx, hy, hz);
-}
-
 // Explicit terms of one cell (CONVECTION_*_io, VISCOUS_ALL_EXPLT_*_io) and
 // RHS_MOM_EXPLICIT_io up to DPGRNS: h = the explicit terms, r = the RHS.
 // G*, Q* by AQ; MU, MU0, DivU, MU_STG, PR by AS; E = EXPLT0 of the cell,
@@ -871,10 +860,6 @@ __global__ void __launch_bounds__(256) k_io_massflux(IoGeo g, double* __restrict
         G[2 * CS + c] = 0.0;
         return;
     }
-    if (!inc) {   // the RK-CN branch updated G in its y solves: wall values only
-        if (J == 1) G[CS + c] = 0.0;
-        return;
-    }
     const int NC = L * M * N;
     const int e = IC + L * (J - 1) + L * M * KC;
     const double dp = *dpg;
@@ -1032,210 +1017,272 @@ __global__ void __launch_bounds__(256) k_io_max2(const double* __restrict__ part
 // VISCOUS_PAR_EXPLT_X/Y/Z_io (src/VISCOUS_X_EXPLICIT_io.f90:116-289,
 // src/VISCOUS_Y_EXPLICIT_io.f90:264-423, src/VISCOUS_Z_EXPLICIT_io.f90:289-460)
 // with the convection, and the RK-CN branch of RHS_MOM_EXPLICIT_io
-// (src/RHS_MOM_EXPLICIT_io.f90:79-93) up to DPGRNS.  inc <- RHS (row 1 of v
-// zero), explt0 <- convection + explicit stress part, divu <- the z density
-// correction (what the reference leaves in DIVU_io), part <- block sums.
-template <int GRAV>
-__global__ void __launch_bounds__(256) k_io_terms_cn(IoGeo g, const double* __restrict__ G,
-                                                     const double* __restrict__ Q, const double* __restrict__ MU,
-                                                     const double* __restrict__ MS, const double* __restrict__ DR,
-                                                     const double* __restrict__ PR, const double* __restrict__ RS,
-                                                     double* __restrict__ E, double* __restrict__ DUo, IoParams p,
-                                                     double tg, double tr, double dt, double adt,
-                                                     double* __restrict__ inc, double* __restrict__ part) {
+// (src/RHS_MOM_EXPLICIT_io.f90:79-93) up to DPGRNS, at one cell: h = the
+// convection and explicit stress part, r = the RHS, ad3 = the z density
+// correction.  G*, Q* by AQ, the rest from global memory by AG; E = EXPLT0.
+template <int GRAV, class AQ, class AG>
+__device__ __forceinline__ void io_terms_cn_cell(const IoGeo& g, const AQ& G1, const AQ& G2, const AQ& G3, const AQ& Q1,
+                                                 const AQ& Q2, const AQ& Q3, const AG& MU, const AG& MS1, const AG& MS2,
+                                                 const AG& MS3, const AG& D1, const AG& D2, const AG& D3, const AG& PR,
+                                                 int JC, const double* E, double rsg, const IoParams& p, double tg,
+                                                 double tr, double dt, double adt, double* h, double* r, double& ad3) {
 #pragma clang fp contract(off)
-    __shared__ double red[256];
+    // row 1 of v is evaluated with a clamped metric index and discarded
+    const int JJ = JC, JJP = JC + 1, JJM = JC >= 2 ? JC - 1 : 1;
+    const double CV = g.cvisc, E1 = E[0], E2 = E[1], E3 = E[2];
+    double hx, hy, hz;
+    io_conv_a(g, G1, G2, G3, Q1, Q2, Q3, JC, hx, hy, hz);
+    double IM1, AD1, IM2, AD2, IM3, AD3;
+    {   // x
+        const double COE1 = -2.0 / 3.0 * g.dxi * CV, COE2 = ldc(g.dyfi, JJ - 1) * CV * 1.0, COE32 = g.dzi * CV * 1.0;
+        double DUDX = (Q1(1, 0, 0) - Q1(0, 0, 0)) * g.dxi;
+        double DVDY = (Q2(0, 1, 0) - Q2(0, 0, 0)) * ldc(g.dyfi, JJ - 1) * 1.0;
+        double DWDZ = (Q3(0, 0, 1) - Q3(0, 0, 0)) * g.dzi * 1.0;
+        const double F_EX = MU(0, 0, 0) * (DVDY + DWDZ), F_IM = MU(0, 0, 0) * DUDX;
+        DUDX = (G1(1, 0, 0) * D1(1, 0, 0) - G1(0, 0, 0) * D1(0, 0, 0)) * g.dxi;
+        const double F_AD = MU(0, 0, 0) * DUDX;
+        DUDX = (Q1(0, 0, 0) - Q1(-1, 0, 0)) * g.dxi;
+        DVDY = (Q2(-1, 1, 0) - Q2(-1, 0, 0)) * ldc(g.dyfi, JJ - 1) * 1.0;
+        DWDZ = (Q3(-1, 0, 1) - Q3(-1, 0, 0)) * g.dzi * 1.0;
+        const double B_EX = MU(-1, 0, 0) * (DVDY + DWDZ), B_IM = MU(-1, 0, 0) * DUDX;
+        DUDX = (G1(0, 0, 0) * D1(0, 0, 0) - G1(-1, 0, 0) * D1(-1, 0, 0)) * g.dxi;
+        const double B_AD = MU(-1, 0, 0) * DUDX;
+        const double X_EX = (F_EX - B_EX) * COE1, X_IM = (F_IM - B_IM) * COE1 * (-2.0);
+        const double X_AD = (F_AD - B_AD) * COE1 * (-2.0);
+        double VP = MS1(0, 1, 0);
+        double DVDX = (Q2(0, 1, 0) - Q2(-1, 1, 0)) * g.dxi;
+        double DUDY = (Q1(0, 1, 0) - Q1(0, 0, 0)) * ldc(g.dyci, JJP - 1) / 1.0;
+        const double F2_EX = VP * DVDX, F2_IM = VP * DUDY;
+        DUDY = (G1(0, 1, 0) * D1(0, 1, 0) - G1(0, 0, 0) * D1(0, 0, 0)) * ldc(g.dyci, JJP - 1) / 1.0;
+        const double F2_AD = VP * DUDY;
+        double VC = MS1(0, 0, 0);
+        DUDY = (Q1(0, 0, 0) - Q1(0, -1, 0)) * ldc(g.dyci, JJ - 1) / 1.0;
+        DVDX = (Q2(0, 0, 0) - Q2(-1, 0, 0)) * g.dxi;
+        const double B2_EX = VC * DVDX, B2_IM = VC * DUDY;
+        DUDY = (G1(0, 0, 0) * D1(0, 0, 0) - G1(0, -1, 0) * D1(0, -1, 0)) * ldc(g.dyci, JJ - 1) / 1.0;
+        const double B2_AD = VC * DUDY;
+        const double Y_EX = (F2_EX - B2_EX) * COE2, Y_IM = (F2_IM - B2_IM) * COE2, Y_AD = (F2_AD - B2_AD) * COE2;
+        VP = MS2(0, 0, 1);
+        double DUDZ = (Q1(0, 0, 1) - Q1(0, 0, 0)) * g.dzi;
+        double DWDX = (Q3(0, 0, 1) - Q3(-1, 0, 1)) * g.dxi;
+        const double F3_EX = VP * DWDX, F3_IM = VP * DUDZ;
+        DUDZ = (Q1(0, 0, 1) * D1(0, 0, 1) - Q1(0, 0, 0) * D1(0, 0, 0)) * g.dzi;
+        const double F3_AD = VP * DUDZ;
+        VC = MS2(0, 0, 0);
+        DUDZ = (Q1(0, 0, 0) - Q1(0, 0, -1)) * g.dzi;
+        DWDX = (Q3(0, 0, 0) - Q3(-1, 0, 0)) * g.dxi;
+        const double B3_EX = VC * DWDX, B3_IM = VC * DUDZ;
+        DUDZ = (Q1(0, 0, 0) * D1(0, 0, 0) - Q1(0, 0, -1) * D1(0, 0, -1)) * g.dzi;
+        const double B3_AD = VC * DUDZ;
+        const double Z_EX = (F3_EX - B3_EX) * COE32, Z_IM = (F3_IM - B3_IM) * COE32, Z_AD = (F3_AD - B3_AD) * COE32;
+        hx = X_EX + Y_EX + Z_EX + hx;
+        IM1 = X_IM + Y_IM + Z_IM;
+        AD1 = X_AD + Y_AD + Z_AD;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    {   // y (rows 2..M)
+        const double COE1 = g.dxi * CV, COE3 = g.dzi * CV, COE2 = -2.0 / 3.0 * ldc(g.dyci, JJ - 1) * CV;
+        double DUDX = (Q1(1, 0, 0) - Q1(0, 0, 0)) * g.dxi;
+        double DVDY = (Q2(0, 1, 0) - Q2(0, 0, 0)) * ldc(g.dyfi, JJ - 1);
+        double DWDZ = (Q3(0, 0, 1) - Q3(0, 0, 0)) * g.dzi;
+        const double F_EX = MU(0, 0, 0) * (DUDX + DWDZ), F_IM = MU(0, 0, 0) * DVDY;
+        DVDY = (G2(0, 1, 0) * D2(0, 1, 0) - G2(0, 0, 0) * D2(0, 0, 0)) * ldc(g.dyfi, JJ - 1);
+        const double F_AD = MU(0, 0, 0) * DVDY;
+        DUDX = (Q1(1, -1, 0) - Q1(0, -1, 0)) * g.dxi;
+        DVDY = (Q2(0, 0, 0) - Q2(0, -1, 0)) * ldc(g.dyfi, JJM - 1);
+        DWDZ = (Q3(0, -1, 1) - Q3(0, -1, 0)) * g.dzi;
+        const double B_EX = MU(0, -1, 0) * (DUDX + DWDZ), B_IM = MU(0, -1, 0) * DVDY;
+        DVDY = (G2(0, 0, 0) * D2(0, 0, 0) - G2(0, -1, 0) * D2(0, -1, 0)) * ldc(g.dyfi, JJM - 1);
+        const double B_AD = MU(0, -1, 0) * DVDY;
+        const double Y_EX = (F_EX - B_EX) * COE2, Y_IM = (F_IM - B_IM) * COE2 * (-2.0);
+        const double Y_AD = (F_AD - B_AD) * COE2 * (-2.0);
+        double VP = MS1(1, 0, 0);
+        double DVDX = (Q2(1, 0, 0) - Q2(0, 0, 0)) * g.dxi;
+        double DUDY = (Q1(1, 0, 0) - Q1(1, -1, 0)) * ldc(g.dyci, JJ - 1);
+        const double F1_EX = VP * DUDY, F1_IM = VP * DVDX;
+        DVDX = (G2(1, 0, 0) * D2(1, 0, 0) - G2(0, 0, 0) * D2(0, 0, 0)) * g.dxi;
+        const double F1_AD = VP * DVDX;
+        double VC = MS1(0, 0, 0);
+        DVDX = (Q2(0, 0, 0) - Q2(-1, 0, 0)) * g.dxi;
+        DUDY = (Q1(0, 0, 0) - Q1(0, -1, 0)) * ldc(g.dyci, JJ - 1);
+        const double B1_EX = VC * DUDY, B1_IM = VC * DVDX;
+        DVDX = (G2(0, 0, 0) * D2(0, 0, 0) - G2(-1, 0, 0) * D2(-1, 0, 0)) * g.dxi;
+        const double B1_AD = VC * DVDX;
+        const double X_EX = (F1_EX - B1_EX) * COE1, X_IM = (F1_IM - B1_IM) * COE1, X_AD = (F1_AD - B1_AD) * COE1;
+        VP = MS3(0, 0, 1);
+        double DVDZ = (Q2(0, 0, 1) - Q2(0, 0, 0)) * g.dzi;
+        double DWDY = (Q3(0, 0, 1) - Q3(0, -1, 1)) * ldc(g.dyci, JJ - 1);
+        const double F3_EX = VP * DWDY, F3_IM = VP * DVDZ;
+        DVDZ = (G2(0, 0, 1) * D2(0, 0, 1) - G2(0, 0, 0) * D2(0, 0, 0)) * g.dzi;
+        const double F3_AD = VP * DVDZ;
+        VC = MS3(0, 0, 0);
+        DVDZ = (Q2(0, 0, 0) - Q2(0, 0, -1)) * g.dzi;
+        DWDY = (Q3(0, 0, 0) - Q3(0, -1, 0)) * ldc(g.dyci, JJ - 1);
+        const double B3_EX = VC * DWDY, B3_IM = VC * DVDZ;
+        DVDZ = (G2(0, 0, 0) * D2(0, 0, 0) - G2(0, 0, -1) * D2(0, 0, -1)) * g.dzi;
+        const double B3_AD = VC * DVDZ;
+        const double Z_EX = (F3_EX - B3_EX) * COE3, Z_IM = (F3_IM - B3_IM) * COE3, Z_AD = (F3_AD - B3_AD) * COE3;
+        hy = X_EX + Y_EX + Z_EX + hy;
+        IM2 = X_IM + Y_IM + Z_IM;
+        AD2 = X_AD + Y_AD + Z_AD;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    {   // z
+        const double COE1 = g.dxi * CV, COE3 = -2.0 / 3.0 * g.dzi * CV, COE2 = ldc(g.dyfi, JJ - 1) * CV;
+        double DUDX = (Q1(1, 0, 0) - Q1(0, 0, 0)) * g.dxi;
+        double DVDY = (Q2(0, 1, 0) - Q2(0, 0, 0)) * ldc(g.dyfi, JJ - 1);
+        double DWDZ = (Q3(0, 0, 1) - Q3(0, 0, 0)) * g.dzi;
+        const double F_EX = MU(0, 0, 0) * (DUDX + DVDY), F_IM = MU(0, 0, 0) * DWDZ;
+        DWDZ = (G3(0, 0, 1) * D3(0, 0, 1) - G3(0, 0, 0) * D3(0, 0, 0)) * g.dzi;
+        const double F_AD = MU(0, 0, 0) * DWDZ;
+        DUDX = (Q1(1, 0, -1) - Q1(0, 0, -1)) * g.dxi;
+        DVDY = (Q2(0, 1, -1) - Q2(0, 0, -1)) * ldc(g.dyfi, JJ - 1);
+        DWDZ = (Q3(0, 0, 0) - Q3(0, 0, -1)) * g.dzi;
+        const double B_EX = MU(0, 0, -1) * (DUDX + DVDY), B_IM = MU(0, 0, -1) * DWDZ;
+        DWDZ = (G3(0, 0, 0) * D3(0, 0, 0) - G3(0, 0, -1) * D3(0, 0, -1)) * g.dzi;
+        const double B_AD = MU(0, 0, -1) * DWDZ;
+        const double Z_EX = (F_EX - B_EX) * COE3, Z_IM = (F_IM - B_IM) * COE3 * (-2.0);
+        const double Z_AD = (F_AD - B_AD) * COE3 * (-2.0);
+        double VP = MS2(1, 0, 0);
+        double DWDX = (Q3(1, 0, 0) - Q3(0, 0, 0)) * g.dxi;
+        double DUDZ = (Q1(1, 0, 0) - Q1(1, 0, -1)) * g.dzi;
+        const double F1_EX = VP * DUDZ, F1_IM = VP * DWDX;
+        DWDX = (G3(1, 0, 0) * D3(1, 0, 0) - G3(0, 0, 0) * D3(0, 0, 0)) * g.dxi;
+        const double F1_AD = VP * DWDX;
+        double VC = MS2(0, 0, 0);
+        DWDX = (Q3(0, 0, 0) - Q3(-1, 0, 0)) * g.dxi;
+        DUDZ = (Q1(0, 0, 0) - Q1(0, 0, -1)) * g.dzi;
+        const double B1_EX = VC * DUDZ, B1_IM = VC * DWDX;
+        DWDX = (G3(0, 0, 0) * D3(0, 0, 0) - G3(-1, 0, 0) * D3(-1, 0, 0)) * g.dxi;
+        const double B1_AD = VC * DWDX;
+        const double X_EX = (F1_EX - B1_EX) * COE1, X_IM = (F1_IM - B1_IM) * COE1, X_AD = (F1_AD - B1_AD) * COE1;
+        VP = MS3(0, 1, 0);
+        double DWDY = (Q3(0, 1, 0) - Q3(0, 0, 0)) * ldc(g.dyci, JJP - 1);
+        double DVDZ = (Q2(0, 1, 0) - Q2(0, 1, -1)) * g.dzi;
+        const double F2_EX = VP * DVDZ, F2_IM = VP * DWDY;
+        DWDY = (G3(0, 1, 0) * D3(0, 1, 0) - G3(0, 0, 0) * D3(0, 0, 0)) * ldc(g.dyci, JJP - 1);
+        const double F2_AD = VP * DWDY;
+        VC = MS3(0, 0, 0);
+        DWDY = (Q3(0, 0, 0) - Q3(0, -1, 0)) * ldc(g.dyci, JJ - 1);
+        DVDZ = (Q2(0, 0, 0) - Q2(0, 0, -1)) * g.dzi;
+        const double B2_EX = VC * DVDZ, B2_IM = VC * DWDY;
+        DWDY = (G3(0, 0, 0) * D3(0, 0, 0) - G3(0, -1, 0) * D3(0, -1, 0)) * ldc(g.dyci, JJ - 1);
+        const double B2_AD = VC * DWDY;
+        const double Y_EX = (F2_EX - B2_EX) * COE2, Y_IM = (F2_IM - B2_IM) * COE2, Y_AD = (F2_AD - B2_AD) * COE2;
+        hz = X_EX + Y_EX + Z_EX + hz;
+        IM3 = X_IM + Y_IM + Z_IM;
+        AD3 = X_AD + Y_AD + Z_AD;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    double r1 = (tg * hx + tr * E1) * dt;
+    r1 = r1 + adt * IM1 + 0.5 * adt * AD1;
+    r1 = r1 - (PR(0, 0, 0) - PR(-1, 0, 0)) * (adt * g.dxi);
+    double r2 = (tg * hy + tr * E2) * dt;
+    r2 = r2 + adt * IM2 + 0.5 * adt * AD2;
+    r2 = r2 - (PR(0, 0, 0) - PR(0, -1, 0)) * (adt * ldc(g.dyci, JC - 1) / 1.0);
+    double r3 = (tg * hz + tr * E3) * dt;
+    r3 = r3 + adt * IM3 + 0.5 * adt * AD3;
+    r3 = r3 - (PR(0, 0, 0) - PR(0, 0, -1)) * (adt * g.dzi);
+    if (GRAV == 1) r1 = r1 + rsg * (adt * p.f_a / 1.0);
+    if (GRAV == 2) r2 = r2 + rsg * (adt * p.f_a / 1.0);
+    if (GRAV == 3) r3 = r3 + rsg * (adt * p.f_a / 1.0);
+    h[0] = hx;
+    h[1] = hy;
+    h[2] = hz;
+    r[0] = r1;
+    r[1] = r2;
+    r[2] = r3;
+    ad3 = AD3;
+}
+
+// One component of the LDS tile of k_io_terms_cn at a cell.
+constexpr int TCJ = 4, TCK = 2, TCX = 64 + 2, TCP = (TCJ + 2) * (TCK + 2) * TCX;
+struct CellTile {
+    const double* c;
+    __device__ __forceinline__ double operator()(int di, int dj, int dk) const {
+        return c[di + TCX * (dk + (TCK + 2) * dj)];
+    }
+};
+
+// io_terms_cn_cell on tiles of 64 i x TCJ j x TCK k, one thread per cell; G and
+// Q of the tile and its halo are staged in LDS, whose strides are constants.
+// inc <- RHS (row 1 of v zero), explt0 <- h, divu <- ad3 (what the reference
+// leaves in DIVU_io), part <- block sums.  Bound: the cells' reads through L2
+// (123 loads a cell without the tile, 11.8 TB/s of L2 traffic, 182 us at
+// 160x96x120 and 1082 at 256x192x256; 57 here, 157 and 902 us).  Two blocks to
+// a CU: the scheduling barriers between the three components' terms keep the
+// loads of one in flight at a time (128 registers; without them 174 and one
+// block, 171 and 967 us; forced to 128, spills, 276 and 1600 us).
+template <int GRAV>
+__global__ void __launch_bounds__(64 * TCJ * TCK, 4) k_io_terms_cn(
+    IoGeo g, const double* __restrict__ G, const double* __restrict__ Q, const double* __restrict__ MU,
+    const double* __restrict__ MS, const double* __restrict__ DR, const double* __restrict__ PR,
+    const double* __restrict__ RS, double* __restrict__ E, double* __restrict__ DUo, IoParams p, double tg, double tr,
+    double dt, double adt, double* __restrict__ inc, double* __restrict__ part) {
+#pragma clang fp contract(off)
+    extern __shared__ double tile[];   // [component][j][k][x]
     const int L = g.L, M = g.M, N = g.N;
-    int it, jt, kt, tile;
-    if (!row_tile(L, N, M, &it, &jt, &kt, &tile)) return;
-    const int IC = it * 64 + threadIdx.x;
-    const int KC = kt * 4 + threadIdx.y;
-    const int JC = jt + 1;
-    const bool live = IC < L && KC < N;
+    const int ni = (L + 63) / 64, nj = (M + TCJ - 1) / TCJ, nk = (N + TCK - 1) / TCK;
+    const int t = xcd_tile(blockIdx.x, gridDim.x);
+    if (t >= ni * nj * nk) return;
+    const int i0 = t % ni * 64, J0 = t / ni % nj * TCJ, k0 = t / (ni * nj) * TCK;   // J0: the tile's halo row
+    const int lane = threadIdx.x, ty = threadIdx.y;
+    const int LP = L * (M + 2), CS = LP * N, NC = L * M * N;
+    {
+        // rows of the tile: 24 of 64 columns (wrapped), then the two halo columns
+        constexpr int NR = (TCJ + 2) * (TCK + 2), NW = TCJ * TCK, NU = NR / NW;
+        static_assert(NR % NW == 0 && 2 * NR * 6 <= 64 * NW, "whole rows per wave; one halo value per thread");
+        auto row = [&](int r) {
+            int k = k0 - 1 + r % (TCK + 2);
+            k = k < 0 ? k + N : k;
+            return L * min(J0 + r / (TCK + 2), M + 1) + LP * (k >= N ? k % N : k);
+        };
+        double v[6][NU];
+#pragma unroll
+        for (int u = 0; u < NU; ++u) {
+            const int o = (i0 + lane) % L + row(ty + NW * u);
+#pragma unroll
+            for (int q = 0; q < 6; ++q) v[q][u] = q < 3 ? G[o + q * CS] : Q[o + (q - 3) * CS];
+        }
+        const int e = min(ty * 64 + lane, 12 * NR - 1), eq = e / (2 * NR), er = e % (2 * NR) >> 1, es = e & 1;
+        const int he = row(er) + (es ? (i0 + 64) % L : (i0 == 0 ? L : i0) - 1);
+        const double hv = eq < 3 ? G[he + eq * CS] : Q[he + (eq - 3) * CS];
+#pragma unroll
+        for (int u = 0; u < NU; ++u)
+#pragma unroll
+            for (int q = 0; q < 6; ++q) tile[q * TCP + (ty + NW * u) * TCX + 1 + lane] = v[q][u];
+        tile[eq * TCP + er * TCX + (es ? TCX - 1 : 0)] = hv;
+    }
+    __syncthreads();
+    const int kk = ty % TCK, jj = ty / TCK;
+    const int IC = i0 + lane, JC = J0 + 1 + jj, KC = k0 + kk;
     double flow = 0.0;
-    if (live) {
-        const int IP = IC == L - 1 ? 0 : IC + 1, IM = IC == 0 ? L - 1 : IC - 1;
-        const int KP = KC == N - 1 ? 0 : KC + 1, KM = KC == 0 ? N - 1 : KC - 1;
-        const int LP = L * (M + 2), CS = LP * N, NC = L * M * N;
-        auto at = [&](int i, int j, int k) { return i + L * j + LP * k; };
-        // row 1 of v is evaluated with a clamped metric index and discarded
-        const int JM = JC - 1, JP = JC + 1, JJ = JC, JJP = JC + 1, JJM = JC >= 2 ? JC - 1 : 1;
-        const double CV = g.cvisc;
-        const double *G1 = G, *G2 = G + CS, *G3 = G + 2 * CS;
-        const double *Q1 = Q, *Q2 = Q + CS, *Q3 = Q + 2 * CS;
-        const double *MS1 = MS, *MS2 = MS + CS, *MS3 = MS + 2 * CS;
-        const double *D1 = DR, *D2 = DR + CS, *D3 = DR + 2 * CS;
-        const int c = at(IC, JC, KC);
+    if (IC < L && JC <= M && KC < N) {
+        const int ip = IC == L - 1 ? 1 - L : 1, im = IC == 0 ? L - 1 : -1;
+        const int kp = KC == N - 1 ? (1 - N) * LP : LP, km = KC == 0 ? (N - 1) * LP : -LP;
+        const int c = IC + L * JC + LP * KC;
         const int e = IC + L * (JC - 1) + L * M * KC;
-        const double E1 = E[e], E2 = E[NC + e], E3 = E[2 * NC + e];
-        double hx, hy, hz;
-        io_conv(g, G, Q, IC, IP, IM, JC, KC, KP, KM, hx, hy, hz);
-        double IM1, AD1, IM2, AD2, IM3, AD3;
-        {   // x
-            const double COE1 = -2.0 / 3.0 * g.dxi * CV, COE2 = ldc(g.dyfi, JJ - 1) * CV * 1.0, COE32 = g.dzi * CV * 1.0;
-            const int cim = at(IM, JC, KC);
-            double DUDX = (Q1[at(IP, JC, KC)] - Q1[c]) * g.dxi;
-            double DVDY = (Q2[at(IC, JP, KC)] - Q2[c]) * ldc(g.dyfi, JJ - 1) * 1.0;
-            double DWDZ = (Q3[at(IC, JC, KP)] - Q3[c]) * g.dzi * 1.0;
-            const double F_EX = MU[c] * (DVDY + DWDZ), F_IM = MU[c] * DUDX;
-            DUDX = (G1[at(IP, JC, KC)] * D1[at(IP, JC, KC)] - G1[c] * D1[c]) * g.dxi;
-            const double F_AD = MU[c] * DUDX;
-            DUDX = (Q1[c] - Q1[cim]) * g.dxi;
-            DVDY = (Q2[at(IM, JP, KC)] - Q2[cim]) * ldc(g.dyfi, JJ - 1) * 1.0;
-            DWDZ = (Q3[at(IM, JC, KP)] - Q3[cim]) * g.dzi * 1.0;
-            const double B_EX = MU[cim] * (DVDY + DWDZ), B_IM = MU[cim] * DUDX;
-            DUDX = (G1[c] * D1[c] - G1[cim] * D1[cim]) * g.dxi;
-            const double B_AD = MU[cim] * DUDX;
-            const double X_EX = (F_EX - B_EX) * COE1, X_IM = (F_IM - B_IM) * COE1 * (-2.0);
-            const double X_AD = (F_AD - B_AD) * COE1 * (-2.0);
-            double VP = MS1[at(IC, JP, KC)];
-            double DVDX = (Q2[at(IC, JP, KC)] - Q2[at(IM, JP, KC)]) * g.dxi;
-            double DUDY = (Q1[at(IC, JP, KC)] - Q1[c]) * ldc(g.dyci, JJP - 1) / 1.0;
-            const double F2_EX = VP * DVDX, F2_IM = VP * DUDY;
-            DUDY = (G1[at(IC, JP, KC)] * D1[at(IC, JP, KC)] - G1[c] * D1[c]) * ldc(g.dyci, JJP - 1) / 1.0;
-            const double F2_AD = VP * DUDY;
-            double VC = MS1[c];
-            DUDY = (Q1[c] - Q1[at(IC, JM, KC)]) * ldc(g.dyci, JJ - 1) / 1.0;
-            DVDX = (Q2[c] - Q2[cim]) * g.dxi;
-            const double B2_EX = VC * DVDX, B2_IM = VC * DUDY;
-            DUDY = (G1[c] * D1[c] - G1[at(IC, JM, KC)] * D1[at(IC, JM, KC)]) * ldc(g.dyci, JJ - 1) / 1.0;
-            const double B2_AD = VC * DUDY;
-            const double Y_EX = (F2_EX - B2_EX) * COE2, Y_IM = (F2_IM - B2_IM) * COE2, Y_AD = (F2_AD - B2_AD) * COE2;
-            VP = MS2[at(IC, JC, KP)];
-            double DUDZ = (Q1[at(IC, JC, KP)] - Q1[c]) * g.dzi;
-            double DWDX = (Q3[at(IC, JC, KP)] - Q3[at(IM, JC, KP)]) * g.dxi;
-            const double F3_EX = VP * DWDX, F3_IM = VP * DUDZ;
-            DUDZ = (Q1[at(IC, JC, KP)] * D1[at(IC, JC, KP)] - Q1[c] * D1[c]) * g.dzi;
-            const double F3_AD = VP * DUDZ;
-            VC = MS2[c];
-            DUDZ = (Q1[c] - Q1[at(IC, JC, KM)]) * g.dzi;
-            DWDX = (Q3[c] - Q3[cim]) * g.dxi;
-            const double B3_EX = VC * DWDX, B3_IM = VC * DUDZ;
-            DUDZ = (Q1[c] * D1[c] - Q1[at(IC, JC, KM)] * D1[at(IC, JC, KM)]) * g.dzi;
-            const double B3_AD = VC * DUDZ;
-            const double Z_EX = (F3_EX - B3_EX) * COE32, Z_IM = (F3_IM - B3_IM) * COE32, Z_AD = (F3_AD - B3_AD) * COE32;
-            hx = X_EX + Y_EX + Z_EX + hx;
-            IM1 = X_IM + Y_IM + Z_IM;
-            AD1 = X_AD + Y_AD + Z_AD;
-        }
-        {   // y (rows 2..M)
-            const double COE1 = g.dxi * CV, COE3 = g.dzi * CV, COE2 = -2.0 / 3.0 * ldc(g.dyci, JJ - 1) * CV;
-            const int cjm = at(IC, JM, KC);
-            double DUDX = (Q1[at(IP, JC, KC)] - Q1[c]) * g.dxi;
-            double DVDY = (Q2[at(IC, JP, KC)] - Q2[c]) * ldc(g.dyfi, JJ - 1);
-            double DWDZ = (Q3[at(IC, JC, KP)] - Q3[c]) * g.dzi;
-            const double F_EX = MU[c] * (DUDX + DWDZ), F_IM = MU[c] * DVDY;
-            DVDY = (G2[at(IC, JP, KC)] * D2[at(IC, JP, KC)] - G2[c] * D2[c]) * ldc(g.dyfi, JJ - 1);
-            const double F_AD = MU[c] * DVDY;
-            DUDX = (Q1[at(IP, JM, KC)] - Q1[cjm]) * g.dxi;
-            DVDY = (Q2[c] - Q2[cjm]) * ldc(g.dyfi, JJM - 1);
-            DWDZ = (Q3[at(IC, JM, KP)] - Q3[cjm]) * g.dzi;
-            const double B_EX = MU[cjm] * (DUDX + DWDZ), B_IM = MU[cjm] * DVDY;
-            DVDY = (G2[c] * D2[c] - G2[cjm] * D2[cjm]) * ldc(g.dyfi, JJM - 1);
-            const double B_AD = MU[cjm] * DVDY;
-            const double Y_EX = (F_EX - B_EX) * COE2, Y_IM = (F_IM - B_IM) * COE2 * (-2.0);
-            const double Y_AD = (F_AD - B_AD) * COE2 * (-2.0);
-            double VP = MS1[at(IP, JC, KC)];
-            double DVDX = (Q2[at(IP, JC, KC)] - Q2[c]) * g.dxi;
-            double DUDY = (Q1[at(IP, JC, KC)] - Q1[at(IP, JM, KC)]) * ldc(g.dyci, JJ - 1);
-            const double F1_EX = VP * DUDY, F1_IM = VP * DVDX;
-            DVDX = (G2[at(IP, JC, KC)] * D2[at(IP, JC, KC)] - G2[c] * D2[c]) * g.dxi;
-            const double F1_AD = VP * DVDX;
-            double VC = MS1[c];
-            DVDX = (Q2[c] - Q2[at(IM, JC, KC)]) * g.dxi;
-            DUDY = (Q1[c] - Q1[cjm]) * ldc(g.dyci, JJ - 1);
-            const double B1_EX = VC * DUDY, B1_IM = VC * DVDX;
-            DVDX = (G2[c] * D2[c] - G2[at(IM, JC, KC)] * D2[at(IM, JC, KC)]) * g.dxi;
-            const double B1_AD = VC * DVDX;
-            const double X_EX = (F1_EX - B1_EX) * COE1, X_IM = (F1_IM - B1_IM) * COE1, X_AD = (F1_AD - B1_AD) * COE1;
-            VP = MS3[at(IC, JC, KP)];
-            double DVDZ = (Q2[at(IC, JC, KP)] - Q2[c]) * g.dzi;
-            double DWDY = (Q3[at(IC, JC, KP)] - Q3[at(IC, JM, KP)]) * ldc(g.dyci, JJ - 1);
-            const double F3_EX = VP * DWDY, F3_IM = VP * DVDZ;
-            DVDZ = (G2[at(IC, JC, KP)] * D2[at(IC, JC, KP)] - G2[c] * D2[c]) * g.dzi;
-            const double F3_AD = VP * DVDZ;
-            VC = MS3[c];
-            DVDZ = (Q2[c] - Q2[at(IC, JC, KM)]) * g.dzi;
-            DWDY = (Q3[c] - Q3[cjm]) * ldc(g.dyci, JJ - 1);
-            const double B3_EX = VC * DWDY, B3_IM = VC * DVDZ;
-            DVDZ = (G2[c] * D2[c] - G2[at(IC, JC, KM)] * D2[at(IC, JC, KM)]) * g.dzi;
-            const double B3_AD = VC * DVDZ;
-            const double Z_EX = (F3_EX - B3_EX) * COE3, Z_IM = (F3_IM - B3_IM) * COE3, Z_AD = (F3_AD - B3_AD) * COE3;
-            hy = X_EX + Y_EX + Z_EX + hy;
-            IM2 = X_IM + Y_IM + Z_IM;
-            AD2 = X_AD + Y_AD + Z_AD;
-        }
-        {   // z
-            const double COE1 = g.dxi * CV, COE3 = -2.0 / 3.0 * g.dzi * CV, COE2 = ldc(g.dyfi, JJ - 1) * CV;
-            const int ckm = at(IC, JC, KM);
-            double DUDX = (Q1[at(IP, JC, KC)] - Q1[c]) * g.dxi;
-            double DVDY = (Q2[at(IC, JP, KC)] - Q2[c]) * ldc(g.dyfi, JJ - 1);
-            double DWDZ = (Q3[at(IC, JC, KP)] - Q3[c]) * g.dzi;
-            const double F_EX = MU[c] * (DUDX + DVDY), F_IM = MU[c] * DWDZ;
-            DWDZ = (G3[at(IC, JC, KP)] * D3[at(IC, JC, KP)] - G3[c] * D3[c]) * g.dzi;
-            const double F_AD = MU[c] * DWDZ;
-            DUDX = (Q1[at(IP, JC, KM)] - Q1[ckm]) * g.dxi;
-            DVDY = (Q2[at(IC, JP, KM)] - Q2[ckm]) * ldc(g.dyfi, JJ - 1);
-            DWDZ = (Q3[c] - Q3[ckm]) * g.dzi;
-            const double B_EX = MU[ckm] * (DUDX + DVDY), B_IM = MU[ckm] * DWDZ;
-            DWDZ = (G3[c] * D3[c] - G3[ckm] * D3[ckm]) * g.dzi;
-            const double B_AD = MU[ckm] * DWDZ;
-            const double Z_EX = (F_EX - B_EX) * COE3, Z_IM = (F_IM - B_IM) * COE3 * (-2.0);
-            const double Z_AD = (F_AD - B_AD) * COE3 * (-2.0);
-            double VP = MS2[at(IP, JC, KC)];
-            double DWDX = (Q3[at(IP, JC, KC)] - Q3[c]) * g.dxi;
-            double DUDZ = (Q1[at(IP, JC, KC)] - Q1[at(IP, JC, KM)]) * g.dzi;
-            const double F1_EX = VP * DUDZ, F1_IM = VP * DWDX;
-            DWDX = (G3[at(IP, JC, KC)] * D3[at(IP, JC, KC)] - G3[c] * D3[c]) * g.dxi;
-            const double F1_AD = VP * DWDX;
-            double VC = MS2[c];
-            DWDX = (Q3[c] - Q3[at(IM, JC, KC)]) * g.dxi;
-            DUDZ = (Q1[c] - Q1[ckm]) * g.dzi;
-            const double B1_EX = VC * DUDZ, B1_IM = VC * DWDX;
-            DWDX = (G3[c] * D3[c] - G3[at(IM, JC, KC)] * D3[at(IM, JC, KC)]) * g.dxi;
-            const double B1_AD = VC * DWDX;
-            const double X_EX = (F1_EX - B1_EX) * COE1, X_IM = (F1_IM - B1_IM) * COE1, X_AD = (F1_AD - B1_AD) * COE1;
-            VP = MS3[at(IC, JP, KC)];
-            double DWDY = (Q3[at(IC, JP, KC)] - Q3[c]) * ldc(g.dyci, JJP - 1);
-            double DVDZ = (Q2[at(IC, JP, KC)] - Q2[at(IC, JP, KM)]) * g.dzi;
-            const double F2_EX = VP * DVDZ, F2_IM = VP * DWDY;
-            DWDY = (G3[at(IC, JP, KC)] * D3[at(IC, JP, KC)] - G3[c] * D3[c]) * ldc(g.dyci, JJP - 1);
-            const double F2_AD = VP * DWDY;
-            VC = MS3[c];
-            DWDY = (Q3[c] - Q3[at(IC, JM, KC)]) * ldc(g.dyci, JJ - 1);
-            DVDZ = (Q2[c] - Q2[ckm]) * g.dzi;
-            const double B2_EX = VC * DVDZ, B2_IM = VC * DWDY;
-            DWDY = (G3[c] * D3[c] - G3[at(IC, JM, KC)] * D3[at(IC, JM, KC)]) * ldc(g.dyci, JJ - 1);
-            const double B2_AD = VC * DWDY;
-            const double Y_EX = (F2_EX - B2_EX) * COE2, Y_IM = (F2_IM - B2_IM) * COE2, Y_AD = (F2_AD - B2_AD) * COE2;
-            hz = X_EX + Y_EX + Z_EX + hz;
-            IM3 = X_IM + Y_IM + Z_IM;
-            AD3 = X_AD + Y_AD + Z_AD;
-        }
-        double r1 = (tg * hx + tr * E1) * dt;
-        r1 = r1 + adt * IM1 + 0.5 * adt * AD1;
-        r1 = r1 - (PR[c] - PR[at(IM, JC, KC)]) * (adt * g.dxi);
-        double r2 = (tg * hy + tr * E2) * dt;
-        r2 = r2 + adt * IM2 + 0.5 * adt * AD2;
-        r2 = r2 - (PR[c] - PR[at(IC, JM, KC)]) * (adt * ldc(g.dyci, JC - 1) / 1.0);
-        double r3 = (tg * hz + tr * E3) * dt;
-        r3 = r3 + adt * IM3 + 0.5 * adt * AD3;
-        r3 = r3 - (PR[c] - PR[at(IC, JC, KM)]) * (adt * g.dzi);
-        if (GRAV == 1) r1 = r1 + RS[c] * (adt * p.f_a / 1.0);
-        if (GRAV == 2) r2 = r2 + RS[CS + c] * (adt * p.f_a / 1.0);
-        if (GRAV == 3) r3 = r3 + RS[2 * CS + c] * (adt * p.f_a / 1.0);
-        E[e] = hx;
-        E[2 * NC + e] = hz;
-        inc[e] = r1;
-        inc[2 * NC + e] = r3;
-        inc[NC + e] = JC >= 2 ? r2 : 0.0;
-        if (JC >= 2) E[NC + e] = hy;
-        DUo[c] = AD3;
-        const double rf = p.nflow == 1 ? r1 : (p.nflow == 2 ? (JC >= 2 ? r2 : 0.0) : r3);
+        auto A = [&](const double* b) { return cell_acc(b, c, ip, im, kp, km, L); };
+        const double* tc = tile + ((jj + 1) * (TCK + 2) + kk + 1) * TCX + 1 + lane;
+        auto T = [&](int q) { return CellTile{tc + q * TCP}; };
+        const double Ev[3] = {E[e], E[NC + e], E[2 * NC + e]};
+        const double rsg = GRAV == 0 ? 0.0 : RS[(GRAV - 1) * CS + c];
+        double h[3], r[3], ad3;
+        io_terms_cn_cell<GRAV>(g, T(0), T(1), T(2), T(3), T(4), T(5), A(MU), A(MS), A(MS + CS), A(MS + 2 * CS), A(DR),
+                               A(DR + CS), A(DR + 2 * CS), A(PR), JC, Ev, rsg, p, tg, tr, dt, adt, h, r, ad3);
+        E[e] = h[0];
+        E[2 * NC + e] = h[2];
+        inc[e] = r[0];
+        inc[2 * NC + e] = r[2];
+        inc[NC + e] = JC >= 2 ? r[1] : 0.0;
+        if (JC >= 2) E[NC + e] = h[1];
+        DUo[c] = ad3;
+        const double rf = p.nflow == 1 ? r[0] : (p.nflow == 2 ? (JC >= 2 ? r[1] : 0.0) : r[2]);
         flow = rf / ldc(g.dyfi, JC - 1) / 1.0;
     }
-    const double bs = io_block_sum<256>(flow, red);
-    if (threadIdx.x == 0 && threadIdx.y == 0) part[tile] = bs;
+    __syncthreads();   // the tile has been read
+    const double bs = io_block_sum<64 * TCJ * TCK>(flow, tile);
+    if (lane == 0 && ty == 0) part[t] = bs;
 }
 
 struct IoCnCoef {
@@ -1251,7 +1298,8 @@ struct IoCnCoef {
 // (j, k)), 2 = z (cyclic, lines (i, j)), 1 = y (non-cyclic, lines (i, k),
 // zero boundary values).  The x pass subtracts DPGRNS from the NFLOW
 // component (rows it applies to); the y pass adds the result to G from row
-// N2I and keeps the values it found as G0 (src/SOLVERRK3_MOM_IO.f90:15).
+// N2I, keeps the values it found as G0 (src/SOLVERRK3_MOM_IO.f90:15) and sets
+// the wall values of BC_WALL_G_io.
 // Bound: HBM, 32 B/cell and component (y: 48), in 128-byte pieces of 16 lines
 // and in the phases that small blocks overlap.  All components, one launch
 // and solve per component before: 160x96x120 x 125 -> 63, z 62 -> 44, y 128
@@ -1370,10 +1418,17 @@ __global__ void __launch_bounds__(512, DIR == 1 ? 4 : 1) k_io_cn(IoGeo g, int nf
             const int JC = seg * MS + l + 1;
             if (JC > n) continue;
             Gc0[L * JC] = go[l];
-            if (JC >= (idr == 2 ? 2 : 1)) Gc[L * JC] = d[l] + go[l];
+            Gc[L * JC] = idr == 2 && JC == 1 ? 0.0 : d[l] + go[l];
         }
-        if (seg == 0) Gc0[0] = Gc[0];   // the ghost rows, which no solve changes
-        if (seg == P - 1) Gc0[L * (M + 1)] = Gc[L * (M + 1)];
+        // BC_WALL_G_io: v on the bottom wall face (above) and the ghost rows are zero
+        if (seg == 0) {
+            Gc0[0] = Gc[0];
+            Gc[0] = 0.0;
+        }
+        if (seg == P - 1) {
+            Gc0[L * (M + 1)] = Gc[L * (M + 1)];
+            Gc[L * (M + 1)] = 0.0;
+        }
         return;
     }
 #pragma unroll
@@ -1626,12 +1681,18 @@ static int io_substep_cn(chs_handle* h, const chs_io_fields* f, const IoArrays& 
     const hipStream_t s = h->stream;
     const IoGeo g = io_geo(h);
     const dim3 gi = io_grid(h, h->M);
-    const long nb = io_tiles(h, h->M);
+    const int nb = ((h->L + 63) / 64) * ((h->M + TCJ - 1) / TCJ) * ((h->N + TCK - 1) / TCK);
+    constexpr size_t smt = sizeof(double) * 6 * TCP;
     hipEvent_t ev;
     h->timer.begin("io_terms_cn", s, &ev);
 #define IO_TERMS_CN(GR)                                                                                          \
-    CHS_LAUNCH(k_io_terms_cn<GR>, gi, dim3(64, 4), 0, s, g, a.g, a.q, a.mu, a.ms, f->drhoi_stg, a.pr, a.rs,      \
-               a.explt0, a.divu, p, TGAM_IO[ns], TROH_IO[ns], dt, talp * dt, h->rhs, h->partials)
+    do {                                                                                                         \
+        (void)hipFuncSetAttribute((const void*)k_io_terms_cn<GR>, hipFuncAttributeMaxDynamicSharedMemorySize,    \
+                                  (int)smt);                                                                     \
+        CHS_LAUNCH(k_io_terms_cn<GR>, dim3((unsigned)(8 * ((nb + 7) / 8))), dim3(64, TCJ * TCK), smt, s, g, a.g, \
+                   a.q, a.mu, a.ms, f->drhoi_stg, a.pr, a.rs, a.explt0, a.divu, p, TGAM_IO[ns], TROH_IO[ns], dt, \
+                   talp * dt, h->rhs, h->partials);                                                              \
+    } while (0)
     switch (p.gravdir) {
         case 1: IO_TERMS_CN(1); break;
         case 2: IO_TERMS_CN(2); break;
@@ -1640,7 +1701,7 @@ static int io_substep_cn(chs_handle* h, const chs_io_fields* f, const IoArrays& 
     }
 #undef IO_TERMS_CN
     h->timer.end(ev, "io_terms_cn", s);
-    CHS_LAUNCH(k_io_dpgrns, dim3(1), dim3(1024), 0, s, h->partials, (int)nb, h->volm, p.flowdrvtp,
+    CHS_LAUNCH(k_io_dpgrns, dim3(1), dim3(1024), 0, s, h->partials, nb, h->volm, p.flowdrvtp,
                -0.5 * p.cfgv * (talp * dt), h->scalars);
     // MOMFA_io: FACOE_io = alpha dt / (2 Re) (src/MOMFA_io.f90:29)
     const double FACOE = 0.5 * talp * dt * h->cvisc;
@@ -1650,7 +1711,6 @@ static int io_substep_cn(chs_handle* h, const chs_io_fields* f, const IoArrays& 
     CHS_TRY(io_cn_launch<0>(h, g, p.nflow, a, cx));
     CHS_TRY(io_cn_launch<2>(h, g, p.nflow, a, cz));
     CHS_TRY(io_cn_launch<1>(h, g, p.nflow, a, cy));
-    CHS_LAUNCH(k_io_massflux, io_grid(h, h->M + 2), dim3(64, 4), 0, s, g, a.g, nullptr, h->scalars, p.nflow);
     h->timer.begin("io_divg", s, &ev);
     CHS_LAUNCH(k_io_divg, gi, dim3(64, 4), 0, s, g, a.g, nullptr, a.drhodtp, 1.0 / dt / talp, h->rhsllphi);
     h->timer.end(ev, "io_divg", s);
