@@ -40,10 +40,12 @@ def alg_bytes_per_cell(L, precision="fp64"):
                 "fft_x_inv": sp32 + 8,     # read S; write phi1 (FP32) / read phi1, write phi: 4 and 12, averaged
                 "poisson_residual": 24.0,
                 "rhs_x": 68.0,             # read Q x3, PR, CONVH0 x3 (FP32); write RHS x3, CONVH0 x3 (FP32)
-                "z_solve": 24.0, "y_solve": 60.0, "divg": 32.0, "update": 80.0}
+                "z_solve": 24.0, "y_solve": 60.0, "divg": 32.0, "update": 80.0,
+                "zy_solve": 60.0}          # read RHS x3 (FP32), Q x3; write Q x3
     return {"rhs_x": 104.0,          # read Q x3, PR, CONVH0 x3; write RHS x3, CONVH0 x3
             "z_solve": 48.0,         # read/write RHS x3
             "y_solve": 72.0,         # read RHS x3, Q x3; write Q x3
+            "zy_solve": 72.0,        # read RHS x3, Q x3; write Q x3 (both solves in one pass)
             "divg": 32.0,            # read Q x3; write f
             "fft_x_fwd": 8 + sp,     # read f; write S
             "fft_z": 2 * sp,         # read/write S
@@ -337,7 +339,7 @@ def props_bench(g, q_fp64, stream, steps):
     ts.params.visimplicit = 0
     # algorithmic bytes per cell of the explicit branch with NFLOW = 1: the
     # terms kernel also writes G0 and G + RHS (no separate copy or mass-flux pass)
-    ab = {"io_prepare": 160.0, "io_divu": 32.0, "io_terms": 200.0, "io_massflux": 72.0, "io_divg": 40.0,
+    ab = {"io_prepare": 160.0, "io_terms": 200.0, "io_massflux": 72.0, "io_divg": 40.0,
           "io_update": 72.0}
     kern = {}
     for name, (ms_tot, calls) in prof.items():

@@ -130,9 +130,10 @@ class ChannelSolver:
 
     def set_cn_solver(self, mode: str):
         """'auto' (truncated-inverse stencils where their bound holds; the
-        y-marching RHS kernels where their chunks have 8 rows or more),
-        'thomas', 'rowtile' ('auto' with the per-row RHS kernels only) or
-        'marching' ('auto' with the y-marching RHS kernels wherever they fit)."""
+        y-marching RHS kernels where their chunks have 8 rows or more, the z
+        and y solves in one pass where its blocks have 20 rows), 'thomas',
+        'rowtile' ('auto' with the per-row RHS kernels only) or 'marching'
+        ('auto' with those kernels and the one pass wherever they fit)."""
         nat.check(self.lib.chs_set_cn_solver(self.h, {"auto": 0, "thomas": 1, "rowtile": 2, "marching": 3}[mode]))
 
     def cn_info(self, ns: int, dt: float):

@@ -120,9 +120,10 @@ int chs_poisson_stats(chs_handle *h, int *iters, double *rel_resid);
  * on the host in extended precision); otherwise, and always with mode 1, as
  * segmented Thomas solves.  Mode 0 evaluates the right-hand sides (here, in
  * chs_solverrk3_mom_io and chs_energy_substep) marching along y where each
- * block's chunk has at least 8 rows, one y row per block otherwise (small
- * grids); mode 2 always one row per block, mode 3 always marching where the
- * marching kernels fit (same results to rounding). */
+ * block's chunk has at least 8 rows (12 beyond NCL1 = 256), one y row per block
+ * otherwise (small grids), and the z and y solves in one pass where its blocks
+ * have at least 20 rows; mode 2 always one row per block, mode 3 always marching
+ * and one pass where those kernels fit (same results to rounding). */
 int chs_set_cn_solver(chs_handle *h, int mode);
 /* Which path substep NS with time step dt takes (1 = stencils, 0 = Thomas)
  * and the stencil half-widths in x, z, y (> 16 when too wide). */
@@ -177,11 +178,11 @@ int chs_tdma_batched(const double *a_dev, const double *b_dev, const double *c_d
 
 /* chs_tdma_batched without any device allocation, for callers that cannot
  * allocate (code under HIP graph capture, tight serving loops, harnesses that
- * forbid hipMalloc).  No counterpart in the reference.  Lines the segmented
- * kernel splits need no workspace; the others (e.g. cyclic lines of odd
- * length, or more than 512 rows) take 3*n*nlines doubles from a static array
- * of 4194304 doubles (32 MiB) that each GPU holds until the process ends, and
- * larger such calls return CHS_E_ARG.  Calls that overlap on one GPU share that
+ * forbid hipMalloc).  No counterpart in the reference.  Non-cyclic lines of up
+ * to 512 rows and cyclic ones of a multiple of 4 rows need no workspace; calls
+ * with other lines are held to 3*n*nlines <= 4194304 doubles, those of a static
+ * array (32 MiB) that each GPU holds until the process ends and that the
+ * longest of them use (a few thousand rows); larger such calls return CHS_E_ARG.  Calls that overlap on one GPU share that
  * array and race; its contents are not cleared between calls (nothing in it
  * is read before it is written).  Same arguments and results as
  * chs_tdma_batched. */
