@@ -1598,10 +1598,11 @@ int io_prepare(chs_handle* h, const chs_thermal_fields* tf, const chs_io_fields*
     const double ca = TGAM_IO[ns] + TROH_IO[ns], cb = TROH_IO[ns], cd = TGAM_IO[ns] - 2.0;
     const IoGeo g = io_geo(h);
     const long ncol = (long)((h->L + 63) / 64) * ((h->N + 3) / 4);
-    // on grids of fewer than 4096 row tiles (64^3: 1056) the row tiles are
-    // faster (13.3 against 20.4 us with the march and its edge rows apart); at
-    // 128^3 (8320) the march wins (86 against 101 us)
-    if (prm->thermal && h->M >= 3 && h->cn_mode != 2 && (h->cn_mode == 3 || ncol * (h->M + 2) >= 4096)) {
+    // on grids of fewer than 1000 row tiles the row-tile form is as fast (a
+    // heated step at 48^3, 600 tiles, 271 us against 274); at 64^3 (1056) the
+    // march wins (298 against 304 us), at 96x64x64 (2112) 377 against 386, at
+    // 128^3 (8320) the kernels take 86 against 101 us
+    if (prm->thermal && h->M >= 3 && h->cn_mode != 2 && (h->cn_mode == 3 || ncol * (h->M + 2) >= 1000)) {
         // rows 2..M marching (about 8 blocks per CU), rows 0, 1 and M+1 a cell per thread
         int nyc = (int)std::max(1L, std::min((long)(h->M - 1) / 4, (2048 + ncol - 1) / ncol));
         const int jc = (h->M - 1 + nyc - 1) / nyc;
