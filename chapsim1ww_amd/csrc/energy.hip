@@ -253,25 +253,23 @@ __global__ void __launch_bounds__(1024) k_energy_rhs_m(EGeo g, EFields f, double
 // gives NaN (as the reference's evaluators do).
 // S_HT (hack: ENTHALPY_UPDATE's |h| < 1e-10 gives T = 1)
 template <int KW, bool WIDE>
-__device__ __forceinline__ double ht_nb(const PropTab& t, const LdsTab<WIDE>& l, double hv, bool hack, bool& ok) {
+__device__ __forceinline__ double ht_nb(const PropTab& t, const LdsTab<WIDE>& l, double hv, bool hack, bool& ok,
+                                        int& i) {
     const bool nan = hv != hv, in = hv > t.h_lo && hv < t.h_hi;
     ok = nan || in;
     const double hq = in ? hv : t.h_lo;
-    const int i = find_iv<KW>(l.xh, l.sh, t.n, t.nbh, t.h_lo, t.hbi, hq);
+    i = find_iv<KW>(l.xh, l.sh, t.n, t.nbh, t.h_lo, t.hbi, hq);
     const double4 r = l.ht(t, i);
     double T = cubic_nc(r.x, r.y, r.z, r.w, hq - l.xh[i]);
     if (hack && fabs(hv) < 1.0e-10) T = 1.0;
     return nan ? hv : T;
 }
 
-// the interval of T (clamped) and its record's first double4 (S_TD) or all
-// four (S_TD, S_TM, S_TK, S_TCp)
-template <int KW, bool WIDE>
-__device__ __forceinline__ int t_iv_nb(const PropTab& t, const LdsTab<WIDE>& l, double tv, bool& ok, double& tq) {
+// T clamped into the table for its interval search
+__device__ __forceinline__ double t_nb(const PropTab& t, double tv, bool& ok) {
     const bool nan = tv != tv, in = tv > t.t_lo && tv < t.t_hi;
     ok = nan || in;
-    tq = in ? tv : t.t_lo;
-    return find_iv<KW>(l.xt, l.st, t.n, t.nbt, t.t_lo, t.tbi, tq);
+    return in ? tv : t.t_lo;
 }
 
 // rotations of the property history on every cell, the property cascade on
@@ -279,7 +277,10 @@ __device__ __forceinline__ int t_iv_nb(const PropTab& t, const LdsTab<WIDE>& l, 
 // THERM_PROP_UPDATE, src/THERM_PROP_UPDATE.f90); persistent blocks, ECELL
 // cells per thread and pass with every load issued first and the lookup
 // chains of the cells side by side (the same arithmetic per cell as the
-// one-cell form, so the outputs are unchanged bit for bit).
+// one-cell form, so the outputs are unchanged bit for bit).  The T intervals
+// come from H's (t_intervals) and the M and K records by quads (quad_mk), which
+// the property lookup alone gains most from (238 -> 177 us at 12.6 M cells); here
+// the cells of a wave lie close in the table: 270 -> 256 us at 256x192x256.
 // second = 0: the final THERM_PROP_UPDATE lookup is left to the learned
 // surrogate (chs_props_set_mode), which runs after this kernel on h
 template <int KW, bool WIDE, int EPT, int ECELL>
@@ -303,7 +304,8 @@ __global__ void __launch_bounds__(EPT) k_energy_props(PropTab t, EGeo g, EFields
     const bool few = ntot <= 8 * RC * nb;
     const int per = few ? ((ntot + nb - 1) / nb + 63) & ~63 : RC, step = few ? RC : nb * RC;
     const int end = few ? min(ntot, ((int)blockIdx.x + 1) * per) : ntot;
-    for (int q0 = blockIdx.x * per + threadIdx.x; q0 < end; q0 += step) {
+    const int lane = threadIdx.x & 63;
+    for (int q0 = blockIdx.x * per + threadIdx.x; q0 - lane < end; q0 += step) {   // whole waves (quad_mk)
         int q[ECELL];
         bool live[ECELL], inner[ECELL];
         double mu_old[ECELL], rho_old[ECELL], rho0_old[ECELL], rh[ECELL];
@@ -311,7 +313,7 @@ __global__ void __launch_bounds__(EPT) k_energy_props(PropTab t, EGeo g, EFields
         for (int u = 0; u < ECELL; ++u) {
             const int qq = q0 + u * EPT;
             live[u] = qq < end;
-            q[u] = live[u] ? qq : q0;
+            q[u] = live[u] ? qq : q0 - lane;
             const int j = (q[u] / L) % (M + 2);
             inner[u] = live[u] && j != 0 && j != M + 1;
             mu_old[u] = f.mu[q[u]];
@@ -330,20 +332,19 @@ __global__ void __launch_bounds__(EPT) k_energy_props(PropTab t, EGeo g, EFields
         double D1[ECELL];
         bool ok1[ECELL];
         {
-            double T1[ECELL];
-            bool okh[ECELL];
-#pragma unroll
-            for (int u = 0; u < ECELL; ++u) T1[u] = ht_nb<KW>(t, l, rh[u] / rho_old[u], true, okh[u]);
-            int k1[ECELL];
-            double tq[ECELL];
+            double T1[ECELL], tq[ECELL];
+            int i1[ECELL], k1[ECELL];
             double4 cd[ECELL];
 #pragma unroll
             for (int u = 0; u < ECELL; ++u) {
-                bool okt;
-                k1[u] = t_iv_nb<KW>(t, l, T1[u], okt, tq[u]);
-                ok1[u] = okh[u] && okt;
-                cd[u] = l.td(t, k1[u]);
+                bool okh, okt;
+                T1[u] = ht_nb<KW>(t, l, rh[u] / rho_old[u], true, okh, i1[u]);
+                tq[u] = t_nb(t, T1[u], okt);
+                ok1[u] = okh && okt;
             }
+            t_intervals<KW>(t, xt, l.st, i1, tq, k1);
+#pragma unroll
+            for (int u = 0; u < ECELL; ++u) cd[u] = l.td(t, k1[u]);
 #pragma unroll
             for (int u = 0; u < ECELL; ++u) {
                 double D = cubic_nc(cd[u].x, cd[u].y, cd[u].z, cd[u].w, tq[u] - xt[k1[u]]);
@@ -354,15 +355,22 @@ __global__ void __launch_bounds__(EPT) k_energy_props(PropTab t, EGeo g, EFields
         // ENTHALPY_UPDATE with the new density, then THERM_PROP_UPDATE
         double h2[ECELL], T2[ECELL];
         bool ok2[ECELL];
-        int k2[ECELL];
+        int i2[ECELL], k2[ECELL];
         double tq2[ECELL];
 #pragma unroll
         for (int u = 0; u < ECELL; ++u) {
             h2[u] = rh[u] / D1[u];
             bool okh, okt;
-            T2[u] = ht_nb<KW>(t, l, h2[u], false, okh);
-            k2[u] = t_iv_nb<KW>(t, l, T2[u], okt, tq2[u]);
+            T2[u] = ht_nb<KW>(t, l, h2[u], false, okh, i2[u]);
+            tq2[u] = t_nb(t, T2[u], okt);
             ok2[u] = okh && okt;
+        }
+        t_intervals<KW>(t, xt, l.st, i2, tq2, k2);
+        double4 cd2[ECELL], cm2[ECELL], ck2[ECELL];
+#pragma unroll
+        for (int u = 0; u < ECELL; ++u) {
+            cd2[u] = l.td(t, k2[u]);
+            quad_mk(t.rt, k2[u], cm2[u], ck2[u]);
         }
 #pragma unroll
         for (int u = 0; u < ECELL; ++u) {
@@ -384,8 +392,7 @@ __global__ void __launch_bounds__(EPT) k_energy_props(PropTab t, EGeo g, EFields
                 f.rho[q[u]] = D1[u];
                 continue;
             }
-            const double4* r4 = reinterpret_cast<const double4*>(t.rt) + 4 * (size_t)k2[u];
-            const double4 cd = l.td(t, k2[u]), cm = r4[1], ck = r4[2];
+            const double4 cd = cd2[u], cm = cm2[u], ck = ck2[u];
             const double dt = tq2[u] - xt[k2[u]];
             double D = cubic_nc(cd.x, cd.y, cd.z, cd.w, dt);
             double Mu = cubic_nc(cm.x, cm.y, cm.z, cm.w, dt);

@@ -81,8 +81,12 @@ int props_counts_out(unsigned long long* c, unsigned long long* host, hipStream_
 }
 
 // PT threads, PCELL cells per thread and chunk of persistent blocks.  WIDE
-// (LdsTab): bound by the LDS reads of the searches and records and by the
-// gathers of the M, K and CP records; 12.6 M cells 290 -> 267 us a call.
+// (LdsTab): HBM (48 B a cell, 121 us of 12.6 M cells at 5.0 TB/s, 20 more with
+// cp), the LDS reads of the search and the records, and the gathers of the M,
+// K and CP records between them.  12.6 M cells a call: 290 us with all records
+// from L2, 253 with two of them in LDS, 214 (177 without cp, from 238) with
+// the others gathered by quads and pairs of lanes (quad_mk) and the T interval
+// taken from H's (t_intervals).
 template <int KW, bool WIDE, int PT, int PCELL>
 __global__ void __launch_bounds__(PT) k_props_table(PropTab t, Rows rw, const double* __restrict__ h,
                                                     double* __restrict__ To, double* __restrict__ rho,
@@ -92,7 +96,6 @@ __global__ void __launch_bounds__(PT) k_props_table(PropTab t, Rows rw, const do
     extern __shared__ unsigned char smem[];
     const LdsTab<WIDE> l = stage_tab<WIDE>(t, smem);
     const double *xh = l.xh, *xt = l.xt;
-    constexpr int TC = PCELL < 2 ? 1 : 2;   // cells whose T records are in flight together
     const long long chunk = (long long)PT * PCELL;
     const long long cpr = (rw.rowlen + chunk - 1) / chunk;   // chunks per row
     const long long nch = cpr * rw.nrow;
@@ -130,52 +133,46 @@ __global__ void __launch_bounds__(PT) k_props_table(PropTab t, Rows rw, const do
             okh[u] = nan || (hv[u] > t.h_lo && hv[u] < t.h_hi);
             tv[u] = nan ? hv[u] : cubic_nc(rr[u].x, rr[u].y, rr[u].z, rr[u].w, hv[u] - xh[ih[u]]);
         }
-        // S_TD/TM/TK/TCp two cells at a time: both cells' T records are
-        // loaded before either is evaluated
+        // S_TD/TM/TK/TCp a cell at a time (two in flight spill at 128 VGPRs,
+        // and four cells a thread with two in flight took 234 against 214 us)
 #pragma unroll
-        for (int u0 = 0; u0 < PCELL; u0 += TC) {
-            int kt[TC];
-            double4 rq[TC][4];
-#pragma unroll
-            for (int v = 0; v < TC; ++v) {
-                const double tq = tv[u0 + v] > t.t_lo && tv[u0 + v] < t.t_hi ? tv[u0 + v] : t.t_lo;
-                kt[v] = find_iv<KW>(xt, l.st, t.n, t.nbt, t.t_lo, t.tbi, tq);
-                const double4* q = reinterpret_cast<const double4*>(t.rt) + 4 * (size_t)kt[v];
-                rq[v][0] = l.td(t, kt[v]);
-                rq[v][1] = q[1];
-                rq[v][2] = q[2];
-                rq[v][3] = cp ? q[3] : q[2];
+        for (int u = 0; u < PCELL; ++u) {
+            __builtin_amdgcn_sched_barrier(0);   // (218 us without)
+            const double T = tv[u];
+            const int it[1] = {ih[u]};
+            const double tq[1] = {T > t.t_lo && T < t.t_hi ? T : t.t_lo};
+            int kt[1];
+            t_intervals<KW>(t, xt, l.st, it, tq, kt);
+            // every lane loads; those without a value hold a clamped interval
+            const double4 rd = l.td(t, kt[0]);
+            double4 rm, rk;
+            quad_mk(t.rt, kt[0], rm, rk);
+            const double4 rc = cp ? pair_cp(t.rt, kt[0]) : rk;
+            // THERM_PROP_UPDATE leaves |h| < 1e-10 (and cells past the row) as they are
+            if (!in[u] || fabs(hv[u]) < 1.0e-10) continue;
+            ++looked;
+            const bool nan = T != T;
+            if (!okh[u] || (!nan && (T <= t.t_lo || T >= t.t_hi))) {
+                ++bad;
+                continue;
             }
-#pragma unroll
-            for (int v = 0; v < TC; ++v) {
-                const int u = u0 + v;
-                // THERM_PROP_UPDATE leaves |h| < 1e-10 (and cells past the row) as they are
-                if (!in[u] || fabs(hv[u]) < 1.0e-10) continue;
-                ++looked;
-                const double T = tv[u];
-                const bool nan = T != T;
-                if (!okh[u] || (!nan && (T <= t.t_lo || T >= t.t_hi))) {
-                    ++bad;
-                    continue;
-                }
-                double D, Mu, K, CP;
-                if (nan) {
-                    D = Mu = K = CP = T;
-                } else {
-                    const double dt = T - xt[kt[v]];
-                    D = cubic_nc(rq[v][0].x, rq[v][0].y, rq[v][0].z, rq[v][0].w, dt);
-                    Mu = cubic_nc(rq[v][1].x, rq[v][1].y, rq[v][1].z, rq[v][1].w, dt);
-                    K = cubic_nc(rq[v][2].x, rq[v][2].y, rq[v][2].z, rq[v][2].w, dt);
-                    CP = cubic_nc(rq[v][3].x, rq[v][3].y, rq[v][3].z, rq[v][3].w, dt);
-                    if (fabs(T - 1.0) < 1.0e-10) D = Mu = K = CP = 1.0;
-                }
-                const long long q = base + c0 + u * PT + threadIdx.x;
-                To[q] = T;
-                mu[q] = Mu;
-                kap[q] = K;
-                rho[q] = D;
-                if (cp) cp[q] = CP;
+            double D, Mu, K, CP;
+            if (nan) {
+                D = Mu = K = CP = T;
+            } else {
+                const double dt = T - xt[kt[0]];
+                D = cubic_nc(rd.x, rd.y, rd.z, rd.w, dt);
+                Mu = cubic_nc(rm.x, rm.y, rm.z, rm.w, dt);
+                K = cubic_nc(rk.x, rk.y, rk.z, rk.w, dt);
+                CP = cubic_nc(rc.x, rc.y, rc.z, rc.w, dt);
+                if (fabs(T - 1.0) < 1.0e-10) D = Mu = K = CP = 1.0;
             }
+            const long long q = base + c0 + u * PT + threadIdx.x;
+            To[q] = T;
+            mu[q] = Mu;
+            kap[q] = K;
+            rho[q] = D;
+            if (cp) cp[q] = CP;
         }
     }
     // out-of-range count (and, on request, the lookups): one atomic per wave
@@ -189,10 +186,15 @@ __global__ void __launch_bounds__(PT) k_props_table(PropTab t, Rows rw, const do
     }
 }
 
-// Calls of fewer cells than a chunk of 8 per thread of 1024 would spread over
-// the CUs run one cell per thread: 4,096 cells 53 -> 33 us a call, 262,144
-// 65 -> 39, 1,048,576 69 -> 59; 2,097,152 70 against 78 (with the same host path)
-constexpr long long PSMALL = 3ll << 19;
+// Forms by the cells of a call.  Few cells: one per thread in blocks of 256,
+// whose staging is short and which fill the CUs (262,144 cells 25 against 29
+// us with 2 cells in blocks of 1024, 524,288 28 against 30, 1,048,576 36.4
+// against 35.4).  Up to some six rounds of the grid: 2 cells per thread, which
+// leave less of the last round empty than 8 (2,097,152 cells 45.0 against 46.5,
+// 3,000,000 54 against 63, 4,200,000 67 against 80); more: 8, with more loads in
+// flight (6,300,000 128 with 2 against 125, 9,000,000 189 against 174).  Tables
+// too large for the wide form: one cell below PSMALL_N, 8 from there.
+constexpr long long PSMALL = 1ll << 20, PMID = 3ll << 21, PSMALL_N = 3ll << 19;
 
 int props_table_launch(chs_props* p, const double* h, Rows rw, double* T, double* rho, double* mu, double* kap,
                        double* cp, unsigned long long* cnt, int count_lookups, hipStream_t stream) {
@@ -212,8 +214,10 @@ int props_table_launch(chs_props* p, const double* h, Rows rw, double* T, double
     } while (0)
 #define CHS_PROPS_K(KK)                                                                                          \
     do {                                                                                                         \
-        if (cells < PSMALL)                                                                                      \
+        if (cells < (wide ? PSMALL : PSMALL_N))                                                                  \
             CHS_PROPS_L(KK, false, 256, 1);                                                                      \
+        else if (wide && cells < PMID)                                                                           \
+            CHS_PROPS_L(KK, true, 1024, 2);                                                                      \
         else if (wide)                                                                                           \
             CHS_PROPS_L(KK, true, 1024, 8);                                                                      \
         else                                                                                                     \

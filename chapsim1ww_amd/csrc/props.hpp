@@ -266,6 +266,75 @@ __device__ __forceinline__ LdsTab<WIDE> stage_tab(const PropTab& t, unsigned cha
     return LdsTab<WIDE>{a, b, hb, ty, tb, c, d};
 }
 
+// The T intervals k of N cells whose T came out of the H intervals i.  The T
+// knots are the H -> T spline's values at the H knots, so k = i unless the
+// spline overshoots or rounds past a knot, or T was set: the search is left to
+// those cells, in one branch for all N so that their chains still interleave.
+template <int KW, int N, class Ix>
+__device__ __forceinline__ void t_intervals(const PropTab& t, const double* xt, const Ix* st, const int (&i)[N],
+                                            const double (&tq)[N], int (&k)[N]) {
+    bool miss = false;
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+        k[u] = i[u];
+        miss |= !(xt[i[u]] <= tq[u] && tq[u] < xt[i[u] + 1]);
+    }
+    if (miss) {
+#pragma unroll
+        for (int u = 0; u < N; ++u) k[u] = find_iv<KW>(xt, st, t.n, t.nbt, t.t_lo, t.tbi, tq[u]);
+    }
+}
+
+// A DPP move of a double2 (CTRL: quad_perm)
+template <int CTRL>
+__device__ __forceinline__ int dpp_i(int v) {
+    return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
+}
+template <int CTRL>
+__device__ __forceinline__ double2 dpp_d2(double2 v) {
+    const double x = __hiloint2double(dpp_i<CTRL>(__double2hiint(v.x)), dpp_i<CTRL>(__double2loint(v.x)));
+    const double y = __hiloint2double(dpp_i<CTRL>(__double2hiint(v.y)), dpp_i<CTRL>(__double2loint(v.y)));
+    return make_double2(x, y);
+}
+
+// One step of a transpose between lanes l and l ^ 1 (CTRL 0xB1) or l ^ 2
+// (0x4E): the lane with the bit set gives a and takes the other's b for it,
+// the other gives b.
+template <int CTRL>
+__device__ __forceinline__ void lane_swap(bool bit, double2& a, double2& b) {
+    const double2 send = make_double2(bit ? a.x : b.x, bit ? a.y : b.y), got = dpp_d2<CTRL>(send);
+    a = make_double2(bit ? got.x : a.x, bit ? got.y : a.y);
+    b = make_double2(bit ? b.x : got.x, bit ? b.y : got.y);
+}
+
+// The records of interval k from global memory, by the lanes of a quad
+// together (every lane of the wave takes part): a lane's own 16-byte loads
+// touch 64 cache lines an instruction, one line a cycle, while four lanes that
+// load the four 16-byte pieces of one cell's M and K records touch 16.  The
+// pieces then change lanes (DPP).  D and CP by quads as well: 212 us a call of
+// k_props_table with cp, 189 without, against 214 and 177.
+__device__ __forceinline__ void quad_mk(const double* rt, int k, double4& cm, double4& ck) {
+    const int p = threadIdx.x & 3;
+    const int k0 = dpp_i<0x00>(k), k1 = dpp_i<0x55>(k), k2 = dpp_i<0xAA>(k), k3 = dpp_i<0xFF>(k);
+    const double2* b = reinterpret_cast<const double2*>(rt) + 2 + p;   // 8 double2 a record of four; M and K: 2 to 5
+    double2 v0 = b[8 * (size_t)k0], v1 = b[8 * (size_t)k1], v2 = b[8 * (size_t)k2], v3 = b[8 * (size_t)k3];
+    lane_swap<0xB1>(p & 1, v0, v1);
+    lane_swap<0xB1>(p & 1, v2, v3);
+    lane_swap<0x4E>(p & 2, v0, v2);
+    lane_swap<0x4E>(p & 2, v1, v3);
+    cm = make_double4(v0.x, v0.y, v1.x, v1.y);
+    ck = make_double4(v2.x, v2.y, v3.x, v3.y);
+}
+// the CP record, by pairs of lanes
+__device__ __forceinline__ double4 pair_cp(const double* rt, int k) {
+    const int p = threadIdx.x & 1;
+    const int k0 = dpp_i<0xA0>(k), k1 = dpp_i<0xF5>(k);   // of the pair's even and odd lane
+    const double2* b = reinterpret_cast<const double2*>(rt) + 6 + p;
+    double2 v0 = b[8 * (size_t)k0], v1 = b[8 * (size_t)k1];
+    lane_swap<0xB1>(p, v0, v1);
+    return make_double4(v0.x, v0.y, v1.x, v1.y);
+}
+
 // S_HT (NIST_SLEVAL_HT, src/Flow_State.f90:1015-1070): false when h leaves
 // the table (the reference STOPs); hack: |h| < 1e-10 gives T = 1.  A NaN
 // passes the range tests and gives NaN, as there.
