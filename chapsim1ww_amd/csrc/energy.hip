@@ -280,7 +280,9 @@ __device__ __forceinline__ double t_nb(const PropTab& t, double tv, bool& ok) {
 // one-cell form, so the outputs are unchanged bit for bit).  The T intervals
 // come from H's (t_intervals) and the M and K records by quads (quad_mk), which
 // the property lookup alone gains most from (238 -> 177 us at 12.6 M cells); here
-// the cells of a wave lie close in the table: 270 -> 256 us at 256x192x256.
+// the cells of a wave lie closer in the table: 270 -> 256 us at 256x192x256 on
+// a fluctuating field (a time step at 128^3 1342 -> 1334 us), 239 -> 245 on a
+// smooth one, whose lanes share records.
 // second = 0: the final THERM_PROP_UPDATE lookup is left to the learned
 // surrogate (chs_props_set_mode), which runs after this kernel on h
 template <int KW, bool WIDE, int EPT, int ECELL>
