@@ -368,11 +368,13 @@ __global__ void __launch_bounds__(EPT) k_energy_props(PropTab t, EGeo g, EFields
             ok2[u] = okh && okt;
         }
         t_intervals<KW>(t, xt, l.st, i2, tq2, k2);
-        double4 cd2[ECELL], cm2[ECELL], ck2[ECELL];
+        double4 cd2[ECELL], cm2[ECELL], ck2[ECELL];   // unused unless second
+        if (second) {
 #pragma unroll
-        for (int u = 0; u < ECELL; ++u) {
-            cd2[u] = l.td(t, k2[u]);
-            quad_mk(t.rt, k2[u], cm2[u], ck2[u]);
+            for (int u = 0; u < ECELL; ++u) {
+                cd2[u] = l.td(t, k2[u]);
+                quad_mk(t.rt, k2[u], cm2[u], ck2[u]);
+            }
         }
 #pragma unroll
         for (int u = 0; u < ECELL; ++u) {
