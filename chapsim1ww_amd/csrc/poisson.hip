@@ -854,6 +854,20 @@ __global__ void k_zero(double* __restrict__ p, size_t n) {
 // ---------------------------------------------------------------------------
 bool tdma_seg_config(int n, bool cyclic, int* MS, int* P, int* LPB, int maxthr, bool lpb_small = false);
 
+// rows j per block of k_reg_z: 8 T threads a row, 72 to 128 a block for the
+// two-stage lengths (T up to 16), one row of up to 1024 for the others
+inline int reg_z_rows(const RegPlan& p) { return std::max(1, 16 / p.T); }
+
+// LDS bytes of a block of the z transforms of h (NCL3 = 256 and lengths with a
+// register plan need less than the Stockham stages' two buffers).
+size_t poisson_z_lds(const chs_handle* h) {
+    const bool f64 = h->precision == CHS_FP64;
+    RegPlan rz;
+    if (h->N == 256) return sizeof(double2) * (size_t)8 * (F16T + 1);
+    if (f64 && reg_plan(h->N, false, &rz)) return sizeof(double2) * (size_t)8 * reg_z_rows(rz) * h->N;
+    return (f64 ? sizeof(double2) : sizeof(float2)) * (size_t)2 * ZTX * h->N;
+}
+
 template <typename Rl, typename TI = double>
 static int poisson_pass(chs_handle* h, const TI* f, double* dph, int ghost, cpx_t<Rl>* S, const cpx_t<Rl>* twx,
                         const cpx_t<Rl>* twz, const float* rphi = nullptr, float* phf = nullptr) {
@@ -890,7 +904,7 @@ static int poisson_pass(chs_handle* h, const TI* f, double* dph, int ghost, cpx_
     const int pb = xr ? std::max(1, (rx.nst == 2 ? 128 : 256) / rx.T) : 1;   // row pairs per block
     const dim3 gxr((nrows + 2 * pb - 1) / (2 * pb)), bxr(pb * (xr ? rx.T : 1));
     const size_t smxr = xr ? sizeof(double2) * (size_t)pb * (L + rx.T) : 0;
-    const int jb = zr ? std::max(1, 16 / rz.T) : 1;   // rows j per block: 128 threads at least
+    const int jb = zr ? reg_z_rows(rz) : 1;
     const dim3 gzr(LHP / 8, (M + jb - 1) / jb), bzr(8 * jb * (zr ? rz.T : 1));
     const size_t smzr = zr ? sizeof(double2) * (size_t)8 * jb * N : 0;
     auto fft_z_reg = [&](int dir) -> int {

@@ -1583,6 +1583,7 @@ __global__ void __launch_bounds__(256) k_max2_tiles(const double* __restrict__ p
 bool tdma_seg_config(int n, bool cyclic, int* MS, int* P, int* LPB, int maxthr, bool lpb_small = false);
 int poisson_solve(chs_handle* h, const double* f, double* dph, int ghost, double abs_tol);
 int poisson_solve_unchecked(chs_handle* h, const double* f, double* dph, int ghost);
+size_t poisson_z_lds(const chs_handle* h);
 
 // The verdict of the last mixed-precision substep's convergence check, once
 // its values have reached the host: wait = false leaves it pending while the
@@ -1954,6 +1955,24 @@ static int zwin_chunk(const chs_handle* h) {
     return std::max(8, rows(nch));
 }
 
+// One substep's hold on the handle's stencil cache: the lock, and on every way
+// out, a launch that fails included, the last-use event after what was queued
+// (an entry evicted later then waits for it).
+struct CnUse {
+    std::unique_lock<std::mutex> lk;
+    CnStencils* cn;
+    hipStream_t s;
+    hipError_t release() {
+        hipError_t e = hipSuccess;
+        if (lk.owns_lock()) {
+            if (cn && cn->dev) e = hipEventRecord(cn->buf.used, s);
+            lk.unlock();
+        }
+        return e;
+    }
+    ~CnUse() { (void)release(); }
+};
+
 int rk3_substep(chs_handle* h, int ns, double dt) {
     CHS_TRY(mixed_check(h, false));
     const Geo g = geo_of(h);
@@ -1967,10 +1986,20 @@ int rk3_substep(chs_handle* h, int ns, double dt) {
     hipEvent_t ev;
     // the handle's stencil cache stays locked until the substep's kernels
     // that read the stencils are queued and their last-use event recorded
-    std::unique_lock<std::mutex> lk(h->cn_mu);
-    CnStencils* cn = nullptr;
-    CHS_TRY(cn_stencils_locked(h, facoe, &cn));
+    CnUse use{std::unique_lock<std::mutex>(h->cn_mu), nullptr, s};
+    CHS_TRY(cn_stencils_locked(h, facoe, &use.cn));
+    const CnStencils* cn = use.cn;
     const bool use_st = stencil_path(h, *cn);
+    // what the grid may be refused for, before anything is written: the
+    // segments of the Thomas path's z lines, the LDS of the z transforms, the
+    // block sums of the right-hand side
+    int zMS = 0, Pz = 0, zLPB = 0;
+    CHS_CHECK(use_st || tdma_seg_config(h->N, true, &zMS, &Pz, &zLPB, 1024), CHS_E_ARG,
+              "substep: unsupported NCL3 (no segments for the Thomas path's z lines)");
+    CHS_CHECK(poisson_z_lds(h) <= (size_t)h->lds_max, CHS_E_ARG,
+              "substep: unsupported NCL3 (z transforms too long for the LDS)");
+    CHS_CHECK((long)h->M * (h->N / KR) <= 2L * h->npart, CHS_E_ARG,
+              "substep: NCL2 * NCL3 too large for the block-sum buffer");
     // the mixed form's FP32 stencils run where NCL3 is a multiple of 64 and
     // NCL1 one of 16; its other grids keep the precision they have always had,
     // FP64 stencils
@@ -2173,25 +2202,20 @@ int rk3_substep(chs_handle* h, int ns, double dt) {
             }
             h->timer.end(ev, "z_solve", s);
         }
-        int MS, Pz, LPB;
-        if (!tdma_seg_config(h->N, true, &MS, &Pz, &LPB, 1024)) {
-            set_error("substep: unsupported NCL3");
-            return CHS_E_ARG;
-        }
-        const int nlines = 3 * h->L * h->M;
-        while (LPB > 16 && LPB * Pz > 128) LPB /= 2;   // small blocks overlap their phases
-        const dim3 gz((nlines + LPB - 1) / LPB), bz(LPB * Pz);
-        const size_t smz = seg_smem_bytes<double>(LPB, Pz, true);
-        const int usedpg = 1;
         if (!use_st) {
-        h->timer.begin("z_solve", s, &ev);
-        switch (MS) {
-            case 16: CHS_LAUNCH(k_z_solve<16>, gz, bz, smz, s, g, h->rhs, h->scalars, xone, za, zb, zc, LPB, Pz, usedpg); break;
-            case 12: CHS_LAUNCH(k_z_solve<12>, gz, bz, smz, s, g, h->rhs, h->scalars, xone, za, zb, zc, LPB, Pz, usedpg); break;
-            case 4: CHS_LAUNCH(k_z_solve<4>, gz, bz, smz, s, g, h->rhs, h->scalars, xone, za, zb, zc, LPB, Pz, usedpg); break;
-            default: CHS_LAUNCH(k_z_solve<8>, gz, bz, smz, s, g, h->rhs, h->scalars, xone, za, zb, zc, LPB, Pz, usedpg); break;
-        }
-        h->timer.end(ev, "z_solve", s);
+            const int nlines = 3 * h->L * h->M, usedpg = 1;
+            int LPB = zLPB;
+            while (LPB > 16 && LPB * Pz > 128) LPB /= 2;   // small blocks overlap their phases
+            const dim3 gz((nlines + LPB - 1) / LPB), bz(LPB * Pz);
+            const size_t smz = seg_smem_bytes<double>(LPB, Pz, true);
+            h->timer.begin("z_solve", s, &ev);
+            switch (zMS) {
+                case 16: CHS_LAUNCH(k_z_solve<16>, gz, bz, smz, s, g, h->rhs, h->scalars, xone, za, zb, zc, LPB, Pz, usedpg); break;
+                case 12: CHS_LAUNCH(k_z_solve<12>, gz, bz, smz, s, g, h->rhs, h->scalars, xone, za, zb, zc, LPB, Pz, usedpg); break;
+                case 4: CHS_LAUNCH(k_z_solve<4>, gz, bz, smz, s, g, h->rhs, h->scalars, xone, za, zb, zc, LPB, Pz, usedpg); break;
+                default: CHS_LAUNCH(k_z_solve<8>, gz, bz, smz, s, g, h->rhs, h->scalars, xone, za, zb, zc, LPB, Pz, usedpg); break;
+            }
+            h->timer.end(ev, "z_solve", s);
         }
     }
     // 3. y solves + Q update + BC_WALL_Q
@@ -2227,7 +2251,6 @@ int rk3_substep(chs_handle* h, int ns, double dt) {
             set_error("substep: unsupported NCL2");
             return CHS_E_ARG;
         }
-        lk.unlock();
         const int nlines = h->L * h->N;
         const dim3 gy((nlines + LPB - 1) / LPB), by(LPB * P);
         const size_t smy = seg_smem_bytes<double>(LPB, P);
@@ -2240,10 +2263,8 @@ int rk3_substep(chs_handle* h, int ns, double dt) {
         }
         h->timer.end(ev, "y_solve", s);
     }
-    if (lk.owns_lock()) {
-        if (cn->dev) CHS_HIP(hipEventRecord(cn->buf.used, s));
-        lk.unlock();
-    }
+    if (!use_st) use.cn = nullptr;   // the Thomas path reads no weights
+    CHS_HIP(use.release());
     // 4. DIVG
     h->timer.begin("divg", s, &ev);
     CHS_LAUNCH(k_divg, dim3(row_tile_blocks(h->L, h->N, (h->M + DVJ - 1) / DVJ)), dim3(256), 0, s, g,
