@@ -9,17 +9,19 @@
 namespace chs {
 
 // Segmented solver: LPB lines per block, P = ceil(n / MS) segments per line.
-template <int MS, bool CYC>
+// Consecutive lanes take consecutive lines (also where the rows are the
+// contiguous ones: non-cyclic 65536 x 192, 0.203 ms, 0.319 with consecutive
+// segments of a line), or with ROWC consecutive segments of one line (short
+// cyclic lines with contiguous rows: 65536 x 32, 8 lines a block, 26.4 against
+// 30.6 us).  SERIAL (cyclic): one thread per line sweeps the reduced system.
+template <int MS, bool CYC, bool ROWC = false, bool SERIAL = false>
 __global__ void __launch_bounds__(1024) k_tdma_seg(const double* __restrict__ A, const double* __restrict__ B,
                                                    const double* __restrict__ Cc, double* __restrict__ Rr,
                                                    const double* __restrict__ bc, int n, int nlines,
                                                    long long es, long long ls, int LPB, int P) {
     extern __shared__ unsigned char smem[];
     const int tid = threadIdx.x;
-    // consecutive lanes take consecutive lines, also where the rows are the
-    // contiguous ones (measured at 65536 x 192, es = 1, with consecutive
-    // segments of a line instead: 0.203 -> 0.319 ms)
-    int ll = tid % LPB, seg = tid / LPB;
+    int ll = ROWC ? tid / P : tid % LPB, seg = ROWC ? tid % P : tid / LPB;
     // hides that ll and seg come from one division: with that known the loads'
     // addresses are kept apart in registers (126 instead of 92 at MS = 8)
     asm("" : "+v"(ll), "+v"(seg));
@@ -63,7 +65,7 @@ __global__ void __launch_bounds__(1024) k_tdma_seg(const double* __restrict__ A,
                 }
         }
     }
-    seg_solve<MS, double>(a, b, c, d, LPB, P, ll, seg, valid, CYC, smem);
+    seg_solve<MS, double, SERIAL>(a, b, c, d, LPB, P, ll, seg, valid, CYC, smem);
     if (valid) {
 #pragma unroll
         for (int l = 0; l < MS; ++l) {
@@ -245,60 +247,142 @@ static int lines_per_block(int p, int lpb0, int lo, int thr) {
     return lpb;
 }
 
-// ws: the sequential fallback's workspace of 3 n nlines doubles, or nullptr to
-// take it from the stream-ordered pool for this launch
+// The kernel of a batch of lines: k_tdma_seg with its reduced systems by
+// parallel cyclic reduction (Pcr) or, cyclic, by one thread per line (Serial);
+// k_tdma_cyc (Split); k_tdma_seq (Seq), the only one with a workspace.
+enum class TdmaKind { Pcr, Serial, Split, Seq };
+struct TdmaPlan {
+    TdmaKind kind;
+    int ms, lpb;   // rows per segment, lines per block
+    bool rowc;     // consecutive lanes take consecutive segments of a line
+};
+
+// Rows per segment and lines per block by the number of lines and rows, from a
+// sweep of all of them on an MI355X: 42 lengths from 8 to 512 rows x 20 to 23
+// counts from 16 to 65536 lines, both layouts.  Over the sweep the choice is on
+// average 2% (lines contiguous), 11% and 7% (rows contiguous, non-cyclic and
+// cyclic) behind the fastest
+// candidate of each point; what it loses most at: 30% to 2 lines a block (64
+// lines of 512 rows, 11.5 against 8.9 us), 20% to 2 lines of 4-row segments
+// (65536x192, rows contiguous, 181 against 145).  What decides:
+//   fullest CU    on_cu(lpb): the lines of the CU with the most, in whole
+//     blocks.  Where 32 lines a block leave it no more than 16 do, the larger
+//     accesses win (non-cyclic 65536x128 72 us with 32, 85 with 16; 14000x144,
+//     12 x 32, 21.6, 8 x 16 23.1), otherwise the evener split (20000x128 22.5,
+//     21.3).
+//   straddled     16 lines are one 128-byte line only where the row pitch is a
+//     multiple of 16 values; elsewhere they touch two, 64 lines five for four
+//     (8500x64 16 lines 11.6 us, 32 10.5, 64 9.7; 32767x64 26.4, 21.0, 19.7)
+//   resident      above 4096 lines a block of at most 8 waves, so that two on
+//     a CU overlap their phases: 12-row segments for 257 to 384 rows (10000x360
+//     12 x 16 40.9 us, 8 x 16 50.5, 8 x 8 51.5), 8 lines beyond (10000x504 61.8
+//     against 71.1)
+//   few lines     fewer lines a block, so that no CU is idle: 16 up to 4096
+//     lines (2000x192 8.9 us; 8 lines 10.8, 32 12.1), 8 below 1280 (1000x192
+//     8.0, 16 lines 9.1)
+//   rows contiguous  blocks of about 128 threads: 10000x360 58 us (8 lines 69,
+//     16 80); 4-row segments (8 waves to a SIMD for the 5 of 8-row ones) for
+//     17 to 128 rows from 14000 lines on (65536x28 20 us, 8 x 16 26; 45000x56
+//     27, 8 x 16 37; 32768x120 48, 8 x 16 58)
+//   cyclic        short lines of whole segments: the serial sweep of a reduced
+//     system of up to 20 rows (32 at most) has two barriers where the cyclic
+//     reduction has two a step (10000x16 3.9 us, Split 4.9; 65536x96 12 x 32 57, Split 68;
+//     rows contiguous 65536x8 6.9, Split 10.9); whole 12-row segments
+//     of 132 to 192 rows (65536x192 121 us, Split 150) and of 257 to 384
+//     (10000x360 42, Split 60); everything else Split
+static TdmaPlan tdma_plan(int n, int nlines, long long es, long long ls, bool cyclic) {
+    constexpr int CUS = 256;
+    const int p8 = (n + 7) / 8, p12 = (n + 11) / 12, ps = (n + 6) / 8;   // segments; ps: of the n - 1 rows of Split
+    const bool whole8 = n % 8 == 0, whole12 = n % 12 == 0;
+    auto on_cu = [&](long lpb) { return ((nlines + lpb - 1) / lpb + CUS - 1) / CUS * lpb; };
+    const bool wide = on_cu(32) <= on_cu(16), straddled = es % 16 != 0, few = nlines <= 4096;
+    const bool at_once = nlines <= 64 * CUS;   // every block of 64 lines on a CU of its own
+    auto split = [&](int lpb) {
+        lpb = lines_per_block(ps, lpb, 2, 512);
+        return TdmaPlan{ps * lpb <= 512 ? TdmaKind::Split : TdmaKind::Seq, 8, lpb, es == 1};
+    };
+    auto pcr = [&](int ms, int lpb) {
+        const int p = (n + ms - 1) / ms;
+        lpb = lines_per_block(p, lpb, 4, 1024);
+        return TdmaPlan{p * lpb <= 1024 ? TdmaKind::Pcr : TdmaKind::Seq, ms, lpb, false};
+    };
+    auto serial = [&](int ms, int lpb) { return TdmaPlan{TdmaKind::Serial, ms, lpb, es == 1}; };
+    // 16, 32 or 64 of more than 4096 contiguous lines, in blocks of p threads a line
+    auto lines = [&](int p) { return straddled && nlines > 8192 && (at_once || p <= 8) ? 64 : wide ? 32 : 16; };
+
+    if (!cyclic && ls == 1) {
+        if (p8 <= 2) return pcr(8, 64);
+        if (nlines < 1280) return pcr(8, p8 <= 6 ? 16 : 8);
+        if (few) return pcr(8, 16);
+        if (p8 <= 4) return pcr(8, straddled && nlines > 8192 ? 64 : 32);
+        if (p8 <= 16) return p12 == 8 && wide && !at_once ? pcr(12, 32) : pcr(8, lines(p8));
+        if (p8 <= 32 && nlines <= 8192 && wide) return pcr(8, 32);
+        if (p12 <= 16 && wide) return pcr(12, 32);
+        if (p8 <= 32) return pcr(8, 16);
+        if (p12 <= 32) return pcr(12, wide ? 32 : 16);
+        return pcr(8, 8);
+    }
+    if (!cyclic) {
+        if (p8 >= 3 && p8 <= 16 && nlines >= 14000) return pcr(4, 8);
+        if (p8 <= 2) return pcr(8, p8 == 2 && nlines >= 30000 ? 16 : 32);
+        return pcr(8, lines_per_block(p8, 16, 4, 128));
+    }
+    if (ls == 1) {
+        const int ms = whole12 && n >= 24 ? 12 : whole8 && n >= 16 ? 8 : n % 4 == 0 && n >= 8 && n <= 20 ? 4 : 0;
+        const int p = ms ? n / ms : n;
+        if (ms && few && p <= (ms == 12 ? 4 : 6)) return serial(ms, p <= 3 && ms < 12 ? 32 : 16);
+        if (ms && !few && p <= (ms == 12 ? 8 : 10)) {
+            const bool l64 = on_cu(64) <= on_cu(32) && (at_once || (p <= 8 && (straddled || nlines <= 32768)));
+            return serial(ms, l64 ? 64 : 32);
+        }
+        if (whole8 && p8 <= 16 && straddled && at_once && nlines > 8192) return serial(8, 64);
+        if (whole12 && !few && p12 >= 11 && p12 <= 16) return pcr(12, wide ? 32 : 16);
+        if (n > 256 && n <= 384 && nlines >= 1280) {
+            if (whole12) return pcr(12, 16);
+            if (whole8) return pcr(8, 16);
+        }
+        return split(nlines < 1280 ? (ps <= 4 ? 16 : 8) : few ? 16 : lines(ps));
+    }
+    if (whole8 && p8 >= 2 && p8 <= 8 && (p8 <= 6 || !few))
+        return serial(8, p8 == 2 ? 32 : p8 == 3 && nlines <= 8192 ? 16 : 8);
+    if (n % 4 == 0 && n >= 8 && n <= 28 && (n <= 12 || nlines >= 14000)) return serial(4, n == 12 || n == 28 ? 16 : 32);
+    return split(lines_per_block(ps, 64, 2, 64));
+}
+
+// ws: the workspace of k_tdma_seq, 3 n nlines doubles, or nullptr to take it
+// from the stream-ordered pool for this launch
 int tdma_launch(const double* a, const double* b, const double* c, double* r, const double* bc, int n, int nlines,
                 long long es, long long ls, int cyclic, hipStream_t s, double* ws_given = nullptr) {
-    // Rows per segment and lines per block, swept on an MI355X for both
-    // layouts (lines x rows: best of the sweep; before: one configuration per
-    // layout, 12 x 32 for lines contiguous, 8 x 16 for rows contiguous):
-    //   lines contiguous   500x192 7.7 (11.4) us, 4000x192 11.0 (12.9),
-    //     2000x504 16.7 (37.3), 20000x504 113 (150): 8-row segments, 16 lines
-    //     (a 128-byte access) or 8 where few lines leave CUs idle; only a whole
-    //     grid's lines (65536x192) keep 12 x 32: 113 against 129 us
-    //   rows contiguous    500x192 7.2 (12.9), 10000x360 52.8 (75.3),
-    //     20000x504 131 (214): blocks of about 128 threads, whose phases
-    //     overlap; 65536x192 182 (189)
-    //   cyclic             through the split-off unknown (k_tdma_cyc), whose
-    //     reduced systems have no serial sweep: 500x192 8.3 (15.2), 2000x504
-    //     20.0 (20.1), rows contiguous 500x192 6.9 (20.3), 20000x504 144 (287);
-    //     only a whole grid's contiguous lines of whole 12-row segments stay
-    //     with k_tdma_seg: 65536x192 110 against 148 us, 40000x360 at 12 x 16
-    //     (two blocks per CU; 12 x 32: 170) 132 us
-    const bool grid_lines = nlines >= 32768, lines_contig = ls == 1;
-    int MS = 8, LPB = 0;
-    const int p12 = (n + 11) / 12;   // 12 x 32: blocks whose waves fill a CU's 16 (one block of 9 would leave 7 idle)
-    if (lines_contig && grid_lines && ((p12 >= 4 && p12 <= 16) || (p12 >= 28 && p12 <= 32)) &&
-        (!cyclic || n % 12 == 0)) {
-        MS = 12;
-        LPB = cyclic && p12 > 16 ? 16 : 32;
-    } else if (cyclic) {
-        const int p = (n - 1 + MS - 1) / MS;
-        LPB = es == 1 ? lines_per_block(p, 64, 2, 64)
-                      : lines_per_block(p, p <= 4 ? 32 : nlines < 2048 ? 8 : 16, 2, 512);
-        if (p * LPB <= 512) {
-            const size_t sm = std::max(seg_smem_bytes<double2>(LPB, p), 2 * sizeof(double2) * (size_t)LPB);
-            CHS_LAUNCH(k_tdma_cyc<8>, dim3((nlines + LPB - 1) / LPB), dim3(LPB * p), sm, s, a, b, c, r, n, nlines, es,
-                       ls, LPB, p);
-            return CHS_OK;
-        }
-        LPB = 0;
-    } else if (lines_contig) {
-        const int p = (n + MS - 1) / MS;
-        LPB = lines_per_block(p, p <= 4 ? 32 : nlines < 2048 ? 8 : 16, 4, 1024);
-    } else {
-        LPB = lines_per_block((n + MS - 1) / MS, 32, 4, 128);
+    const TdmaPlan t = tdma_plan(n, nlines, es, ls, cyclic != 0);
+    const int LPB = t.lpb;
+    if (t.kind == TdmaKind::Split) {
+        const int P = (n - 1 + t.ms - 1) / t.ms;
+        const size_t sm = std::max(seg_smem_bytes<double2>(LPB, P), 2 * sizeof(double2) * (size_t)LPB);
+        CHS_LAUNCH(k_tdma_cyc<8>, dim3((nlines + LPB - 1) / LPB), dim3(LPB * P), sm, s, a, b, c, r, n, nlines, es, ls,
+                   LPB, P);
+        return CHS_OK;
     }
-    const int P = (n + MS - 1) / MS;
-    if (LPB > 0 && P * LPB <= 1024) {
+    if (t.kind != TdmaKind::Seq) {
+        const int P = (n + t.ms - 1) / t.ms;
         const dim3 grid((nlines + LPB - 1) / LPB), block(LPB * P);
-        const size_t sm = seg_smem_bytes<double>(LPB, P, cyclic != 0);
-        if (cyclic)
-            CHS_LAUNCH((k_tdma_seg<12, true>), grid, block, sm, s, a, b, c, r, bc, n, nlines, es, ls, LPB, P);
-        else if (MS == 12)
-            CHS_LAUNCH((k_tdma_seg<12, false>), grid, block, sm, s, a, b, c, r, bc, n, nlines, es, ls, LPB, P);
-        else
-            CHS_LAUNCH((k_tdma_seg<8, false>), grid, block, sm, s, a, b, c, r, bc, n, nlines, es, ls, LPB, P);
+        const size_t sm = seg_smem_bytes<double>(LPB, P, cyclic && t.kind == TdmaKind::Pcr);   // at most 64 KiB
+#define CHS_SEG(...) \
+    CHS_LAUNCH((k_tdma_seg<__VA_ARGS__>), grid, block, sm, s, a, b, c, r, bc, n, nlines, es, ls, LPB, P)
+        if (t.kind == TdmaKind::Serial) {
+            if (t.ms == 12) CHS_SEG(12, true, false, true);
+            else if (t.ms == 8 && t.rowc) CHS_SEG(8, true, true, true);
+            else if (t.ms == 8) CHS_SEG(8, true, false, true);
+            else if (t.rowc) CHS_SEG(4, true, true, true);
+            else CHS_SEG(4, true, false, true);
+        } else if (cyclic) {
+            if (t.ms == 12) CHS_SEG(12, true);
+            else CHS_SEG(8, true);
+        } else {
+            if (t.ms == 12) CHS_SEG(12, false);
+            else if (t.ms == 4) CHS_SEG(4, false);
+            else CHS_SEG(8, false);
+        }
+#undef CHS_SEG
         return CHS_OK;
     }
     const int bs = 256;
