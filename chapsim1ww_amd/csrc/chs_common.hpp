@@ -226,11 +226,19 @@ inline int march_chunk_rows(int rows, int nkg, size_t smem, int lds_max, bool fi
 
 // xz-plane sums in two stages of a fixed order: one block of 256 threads per
 // (row j, chunk of kc z rows) leaves its NM sums in part[(chunk M + j) NM + m],
-// then k_xz_finish adds a row's chunks and scales.  Chunks: about 2048 blocks,
-// at least 4 z rows each, at most what cap values hold.
-inline int xz_chunk(int M, int N, int nm, long cap) {
-    const int nch = (int)std::max(1L, std::min({(long)(N + 3) / 4, (2048L + M - 1) / M, cap / ((long)nm * M)}));
-    return (N + nch - 1) / nch;
+// then k_xz_finish adds a row's chunks and scales; of a single chunk the blocks
+// scale their own.  Chunks: about 2048 blocks, at least 4 z rows and XZ_CELLS
+// cells each (fewer leave a block's time to its reduction and the finish to a
+// chain of loads), at most what cap values hold.  A call of chs_mean_xz at
+// 16x40x200 in 50 chunks 53 us, of one block a row 31, now 29; at 64x64x64 37,
+// 30 and 28, of chs_mean_xz_io 61, 65 and 41; at 128x64x128 51, 58 and 33, 88,
+// 199 and 50 (512 cells a chunk at least: 45 and 82 without wave_sums, 1024 39
+// and 67, 2048 36 and 60, but 31 and 53 at 64x64x64).
+constexpr int XZ_CELLS = 1024;
+inline int xz_chunk(int L, int M, int N, int nm, long cap) {
+    const long nch = std::max(1L, std::min({(long)(N + 3) / 4, (2048L + M - 1) / M, (long)L * N / XZ_CELLS,
+                                            cap / ((long)nm * M)}));
+    return (int)((N + nch - 1) / nch);
 }
 // The block's tile: each XCD walks rows in j order, whose v(j + 1) is the next
 // tile's v(j).  f(i, k) for the cells of the tile this thread sums: lanes
@@ -245,27 +253,58 @@ struct XzTile {
     }
     template <class F>
     __device__ __forceinline__ void cells(int L, int N, int kc, F f) const {
-        const int Lr = min(256, (L + 63) & ~63), R = 256 / Lr;
+        const int Lr = L <= 16 ? 16 : L <= 32 ? 32 : min(256, (L + 63) & ~63), R = 256 / Lr;
         const int r = threadIdx.x / Lr, i0 = threadIdx.x - r * Lr, k1 = min(N, (ch + 1) * kc);
         if (r >= R) return;
         for (int k = ch * kc + r; k < k1; k += R)   // unrolled: 299 -> 342 us (k_mean_xz_io), 110 -> 107 us (k_mean_xz)
             for (int i = i0; i < L; i += Lr) f(i, k);
     }
 };
-// The block's sums of acc[0..NM-1] to out (a shuffle tree per wave, then the
-// four waves in order); 256 threads, red: 4 NM doubles of LDS.
-template <int NM>
-__device__ __forceinline__ void xz_block_sums(const double (&acc)[NM], double* red, double* __restrict__ out) {
+// The wave's sums of v[0..N-1], one to a lane: of the values left a lane passes
+// half to its partner at distance O and keeps the other half, so that the six
+// steps move 40 values of 37 where full butterflies move 222 (the same
+// pairings: the same sums).  Returns the lane's sum; m += its index; left: how
+// many of v[] are values (the rest pad the halves), 0 at the end: no sum.
+template <int O, int N>
+__device__ __forceinline__ double wave_sums(const double (&v)[N], int& m, int& left) {
+    if constexpr (O == 0) {
+        return v[0];
+    } else {
+        constexpr int H = (N + 1) / 2;
+        double w[H];
+        if constexpr (N == 1) {
+            w[0] = v[0] + __shfl_xor(v[0], O);
+        } else {
+            const bool up = threadIdx.x & O;
 #pragma unroll
-    for (int m = 0; m < NM; ++m) {
-        double v = acc[m];
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-        if ((threadIdx.x & 63) == 0) red[(threadIdx.x >> 6) * NM + m] = v;
+            for (int i = 0; i < H; ++i) {
+                const double a = v[i], b = i + H < N ? v[i + H] : 0.0;
+                w[i] = (up ? b : a) + __shfl_xor(up ? a : b, O);
+            }
+            m += up ? H : 0;
+            left = up ? max(left - H, 0) : min(left, H);
+        }
+        return wave_sums<O / 2, H>(w, m, left);
     }
+}
+// The block's sums of acc[0..NM-1], as fin(m, sum), to out (a tree over the
+// lanes of a wave, then the four waves in order); 256 threads, red: 4 NM
+// doubles of LDS.
+template <int NM, class F>
+__device__ __forceinline__ void xz_block_sums(const double (&acc)[NM], double* red, double* __restrict__ out, F fin) {
+    int i = 0, left = NM;
+    const double v = wave_sums<32, NM>(acc, i, left);
+    if (left > 0) red[(threadIdx.x >> 6) * NM + i] = v;
     __syncthreads();
     const int m = threadIdx.x;
-    if (m < NM) out[m] = (red[m] + red[NM + m]) + (red[2 * NM + m] + red[3 * NM + m]);
+    if (m < NM) out[m] = fin(m, (red[m] + red[NM + m]) + (red[2 * NM + m] + red[3 * NM + m]));
+}
+// the sum of part[c n + e] over the chunks c in order, eight loads in flight
+__device__ __forceinline__ double xz_chunk_sum(const double* __restrict__ part, int n, int nch, int e) {
+    double s = 0.0;
+#pragma unroll 8
+    for (int c = 0; c < nch; ++c) s += part[(size_t)c * n + e];
+    return s;
 }
 
 struct CnCache;   // truncated-inverse CN stencils of one handle (substep.hip)

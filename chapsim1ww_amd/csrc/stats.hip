@@ -30,7 +30,8 @@ __global__ void __launch_bounds__(256) k_mean_xz_io(StatGeo g, const double* __r
                                                     const double* __restrict__ Gf, const double* __restrict__ PR,
                                                     const double* __restrict__ T, const double* __restrict__ RHO,
                                                     const double* __restrict__ H, const double* __restrict__ MU,
-                                                    int thermal, int kc, int nch, double* __restrict__ part) {
+                                                    int thermal, int kc, int nch, double VL,
+                                                    double* __restrict__ part) {
     __shared__ double red[4 * NIO];
     const int L = g.L, N = g.N;
     XzTile t;
@@ -83,16 +84,14 @@ __global__ void __launch_bounds__(256) k_mean_xz_io(StatGeo g, const double* __r
             }
         }
     });
-    xz_block_sums(acc, red, part + (size_t)NIO * (t.ch * g.M + t.j));
+    xz_block_sums(acc, red, part + (size_t)NIO * (t.ch * g.M + t.j),
+                  [=](int, double v) { return nch == 1 ? v * VL : v; });
 }
 
 // out[e] = scale sum over the chunks of part[c n + e], e < n = 37 M
 __global__ void k_xz_finish(const double* __restrict__ part, int n, int nch, double scale, double* __restrict__ out) {
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= n) return;
-    double s = 0.0;
-    for (int c = 0; c < nch; ++c) s += part[(size_t)c * n + e];
-    out[e] = s * scale;
+    if (e < n) out[e] = xz_chunk_sum(part, n, nch, e) * scale;
 }
 
 // acc = coe3 acc + coe2 val over n values
@@ -123,12 +122,12 @@ int mean_xz_io(chs_handle* h, const chs_thermal_fields* tf, const chs_io_fields*
     const hipStream_t s = h->stream;
     double* xz = xz_of(h, 1);
     const StatGeo g{h->L, h->M, h->N};
-    const int kc = xz_chunk(h->M, h->N, NIO, 2L * h->npart), nch = (h->N + kc - 1) / kc, n = NIO * h->M;
+    const int kc = xz_chunk(h->L, h->M, h->N, NIO, 2L * h->npart), nch = (h->N + kc - 1) / kc, n = NIO * h->M;
+    const double VL = 1.0 / ((double)h->L * (double)h->N);
     CHS_LAUNCH(k_mean_xz_io, dim3(8 * ((h->M * nch + 7) / 8)), dim3(256), 0, s, g, f->q, f->g, f->pr,
                thermal ? tf->temperature : nullptr, thermal ? tf->density : nullptr, thermal ? tf->enthalpy : nullptr,
-               thermal ? tf->viscosity : nullptr, thermal, kc, nch, h->partials);
-    CHS_LAUNCH(k_xz_finish, dim3((n + 255) / 256), dim3(256), 0, s, h->partials, n, nch,
-               1.0 / ((double)h->L * (double)h->N), xz);
+               thermal ? tf->viscosity : nullptr, thermal, kc, nch, VL, nch == 1 ? xz : h->partials);
+    if (nch > 1) CHS_LAUNCH(k_xz_finish, dim3((n + 255) / 256), dim3(256), 0, s, h->partials, n, nch, VL, xz);
     if (out_host) {
         CHS_HIP(hipMemcpyAsync(out_host, xz, (size_t)NIO * h->M * sizeof(double), hipMemcpyDeviceToHost, s));
         CHS_HIP(hipStreamSynchronize(s));

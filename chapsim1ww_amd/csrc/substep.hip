@@ -1437,8 +1437,11 @@ __global__ void __launch_bounds__(256) k_divgck_cfl(Geo g, const double* __restr
 // (xz_chunk), out[13 j + m] as the C ABI documents (cell-centred u, v, w sums,
 // p, their products, u p).  Bound: HBM, 32 B/cell.  One block per row: 186 us
 // at 256x192x256 (2.2 TB/s), in chunks 110 us (3.7 TB/s).
+__device__ __forceinline__ double mean_xz_scale(int m, double VL) {
+    return m == 3 ? VL : (m >= 4 && m < 10) ? VL * (0.5 * 0.5) : VL * 0.5;
+}
 __global__ void __launch_bounds__(256) k_mean_xz(Geo g, const double* __restrict__ Q, const double* __restrict__ PR,
-                                                 int kc, int nch, double* __restrict__ part) {
+                                                 int kc, int nch, double VL, double* __restrict__ part) {
     __shared__ double red[4 * 13];
     const int L = g.L, N = g.N;
     XzTile t;
@@ -1466,17 +1469,15 @@ __global__ void __launch_bounds__(256) k_mean_xz(Geo g, const double* __restrict
 #pragma unroll
             for (int n = m; n < 3; ++n) acc[l++] += U[m] * U[n];
     });
-    xz_block_sums(acc, red, part + (size_t)13 * (t.ch * g.M + t.j));
+    xz_block_sums(acc, red, part + (size_t)13 * (t.ch * g.M + t.j),
+                  [=](int m, double v) { return nch == 1 ? v * mean_xz_scale(m, VL) : v; });
 }
 
 // the rows' chunks added in order, and the reference's scaling
 __global__ void k_mean_xz_finish(const double* __restrict__ part, int n, int nch, double VL, double* __restrict__ out) {
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= n) return;
-    const int m = e % 13;
-    double s = 0.0;
-    for (int c = 0; c < nch; ++c) s += part[(size_t)c * n + e];
-    out[e] = s * (m == 3 ? VL : (m >= 4 && m < 10) ? VL * (0.5 * 0.5) : VL * 0.5);
+    out[e] = xz_chunk_sum(part, n, nch, e) * mean_xz_scale(e % 13, VL);
 }
 
 // NaN-propagating maxima of nb <= 1024 pairs, one per thread
@@ -2330,10 +2331,12 @@ int mean_xz(chs_handle* h, double* out_host) {
     const Geo g = geo_of(h);
     const hipStream_t s = h->stream;
     // kept on the device for the time means (chs_mean_t)
-    const int kc = xz_chunk(h->M, h->N, 13, 2L * h->npart), nch = (h->N + kc - 1) / kc, n = 13 * h->M;
-    CHS_LAUNCH(k_mean_xz, dim3(8 * ((h->M * nch + 7) / 8)), dim3(256), 0, s, g, h->q, h->pr, kc, nch, h->partials);
-    CHS_LAUNCH(k_mean_xz_finish, dim3((n + 255) / 256), dim3(256), 0, s, h->partials, n, nch,
-               1.0 / ((double)h->L * (double)h->N), h->stats);
+    const int kc = xz_chunk(h->L, h->M, h->N, 13, 2L * h->npart), nch = (h->N + kc - 1) / kc, n = 13 * h->M;
+    const double VL = 1.0 / ((double)h->L * (double)h->N);
+    CHS_LAUNCH(k_mean_xz, dim3(8 * ((h->M * nch + 7) / 8)), dim3(256), 0, s, g, h->q, h->pr, kc, nch, VL,
+               nch == 1 ? h->stats : h->partials);
+    if (nch > 1)
+        CHS_LAUNCH(k_mean_xz_finish, dim3((n + 255) / 256), dim3(256), 0, s, h->partials, n, nch, VL, h->stats);
     CHS_HIP(hipMemcpyAsync(out_host, h->stats, 13 * (size_t)h->M * sizeof(double), hipMemcpyDeviceToHost, s));
     CHS_HIP(hipStreamSynchronize(s));
     return CHS_OK;
