@@ -193,7 +193,10 @@ __global__ void __launch_bounds__(PT) k_props_table(PropTab t, Rows rw, const do
 // leave less of the last round empty than 8 (2,097,152 cells 45.0 against 46.5,
 // 3,000,000 54 against 63, 4,200,000 67 against 80); more: 8, with more loads in
 // flight (6,300,000 128 with 2 against 125, 9,000,000 189 against 174).  Tables
-// too large for the wide form: one cell below PSMALL_N, 8 from there.
+// too large for the wide form: one cell below PSMALL_N, 8 from there (3000
+// knots, 1,572,863 cells: 50 against 49 us on a random field, 42 on a smooth
+// one, but 51 against 129 in rows of 700); those whose knots leave a CU a single block of 256, below PSMALL (4000
+// knots: 1,048,576 cells 53 against 41 us, 1,572,863 69 against 42).
 constexpr long long PSMALL = 1ll << 20, PMID = 3ll << 21, PSMALL_N = 3ll << 19;
 
 int props_table_launch(chs_props* p, const double* h, Rows rw, double* T, double* rho, double* mu, double* kap,
@@ -201,6 +204,7 @@ int props_table_launch(chs_props* p, const double* h, Rows rw, double* T, double
     const long long cells = rw.rowlen * rw.nrow;
     if (cells == 0) return CHS_OK;
     const bool wide = props_lds_wide(p) <= (size_t)p->lds_max;
+    const long long small = wide || 2 * props_lds_bytes(p) > (size_t)p->lds_max ? PSMALL : PSMALL_N;
 #define CHS_PROPS_L(KK, WIDE, PT, PCELL)                                                                         \
     do {                                                                                                         \
         const auto kern = k_props_table<KK, WIDE, PT, PCELL>;                                                    \
@@ -214,7 +218,7 @@ int props_table_launch(chs_props* p, const double* h, Rows rw, double* T, double
     } while (0)
 #define CHS_PROPS_K(KK)                                                                                          \
     do {                                                                                                         \
-        if (cells < (wide ? PSMALL : PSMALL_N))                                                                  \
+        if (cells < small)                                                                                       \
             CHS_PROPS_L(KK, false, 256, 1);                                                                      \
         else if (wide && cells < PMID)                                                                           \
             CHS_PROPS_L(KK, true, 1024, 2);                                                                      \
