@@ -437,9 +437,11 @@ extern "C" int chs_tdma_batched(const double* a_dev, const double* b_dev, const 
                             line_stride, cyclic, (hipStream_t)stream);
 }
 
-// chs_tdma_batched without any allocation: the segmented kernel needs only
-// LDS; the sequential fallback (lines the segmented kernel cannot split) takes
-// its 3 n nlines-double workspace from this GPU's static scratch array.
+// chs_tdma_batched without any allocation: of its kernels only k_tdma_seq has a
+// workspace, this GPU's static scratch array.  Lines that no segments of a
+// block of 32 divide (tdma_seg_config) are held to the size of that array,
+// whichever kernel takes them: the limit callers are promised does not move
+// with tdma_plan.
 extern "C" int chs_tdma_batched_noalloc(const double* a_dev, const double* b_dev, const double* c_dev, double* r_dev,
                                         const double* bc_dev, int n, int nlines, long long elem_stride,
                                         long long line_stride, int cyclic, void* stream) {
@@ -450,10 +452,12 @@ extern "C" int chs_tdma_batched_noalloc(const double* a_dev, const double* b_dev
     if (nlines == 0) return CHS_OK;
     int MS = 0, P = 0, LPB = 0;
     double* ws = nullptr;
-    if (!chs::tdma_seg_config(n, cyclic != 0, &MS, &P, &LPB, 1024, false)) {
-        CHS_CHECK(3 * (size_t)n * (size_t)nlines <= chs::TDMA_SCRATCH_DOUBLES, CHS_E_ARG,
-                  "chs_tdma_batched_noalloc: these lines need a workspace of 3*n*nlines doubles, above the "
-                  "4194304 of the static scratch array (use chs_tdma_batched)");
+    CHS_CHECK(chs::tdma_seg_config(n, cyclic != 0, &MS, &P, &LPB, 1024, false) ||
+                  3 * (size_t)n * (size_t)nlines <= chs::TDMA_SCRATCH_DOUBLES,
+              CHS_E_ARG,
+              "chs_tdma_batched_noalloc: lines of this length are held to 3*n*nlines <= 4194304, the doubles of the "
+              "static scratch array (use chs_tdma_batched)");
+    if (chs::tdma_plan(n, nlines, elem_stride, line_stride, cyclic != 0).kind == chs::TdmaKind::Seq) {
         const int st = chs::scratch_address(&ws);
         if (st != CHS_OK) return st;
     }

@@ -179,10 +179,12 @@ int chs_tdma_batched(const double *a_dev, const double *b_dev, const double *c_d
 /* chs_tdma_batched without any device allocation, for callers that cannot
  * allocate (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc).  No counterpart in the reference.  Non-cyclic lines of up
- * to 512 rows and cyclic ones of a multiple of 4 rows need no workspace; calls
- * with other lines are held to 3*n*nlines <= 4194304 doubles, those of a static
- * array (32 MiB) that each GPU holds until the process ends and that the
- * longest of them use (a few thousand rows); larger such calls return CHS_E_ARG.  Calls that overlap on one GPU share that
+ * to 512 rows, and cyclic ones of a multiple of 4 rows up to 128, 8 up to 256,
+ * 12 up to 384 or 16 up to 512, may be any number.  Calls with other lines are
+ * held to 3*n*nlines <= 4194304, the doubles of a static array (32 MiB) that
+ * each GPU holds until the process ends, whether or not their kernel uses it
+ * (lines of more than about 2048 rows do); larger such calls return CHS_E_ARG
+ * before anything is written.  Calls that overlap on one GPU share that
  * array and race; its contents are not cleared between calls (nothing in it
  * is read before it is written).  Same arguments and results as
  * chs_tdma_batched. */
