@@ -1696,10 +1696,11 @@ static int cyclic_stencil(int n, double a, double b, double c, std::vector<doubl
 
 // Device weights with the pinned buffer they are uploaded from, sized for the
 // widest windows; used: recorded after the upload and after each substep that
-// read dev.
+// read dev; captured: a graph may read dev whenever it is replayed.
 struct CnBuf {
     double *dev = nullptr, *host = nullptr;
     hipEvent_t used = nullptr;
+    bool captured = false;
 };
 
 struct CnStencils {
@@ -1714,13 +1715,23 @@ struct CnStencils {
 // The stencils of the last few FACOE values of one handle.  Entries are
 // evicted oldest first; an evicted entry's buffers serve a later one once
 // their last-use event has completed (never while a queued substep may read
-// them).  A run that changes DT with its CFL number brings three new values a
+// them); those of a captured substep stay until the handle goes.  A run that changes DT with its CFL number brings three new values a
 // step: allocating and freeing for each waited for the GPU (a step of its own
 // DT, with the cost of the inverses: 64^3 1244 -> 270, 256x192x256 11254 -> 2981 us).
 struct CnCache {
     std::list<CnStencils> live;   // list: entries keep their addresses; at most 8
     std::vector<CnBuf> retired;
+    std::vector<CnBuf> kept;      // captured
 };
+
+static bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cs) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return cs != hipStreamCaptureStatusNone;
+}
 
 static void free_buf(CnBuf& b) {
     if (b.dev) (void)hipFree(b.dev);
@@ -1737,7 +1748,7 @@ static int take_buf(CnCache& c, size_t n, CnBuf* out) {
         if (wait && i < 4) break;
         const size_t r = wait ? 0 : i;
         if ((wait ? hipEventSynchronize(c.retired[r].used) : hipEventQuery(c.retired[r].used)) != hipSuccess) {
-            (void)hipGetLastError();   // not ready, or recorded into a graph: not to be reused
+            (void)hipGetLastError();   // not ready
             continue;
         }
         *out = c.retired[r];
@@ -1763,6 +1774,7 @@ void release_stencils(chs_handle* h) {
     if (!c) return;
     for (auto& e : c->live)
         if (e.dev) c->retired.push_back(e.buf);
+    c->retired.insert(c->retired.end(), c->kept.begin(), c->kept.end());
     for (auto& b : c->retired) {
         (void)hipEventSynchronize(b.used);
         free_buf(b);
@@ -1874,17 +1886,30 @@ static int cn_stencils_locked(chs_handle* h, double facoe, CnStencils** out) {
                 const double* row = wy[c].data() + (size_t)j * WM + KMAX;
                 std::copy(row - st.Ky, row + st.Ky + 1, buf + st.oy + ((size_t)c * M + j) * W + (st.KW - st.Ky));
             }
-        hipError_t e = hipMemcpyAsync(st.dev, buf, n * sizeof(double), hipMemcpyHostToDevice, h->stream);
-        if (e == hipSuccess) e = hipEventRecord(st.buf.used, h->stream);
+        // Under capture the upload goes out at once on a stream of its own: in
+        // the graph it would only happen with the first replay, while a later
+        // eager substep takes the entry as it stands.
+        hipStream_t up = h->stream;
+        const bool cap = capturing(up);
+        hipError_t e = cap ? hipStreamCreateWithFlags(&up, hipStreamNonBlocking) : hipSuccess;
+        if (e == hipSuccess) {
+            e = hipMemcpyAsync(st.dev, buf, n * sizeof(double), hipMemcpyHostToDevice, up);
+            if (e == hipSuccess) e = hipEventRecord(st.buf.used, up);
+            if (e != hipSuccess || cap) {
+                const hipError_t w = hipStreamSynchronize(up);
+                if (e == hipSuccess) e = w;
+            }
+            if (cap) (void)hipStreamDestroy(up);
+        }
         if (e != hipSuccess) {
-            (void)hipStreamSynchronize(h->stream);
             free_buf(st.buf);
             set_error(std::string("CN stencil upload: ") + hipGetErrorString(e));
             return CHS_E_HIP;
         }
     }
     if (cache.live.size() >= 8) {
-        if (cache.live.front().dev) cache.retired.push_back(cache.live.front().buf);
+        const CnStencils& old = cache.live.front();
+        if (old.dev) (old.buf.captured ? cache.kept : cache.retired).push_back(old.buf);
         cache.live.pop_front();
     }
     cache.live.push_back(std::move(st));
@@ -1958,7 +1983,8 @@ static int zwin_chunk(const chs_handle* h) {
 
 // One substep's hold on the handle's stencil cache: the lock, and on every way
 // out, a launch that fails included, the last-use event after what was queued
-// (an entry evicted later then waits for it).
+// (an entry evicted later then waits for it), or under capture the mark that
+// keeps its buffers.
 struct CnUse {
     std::unique_lock<std::mutex> lk;
     CnStencils* cn;
@@ -1966,7 +1992,10 @@ struct CnUse {
     hipError_t release() {
         hipError_t e = hipSuccess;
         if (lk.owns_lock()) {
-            if (cn && cn->dev) e = hipEventRecord(cn->buf.used, s);
+            if (cn && cn->dev) {
+                if (capturing(s)) cn->buf.captured = true;
+                else e = hipEventRecord(cn->buf.used, s);
+            }
             lk.unlock();
         }
         return e;
