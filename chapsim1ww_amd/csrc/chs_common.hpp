@@ -175,18 +175,6 @@ inline unsigned row_tile_blocks(int L, int N, int nj) {
     return (unsigned)(8 * ((nt + 7) / 8));
 }
 
-// Rows per y chunk of a kernel that marches along y with an LDS ring, one
-// block per group of k rows (nkg groups) and chunk of rows.  A CU holds one
-// block, or, with fill, as many as the ring's LDS lets it (smem bytes of
-// lds_max), at most four; each XCD's 32 CUs take an eighth of the blocks in
-// rounds.  The chunks (of at least 4 rows, none empty) are those with the
-// fewest row steps, rounds x (rows of a chunk + 3 to fill the ring): a round
-// that is nearly empty costs as much as a full one (a tg time step at
-// 200x150x200: 6 chunks, 300 blocks 2089 us, 5 chunks, 250 blocks 1851 us).
-// A march shorter than MARCH_MIN rows (small grids) loses to the row-tile
-// kernels, which need no ring fill: measured at 64^3, FP64 substep 74.9 ->
-// 71.1 us, heated substep 122.1 -> 111.3 us (4-row chunks); at 128^3 (8 and
-// 16 rows) the marching kernels win (244 against 251 us, 492 against 533 us).
 // Threads past the block's last cell (n cells, whole waves) repeat that cell:
 // same loads, same stores of the same values; live says whose sums count.
 struct MarchLane {
@@ -203,6 +191,10 @@ __device__ __forceinline__ void march_split(int tid, int L, int& r, int& i) {
     r = (int)(((float)tid + 0.5f) / (float)L);
     i = tid - r * L;
 }
+// A march shorter than MARCH_MIN rows (small grids) loses to the row-tile
+// kernels, which need no ring fill: measured at 64^3, FP64 substep 74.9 ->
+// 71.1 us, heated substep 122.1 -> 111.3 us (4-row chunks); at 128^3 (8 and
+// 16 rows) the marching kernels win (244 against 251 us, 492 against 533 us).
 constexpr int MARCH_MIN = 8;
 // rows per chunk: ncol columns of blocks, bpc blocks to a CU, fill rows' worth
 // of a chunk's start-up
@@ -220,6 +212,14 @@ inline int chunk_rows(int rows, long ncol, int bpc, int fill) {
     }
     return best;
 }
+// Rows per y chunk of a kernel that marches along y with an LDS ring, one
+// block per group of k rows (nkg groups) and chunk of rows.  A CU holds one
+// block, or, with fill, as many as the ring's LDS lets it (smem bytes of
+// lds_max), at most four; each XCD's 32 CUs take an eighth of the blocks in
+// rounds.  The chunks (of at least 4 rows, none empty) are those with the
+// fewest row steps, rounds x (rows of a chunk + 3 to fill the ring): a round
+// that is nearly empty costs as much as a full one (a tg time step at
+// 200x150x200: 6 chunks, 300 blocks 2089 us, 5 chunks, 250 blocks 1851 us).
 inline int march_chunk_rows(int rows, int nkg, size_t smem, int lds_max, bool fill) {
     return chunk_rows(rows, nkg, fill ? std::max(1, std::min(4, (int)((size_t)lds_max / std::max<size_t>(smem, 1)))) : 1, 3);
 }

@@ -897,7 +897,7 @@ static int poisson_pass(chs_handle* h, const TI* f, double* dph, int ghost, cpx_
         return CHS_E_ARG;
     }
     // FP64, other lengths: register transforms where the length has a plan
-    // (the FP32 spectra keep their Stockham stages and so their roundings)
+    // (FP32 spectra still run the Stockham stages there)
     RegPlan rx, rxi, rz;
     const bool xr = !f32 && !x256 && reg_plan(L, true, &rx) && reg_plan(L, false, &rxi);
     const bool zr = !f32 && !z256 && reg_plan(N, false, &rz);

@@ -13,6 +13,7 @@
 // The reference's four separate bisections over the same T knots collapse
 // into one: they find the same interval.
 #include <algorithm>
+#include <cstring>
 #include <cmath>
 
 #include "props.hpp"
@@ -354,39 +355,45 @@ int props_create(int n, const double* H, const double* T, const double* D, const
                   std::to_string(p->lds_max) + " B)");
         return fail(CHS_E_ARG);
     }
-    const size_t bytes = sizeof(double) * (2 * (size_t)n + 20 * (size_t)n) + sizeof(int) * ((size_t)p->nbh + p->nbt);
+    // one block, uploaded in one copy: the counters (zero) on lines of their
+    // own, then the 32 B records (256 B aligned), the knots, the bucket starts
+    const size_t head = 256, tab = sizeof(double) * 22 * (size_t)n,
+                 bytes = head + tab + sizeof(int) * ((size_t)p->nbh + p->nbt);
+    std::vector<unsigned char> up(bytes, 0);
     unsigned char* blk = nullptr;
-    if (hipMalloc((void**)&blk, bytes + 256) != hipSuccess) {
+    if (hipMalloc((void**)&blk, bytes) != hipSuccess) {
         set_error("chs_props_create: device allocation failed");
         return fail(CHS_E_NOMEM);
     }
-    p->rh = reinterpret_cast<double*>(blk);   // 32 B records first (256 B aligned)
+    p->counters = reinterpret_cast<unsigned long long*>(blk);   // the block's address, for hipFree
+    p->ecnt = p->counters + 4;
+    p->ucnt = p->counters + 8;
+    p->rh = reinterpret_cast<double*>(blk + head);
     p->rt = p->rh + 4 * (size_t)n;
     p->xh = p->rt + 16 * (size_t)n;
     p->xt = p->xh + n;
     p->sh = reinterpret_cast<int*>(p->xt + n);
     p->st = p->sh + p->nbh;
-    if (hipMalloc((void**)&p->counters, 12 * sizeof(unsigned long long)) != hipSuccess ||
-        hipHostMalloc((void**)&p->ecnt_host, 4 * sizeof(unsigned long long),
+    auto put = [&](const void* dev, const void* src, size_t nb) {
+        std::memcpy(up.data() + (static_cast<const unsigned char*>(dev) - blk), src, nb);
+    };
+    put(p->rh, p->hrh.data(), p->hrh.size() * sizeof(double));
+    put(p->rt, p->hrt.data(), p->hrt.size() * sizeof(double));
+    put(p->xh, H, n * sizeof(double));
+    put(p->xt, T, n * sizeof(double));
+    put(p->sh, sh.data(), sh.size() * sizeof(int));
+    put(p->st, st.data(), st.size() * sizeof(int));
+    if (hipHostMalloc((void**)&p->ecnt_host, 4 * sizeof(unsigned long long),
                       hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
         set_error("chs_props_create: allocation of the counters failed");
         return fail(CHS_E_NOMEM);
     }
-    p->ecnt = p->counters + 4;
-    p->ucnt = p->counters + 8;
     for (int q = 0; q < 4; ++q) p->ecnt_host[q] = 0;
     if (hipEventCreateWithFlags(&p->ecnt_ev, hipEventDisableTiming) != hipSuccess) {
         set_error("chs_props_create: event creation failed");
         return fail(CHS_E_HIP);
     }
-    const unsigned long long zeros[12] = {};
-    if (hipMemcpy(p->counters, zeros, sizeof(zeros), hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(p->rh, p->hrh.data(), p->hrh.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(p->rt, p->hrt.data(), p->hrt.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(p->xh, H, n * sizeof(double), hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(p->xt, T, n * sizeof(double), hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(p->sh, sh.data(), sh.size() * sizeof(int), hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(p->st, st.data(), st.size() * sizeof(int), hipMemcpyHostToDevice) != hipSuccess) {
+    if (hipMemcpy(blk, up.data(), bytes, hipMemcpyHostToDevice) != hipSuccess) {
         set_error("chs_props_create: table upload failed");
         return fail(CHS_E_HIP);
     }
@@ -403,8 +410,7 @@ int props_destroy(chs_props* p) {
     if (!p) return CHS_OK;
     if (p->ecnt_pending) (void)hipEventSynchronize(p->ecnt_ev);   // the copy into ecnt_host
     mlp_release(p);
-    if (p->rh) (void)hipFree(p->rh);
-    if (p->counters) (void)hipFree(p->counters);
+    if (p->counters) (void)hipFree(p->counters);   // the tables' block
     if (p->ecnt_host) (void)hipHostFree(p->ecnt_host);
     if (p->ecnt_ev) (void)hipEventDestroy(p->ecnt_ev);
     if (p->own_stream && p->stream) (void)hipStreamDestroy(p->stream);

@@ -29,7 +29,7 @@ struct chs_props {
     int* st = nullptr;         // T bucket -> first candidate interval [nbt]
     double* rh = nullptr;      // [n][4]: T, b, c, d of the H -> T spline
     double* rt = nullptr;      // [n][16]: (y, b, c, d) of T -> D, M, K, CP
-    unsigned long long* counters = nullptr;   // device counters: [4] training and certification, [4] ecnt, [4] ucnt
+    unsigned long long* counters = nullptr;   // device counters: [4] training and certification, [4] ecnt, [4] ucnt; the tables follow
     unsigned long long* ucnt = nullptr;       // those of chs_therm_prop_update, zero between calls
     // host copies used by the surrogate's certification
     std::vector<double> hH, hT, hrh, hrt;

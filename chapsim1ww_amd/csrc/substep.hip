@@ -686,6 +686,8 @@ __global__ void __launch_bounds__(CPT == 1 ? 1024 : 512) k_rhs_xm(Geo g, RkCoef 
             store4(dst, o4);
         }
         if constexpr (AL) {
+            // the update above, written out again: one lambda for both places
+            // costs the other form 4 of its 128 registers and a spill
             __syncthreads();   // the x-solve rows have been read
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
