@@ -196,8 +196,9 @@ __global__ void __launch_bounds__(PT) k_props_table(PropTab t, Rows rw, const do
 // flight (6,300,000 128 with 2 against 125, 9,000,000 189 against 174).  Tables
 // too large for the wide form: one cell below PSMALL_N, 8 from there (3000
 // knots, 1,572,863 cells: 50 against 49 us on a random field, 42 on a smooth
-// one, but 51 against 129 in rows of 700); those whose knots leave a CU a single block of 256, below PSMALL (4000
-// knots: 1,048,576 cells 53 against 41 us, 1,572,863 69 against 42).
+// one, but 51 against 129 in rows of 700); those whose knots leave a CU a
+// single block of 256, below PSMALL (4000 knots: 1,048,576 cells 53 against 41
+// us, 1,572,863 69 against 42).
 constexpr long long PSMALL = 1ll << 20, PMID = 3ll << 21, PSMALL_N = 3ll << 19;
 
 int props_table_launch(chs_props* p, const double* h, Rows rw, double* T, double* rho, double* mu, double* kap,

@@ -25,7 +25,7 @@ struct StatGeo {
 // 1, so v and w's cell averages carry the factor 1.0 the reference multiplies.
 // Bound: HBM, 88 B/cell (11 fields read once).  One block per row left a
 // quarter of the CUs without work and the others with two waves: 976 us at
-// 256x192x256 (1.1 TB/s), in chunks 299 us (3.7 TB/s).
+// 256x192x256 (1.1 TB/s), in chunks 282 us (3.9 TB/s).
 __global__ void __launch_bounds__(256) k_mean_xz_io(StatGeo g, const double* __restrict__ Q,
                                                     const double* __restrict__ Gf, const double* __restrict__ PR,
                                                     const double* __restrict__ T, const double* __restrict__ RHO,

@@ -1434,14 +1434,16 @@ __global__ void __launch_bounds__(256) k_divgck_cfl(Geo g, const double* __restr
     }
 }
 
+// The 1/2 of each cell-centred average in moment m, times VL = 1 / (L N).
+__device__ __forceinline__ double mean_xz_scale(int m, double VL) {
+    return m == 3 ? VL : (m >= 4 && m < 10) ? VL * (0.5 * 0.5) : VL * 0.5;
+}
+
 // xz-mean statistics of PP_MEAN_ZX_FLOW_TG (src/processing/PP_MEAN_ZX.f90:
 // 104-237), first and second moments: one chunk of z rows of row j per block
 // (xz_chunk), out[13 j + m] as the C ABI documents (cell-centred u, v, w sums,
 // p, their products, u p).  Bound: HBM, 32 B/cell.  One block per row: 186 us
-// at 256x192x256 (2.2 TB/s), in chunks 110 us (3.7 TB/s).
-__device__ __forceinline__ double mean_xz_scale(int m, double VL) {
-    return m == 3 ? VL : (m >= 4 && m < 10) ? VL * (0.5 * 0.5) : VL * 0.5;
-}
+// at 256x192x256 (2.2 TB/s), in chunks 108 us (3.7 TB/s).
 __global__ void __launch_bounds__(256) k_mean_xz(Geo g, const double* __restrict__ Q, const double* __restrict__ PR,
                                                  int kc, int nch, double VL, double* __restrict__ part) {
     __shared__ double red[4 * 13];
@@ -1717,9 +1719,10 @@ struct CnStencils {
 // The stencils of the last few FACOE values of one handle.  Entries are
 // evicted oldest first; an evicted entry's buffers serve a later one once
 // their last-use event has completed (never while a queued substep may read
-// them); those of a captured substep stay until the handle goes.  A run that changes DT with its CFL number brings three new values a
-// step: allocating and freeing for each waited for the GPU (a step of its own
-// DT, with the cost of the inverses: 64^3 1244 -> 270, 256x192x256 11254 -> 2981 us).
+// them); those of a captured substep stay until the handle goes.  A run that
+// changes DT with its CFL number brings three new values a step: allocating
+// and freeing for each waited for the GPU (a step of its own DT, with the cost
+// of the inverses: 64^3 1244 -> 270, 256x192x256 11254 -> 2981 us).
 struct CnCache {
     std::list<CnStencils> live;   // list: entries keep their addresses; at most 8
     std::vector<CnBuf> retired;

@@ -261,10 +261,10 @@ struct TdmaPlan {
 // sweep of all of them on an MI355X: 42 lengths from 8 to 512 rows x 20 to 23
 // counts from 16 to 65536 lines, both layouts.  Over the sweep the choice is on
 // average 2% (lines contiguous), 11% and 7% (rows contiguous, non-cyclic and
-// cyclic) behind the fastest
-// candidate of each point; what it loses most at: 30% to 2 lines a block (64
-// lines of 512 rows, 11.5 against 8.9 us), 20% to 2 lines of 4-row segments
-// (65536x192, rows contiguous, 181 against 145).  What decides:
+// cyclic) behind the fastest candidate of each point; what it loses most at:
+// 30% to 2 lines a block (64 lines of 512 rows, 11.5 against 8.9 us), 20% to 2
+// lines of 4-row segments (65536x192, rows contiguous, 181 against 145).  What
+// decides:
 //   fullest CU    on_cu(lpb): the lines of the CU with the most, in whole
 //     blocks.  Where 32 lines a block leave it no more than 16 do, the larger
 //     accesses win (non-cyclic 65536x128 72 us with 32, 85 with 16; 14000x144,
@@ -286,10 +286,10 @@ struct TdmaPlan {
 //     27, 8 x 16 37; 32768x120 48, 8 x 16 58)
 //   cyclic        short lines of whole segments: the serial sweep of a reduced
 //     system of up to 20 rows (32 at most) has two barriers where the cyclic
-//     reduction has two a step (10000x16 3.9 us, Split 4.9; 65536x96 12 x 32 57, Split 68;
-//     rows contiguous 65536x8 6.9, Split 10.9); whole 12-row segments
-//     of 132 to 192 rows (65536x192 121 us, Split 150) and of 257 to 384
-//     (10000x360 42, Split 60); everything else Split
+//     reduction has two a step (10000x16 3.9 us, Split 4.9; 65536x96 12 x 32
+//     57, Split 68; rows contiguous 65536x8 6.9, Split 10.9); whole 12-row
+//     segments of 132 to 192 rows (65536x192 121 us, Split 150) and of 257 to
+//     384 (10000x360 42, Split 60); everything else Split
 static TdmaPlan tdma_plan(int n, int nlines, long long es, long long ls, bool cyclic) {
     constexpr int CUS = 256;
     const int p8 = (n + 7) / 8, p12 = (n + 11) / 12, ps = (n + 6) / 8;   // segments; ps: of the n - 1 rows of Split
